@@ -64,11 +64,12 @@ template <bool ELEC, bool EXT = false>
 __device__ __forceinline__ double cell_lambda(const CellIn<ELEC>& c, int isp) {
   const double T = c.T;
   if (!ELEC) return thermal_coeff(isp) * pow25(T);
-  const double sq = sqrt(T);
+  double sq;
+  const double T25 = pow25(T, sq);
   const double br = ((c.n1 * 1.1e-16) * (1.0 + 5.7e-4 * T) + ((c.n2 * 2.82e-17) * sq) * (1.0 - 1.21e-4 * T))
                     + (c.n3 * 2.2e-16) * (1.0 + 3.6e-2 * sq);
   const double den = 1.0 + ((3.22e4 * (T * T)) / c.n) * br;
-  const double lambda = (((elchrg * 100.0) * 7.7e5) * pow25(T)) / den;
+  const double lambda = (((elchrg * 100.0) * 7.7e5) * T25) / den;
   return EXT ? lambda * c.kap : lambda;
 }
 

@@ -503,7 +503,8 @@ int gemhip_register_grid(int xtype, int gridflag, int flagper, const int* isglob
   if (c.d_geom) hipFree(c.d_geom);
   c.d_geom = nullptr;
   // every array starts 256-byte aligned (the sweeps' DMA loads read 16-byte pairs)
-  if (!hipok(hipMalloc((void**)&c.d_geom, (total + 19 * 32 + 3 * g.hstride) * sizeof(double)),
+  if (!hipok(hipMalloc((void**)&c.d_geom, (total + 20 * 32 + 3 * g.hstride +
+                                             diffusion_rdx_doubles(g)) * sizeof(double)),
              "geometry"))
     return 5;
   const double** dst[] = {&g.h1, &g.h2, &g.h3, &g.h1x1i, &g.h2x1i, &g.h3x1i, &g.h1x2i, &g.h2x2i,
@@ -519,7 +520,11 @@ int gemhip_register_grid(int xtype, int gridflag, int flagper, const int* isglob
   }
   off = (off + 31) & ~31L;                     // 256-byte aligned rows of 64 columns
   g.hcol = c.d_geom + off;                     // the diffusion's copy of h1, h2, h3
-  launch_fill_hcol(g, c.d_geom + off, c.stream);
+  double* rdx = c.d_geom + off + 3 * g.hstride;
+  g.rdx1 = rdx;
+  g.rdx1i = rdx + (c.lx1 + 3);
+  g.rdx1s = rdx + 2 * (c.lx1 + 3);
+  launch_fill_hcol(g, c.d_geom + off, rdx, c.stream);
   if (!hipok(hipStreamSynchronize(c.stream), "geometry reorder")) return 6;
   g.gridflag = gridflag;
   g.flagper = flagper ? 1 : 0;
@@ -1338,7 +1343,7 @@ int gemhip_energy_diffusion_noalloc(double* Ts, const double* ns, const double* 
     fail("kernel timing creates events on demand: disable it before allocation-free calls");
     return 3;
   }
-  const size_t need = diffusion_scratch_bytes(c.g);
+  const size_t need = diffusion_noalloc_bytes(c.g);
   if (need > (size_t)NOALLOC_SCRATCH_BYTES) {
     fail("grid %dx%dx%d needs %zu bytes of diffusion work space; the allocation-free entry "
          "point has %zu", c.lx1, c.lx2, c.lx3, need, (size_t)NOALLOC_SCRATCH_BYTES);

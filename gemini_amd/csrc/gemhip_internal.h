@@ -26,6 +26,8 @@ struct DevGrid {
   // lane) the column's group and lane (hcol_index in diffusion_cell.h)
   const double* hcol;
   long hstride;
+  // correctly rounded reciprocals of dx1(i), dx1i(i) and dx1(i+1) + dx1(i) at index i
+  const double *rdx1, *rdx1i, *rdx1s;
 };
 
 // State pointers in HBM.  ns..Ts point into one fluidvars block of 35 fields,
@@ -112,7 +114,9 @@ void launch_sweep(const DevGrid& g, const DevState& s, int dir, int fields, doub
 // ---- launchers (kernels_diffusion.hip) ----
 size_t diffusion_scratch_bytes(const DevGrid& g);
 long diffusion_hcol_doubles(const DevGrid& g);              // size of DevGrid::hcol
-void launch_fill_hcol(const DevGrid& g, double* hcol, hipStream_t st);
+long diffusion_rdx_doubles(const DevGrid& g);               // and of rdx1, rdx1i, rdx1s together
+void launch_fill_hcol(const DevGrid& g, double* hcol, double* rdx, hipStream_t st);
+size_t diffusion_noalloc_bytes(const DevGrid& g);           // the allocation-free entry's measure
 
 // ---- batched ensemble steps (kernels_advec.hip, kernels_diffusion.hip) ----
 // One member of an ensemble advanced by batched kernels: every kernel of the fused

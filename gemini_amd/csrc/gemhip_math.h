@@ -56,12 +56,13 @@ GEMHIP_HD double fmax_f(double a, double b) { return (b > a) ? b : a; }
 // the FMA residual x - b q0 is exact, and one correction step q0 + r y, rounded once,
 // gives RN(x/b) (Markstein's theorem for a correctly rounded reciprocal).  Where the
 // residual is zero (exact quotients, zero numerators: q0 has the sign IEEE division gives)
-// or not a number (infinite numerators) q0 is the quotient.
+// or not a number (infinite numerators) or infinite (a quotient past the largest double) q0
+// is the quotient.
 __device__ __forceinline__ double div_rcp(double x, double b, double y) {
   const double q0 = x * y;
   const double r = __builtin_fma(-b, q0, x);
   const double q1 = __builtin_fma(r, y, q0);
-  return __builtin_amdgcn_class(r, 0x63) ? q0 : q1;    // sNaN qNaN -0 +0
+  return __builtin_amdgcn_class(r, 0x267) ? q0 : q1;   // sNaN qNaN -inf -0 +0 +inf
 }
 
 // advec.f90:438-447
@@ -82,13 +83,12 @@ GEMHIP_HD double fma_exact(double a, double b, double c) {
 // (its error bound is below 0.52 ulp and exact-or-correct for x^n.5 in practice; the
 // CPU test checks agreement on millions of samples).  x^2.5 = x^2 * sqrt(x) is formed
 // in double-double: x^2 exactly by an FMA product split, sqrt(x) to ~2^-104 by one
-// Newton correction, then one final rounding.  Arguments outside the normal range the
-// transport path sees fall back to the library pow.
-GEMHIP_HD double pow25(double x) {
-  if (!(x > 0x1p-400 && x < 0x1p+400)) return pow(x, 2.5);
-  const double s = sqrt(x);                 // correctly rounded
+// Newton correction (e/(2s), with `ih` a reciprocal of 2s to about an ulp), then one final
+// rounding.  For arguments between 2^-400 and 2^400, where nothing in between over- or
+// underflows.
+GEMHIP_HD double pow25_core(double x, double s, double ih) {
   const double e = fma_exact(-s, s, x);     // x - s*s exactly
-  const double sl = e / (2.0 * s);          // sqrt(x) ~= s + sl
+  const double sl = e * ih;                 // sqrt(x) ~= s + sl
   const double qh = x * x;
   const double ql = fma_exact(x, x, -qh);   // x*x = qh + ql exactly
   const double ph = qh * s;
@@ -96,15 +96,57 @@ GEMHIP_HD double pow25(double x) {
   return ph + pl;
 }
 
-// x**1.5 rounded to nearest in the same way: x * sqrt(x) in double-double, one rounding.
-GEMHIP_HD double pow15(double x) {
-  if (!(x > 0x1p-400 && x < 0x1p+400)) return pow(x, 1.5);
-  const double s = sqrt(x);
-  const double e = fma_exact(-s, s, x);
-  const double sl = e / (2.0 * s);
-  const double ph = x * s;
-  const double pl = fma_exact(x, s, -ph) + x * sl;
-  return ph + pl;
+#if defined(__HIP_DEVICE_COMPILE__)
+// sqrt(x), correctly rounded, and a reciprocal of 2 sqrt(x), for x between 2^-400 and 2^400:
+// v_rsq_f64, one Goldschmidt step, two residual corrections of the root (the sequence the
+// compiler's sqrt uses inside its scaling for the arguments excluded here) and a Newton step
+// of the reciprocal.
+__device__ __forceinline__ double sqrt_rcp(double x, double& ih) {
+  const double r = __builtin_amdgcn_rsq(x);
+  double g = x * r, h = 0.5 * r;
+  const double d = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, d, g);
+  h = __builtin_fma(h, d, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  ih = __builtin_fma(h, __builtin_fma(-h, g + g, 1.0), h);
+  return g;
 }
+
+// x**2.5 and sqrt(x).  Arguments outside the core's range are scaled by an even power of two
+// first (zero, negative, infinite and NaN arguments give pow's results), in a branch taken
+// only by waves that hold one: written as a plain conditional around the library pow, it was
+// turned into selects and every cell of the diffusion evaluated the library pow too (1600 of
+// the solve's 4200 cycles per row on a 128x64x1 grid).
+__device__ __forceinline__ double pow25(double x, double& root) {
+  const bool out = !(x > 0x1p-400 && x < 0x1p+400);
+  double ih;
+  if (__builtin_expect(__any(out), 0)) {
+    const int k = out ? __builtin_amdgcn_frexp_exp(x) >> 1 : 0;
+    const double m = __builtin_amdgcn_ldexp(x, -2 * k);
+    const double s = sqrt_rcp(m, ih);
+    const double y = __builtin_amdgcn_ldexp(pow25_core(m, s, ih), 5 * k);
+    root = sqrt(x);
+    return x > 0.0 && x < __builtin_inf() ? y : x == 0.0 ? 0.0
+           : __builtin_fabs(x) == __builtin_inf() ? __builtin_inf() : __builtin_nan("");
+  }
+  root = sqrt_rcp(x, ih);
+  return pow25_core(x, root, ih);
+}
+__device__ __forceinline__ double pow25(double x) {
+  double root;
+  return pow25(x, root);
+}
+#else
+GEMHIP_HD double pow25(double x, double& root) {
+  root = sqrt(x);
+  if (!(x > 0x1p-400 && x < 0x1p+400)) return pow(x, 2.5);
+  return pow25_core(x, root, 1.0 / (2.0 * root));
+}
+GEMHIP_HD double pow25(double x) {
+  double root;
+  return pow25(x, root);
+}
+#endif
 
 }  // namespace gemhip

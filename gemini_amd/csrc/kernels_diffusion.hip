@@ -31,82 +31,69 @@ struct Coef {
   double c13, c43; // 1/3._wp and 4/3._wp
 };
 
-// State of the pivoted elimination between steps: the row at pivot position j holds
-// (r0, r1) in columns j, j+1 (column j+2 is always zero there) and right-hand side rb.
-struct Elim {
-  double r0, r1, rb;
-  bool singular;
-};
-
 // ---------------------------------------------------------------- column-group kernel
-// One wavefront (the whole workgroup) owns 64 columns of one species, one lane per
-// column, and makes four passes over the rows:
-//   1 (top-down): the input rows arrive in chunks of R rows.  The wave loads a chunk of
-//     all 64 columns cooperatively (lane -> (row, column), so each load instruction reads
-//     whole 64-byte segments), computes conductivity and the coefficients C, B, D of each
-//     (row, column) in parallel into LDS, and each lane then builds its column's rows
-//     and runs the sequential pivoted elimination of the first solve (TR, or backward
-//     Euler) with its right-hand side.  For TRBDF2 the same pass also factors the BDF2
-//     matrix, which does not depend on the TR solution: its pivot rows, multipliers and
-//     row interchanges are stored;
-//   2 (bottom-up): back substitution of the first solve (into Ts for backward Euler);
-//   3 (top-down, TRBDF2): the BDF2 right-hand side from the input temperatures and the
-//     TR solution, taken through the stored interchanges and multipliers (dgbtrs's
-//     forward solve);
-//   4 (bottom-up, TRBDF2): back substitution of the BDF2 solve into Ts.
+// One wavefront (the whole workgroup) owns 64 systems, one lane each: the 64 columns of a
+// column group for the electrons, or 32 columns (half a group) of two ion species.  The two
+// ions of a wave read the columns' metric factors once.  It makes four passes over the rows:
+//   1 (top-down): the input rows arrive in chunks of R rows, loaded by the wave
+//     cooperatively (lane -> (row, column), so each load instruction reads whole 64-byte
+//     segments), the next chunk's loads in flight while a chunk is used.  Conductivity and
+//     the cell factors C, B, D of each (row, column) go through LDS; each lane then forms
+//     its rows' three parabolic terms and runs the pivoted elimination of the first solve
+//     (TR, or backward Euler).  It keeps the terms and the temperature of every row, and
+//     the elimination's state at the first row of every block of R rows; the pivot rows
+//     themselves are not kept;
+//   2 (bottom-up, block by block): the block's pivot rows formed again in registers from
+//     its kept state, and back substitution through them (into Ts for backward Euler; for
+//     TRBDF2 the BDF2 right-hand side of each row, in the temperature's place);
+//   3 (top-down, TRBDF2): the elimination of the BDF2 system, its state kept per block;
+//   4 (bottom-up, TRBDF2): as pass 2, into Ts.
 // Every value is formed with the operations, and in the order, LAPACK's dgbtf2, dgbtrs
-// and dtbsv would use on the reference's band matrix: factorising a matrix before its
-// right-hand side is known changes nothing in either.  The pivot rows, right-hand sides
-// and solutions live in lane-interleaved HBM scratch (one 512-byte segment per row and
-// slot for the wave); outputs are staged through LDS so global stores are coalesced.
-// Blocks are numbered so that the seven species of a column group run on one XCD, the
-// electron groups (the longest waves) first.
+// and dtbsv would use on the reference's band matrix; forming a pivot row a second time
+// from the same state gives the same bits.
+//
+// Why the pivot rows are formed twice: the full-size launch is bound by HBM traffic, and
+// the solve's arithmetic is a fifth of its time.  Keeping both factorisations took nine
+// 8-byte slots per row and species, each written and read (a pivot row, its right-hand
+// side and a multiplier for each solve); the terms, the temperature and the block states
+// take 3.4 slots for an ion and 4.4 for the electrons.  With the ions' shared metric factors
+// and the cheaper x**2.5 and divisions: 512x256x192 7.91 -> 5.88 ms, 255x113x67 0.87 -> 0.62,
+// 301x127x75 1.19 -> 0.83 (backward Euler 256x128x96 0.66 -> 0.50), 128x64x1 0.225 -> 0.209.
+//
+// Rows are kept lane-interleaved in HBM (one 512-byte segment per row and slot for the
+// wave) and outputs are staged through LDS so global stores are coalesced.  Blocks are
+// numbered so that the species of a column group run on one XCD, the electron groups (the
+// longest waves) first.
+//
+// Divisions by values that depend on the row or the step alone (coordinate differences, dt/2,
+// dt/3) are multiplications by correctly rounded reciprocals with one correction (div_rcp),
+// which gives the IEEE quotient; every other division is one.
 //
 // The steady state of every pass issues its memory operations unconditionally (clamped
-// indices; stores that must not land go where a later store of the same lane overwrites
-// them), so the compiler's wait counters stay exact and loads issued ahead stay in
-// flight.  Lanes of a group past the last column solve the last column again and write
-// the same values to the same places.
+// indices; rows 1 and N have slots that no system uses, where rows past the ends land), so
+// the compiler's wait counters stay exact and loads issued ahead stay in flight.  Lanes of a
+// group past the last column solve the last column again and write the same values to the
+// same places.
 constexpr int LP = 65;         // padded LDS row (conflict-free transposed access)
 #ifndef DIFF_CHUNK
 #define DIFF_CHUNK 8           // rows per chunk: 4 x 8 x 65 doubles of LDS per wave
 #endif
-#ifndef DIFF_SPLIT
-#define DIFF_SPLIT 0           // 1: TRBDF2 as two launches (passes 1-2, passes 3-4)
-#endif
-#ifndef DIFF_BATCH_I
-#define DIFF_BATCH_I 8         // ion cells per lane whose inputs are loaded together
-#endif
 #ifndef DIFF_BATCH_E
-#define DIFF_BATCH_E 4         // the same for electron cells (nine inputs each)
+#define DIFF_BATCH_E 2         // electron cells per lane whose inputs are loaded together
 #endif
-// scratch slots per (row, lane)
-enum : int {
-  SU0 = 0, SU1 = 1, SU2 = 2, SY = 3,   // first solve: pivot row (U0 U1 U2) and its rhs y;
-                                       // pass 3 reuses SY for the BDF2 rhs
-  STR = 4,                             // TR solution
-  SV0 = 5, SV1 = 6, SV2 = 7, SL = 8,   // BDF2 pivot rows and multipliers
-  NSLOT = 9                            // (the T part of the BDF2 rhs is formed in pass 3
-};                                     // from Ts, which pass 4 is the first to overwrite)
+// slots of a row: the parabolic terms of its lower and upper neighbour and (electrons) of
+// the drift; the input temperature, which pass 2 replaces by the BDF2 right-hand side
+enum : int { ST1 = 0, ST3 = 1, STV = 2, ST2 = 3 };
+constexpr int NCK = 3;         // kept elimination state: r0, r1, rb
 
-struct Group {
-  int N;
-  double* scr;                 // this lane's scratch: slot k of row i at scr[((i-1)*NSLOT+k)*64]
-  int* swb;                    // BDF2 row interchanges, bit (j&31) of word j>>5 at swb[(j>>5)*64]
-};
-
-__device__ __forceinline__ double& S2(const Group& q, int i, int k) {
-  return q.scr[((long)(i - 1) * NSLOT + k) * 64];
+// units of a column group: one wave of electrons, six of ions (half of its columns, a pair
+// of species)
+__host__ __device__ inline long diffusion_groups(const DevGrid& g) {
+  return ((long)g.lx2 * g.lx3 + 63) / 64;
 }
-// Scratch traffic is non-temporal (the nt bit: streamed through L2 at low priority).  A
-// slot is written once and read once, a pass later; as ordinary accesses the ~256 waves
-// of an XCD streaming their pivot rows evicted the input lines that the cooperative loads
-// of the next row chunk still needed (those loads read 64-byte halves of 128-byte lines).
-__device__ __forceinline__ void put2(const Group& q, int i, int k, double v) {
-  __builtin_nontemporal_store(v, &S2(q, i, k));
-}
-__device__ __forceinline__ double get2(const Group& q, int i, int k) {
-  return __builtin_nontemporal_load(&S2(q, i, k));
+__host__ __device__ inline int kept_blocks(const DevGrid& g) { return (g.lx1 + 6) / 4 + 1; }
+__host__ __device__ inline long unit_doubles(const DevGrid& g, bool elec) {
+  return ((long)g.lx1 * (elec ? 4 : 3) + (long)kept_blocks(g) * NCK) * 64;
 }
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -115,91 +102,105 @@ __device__ __forceinline__ void column_of(const DevGrid& g, int gcol, int& i2, i
   i2 = gcol % g.lx2 + 1;
   i3 = gcol / g.lx2 + 1;
 }
-
-// Pivoted elimination step j (dgbtf2 with dgbtrs's forward solve) bringing in row j+1 =
-// (a, b, cc | d), applied to the state only when `real`.  The row at pivot position j is
-// stored at row sj (a step that is not real stores where the real step sj stores later).
-__device__ __forceinline__ bool elim_rhs(const Group& q, Elim& e, int j, int sj, bool real,
-                                         double a, double b, double cc, double d) {
-  const bool swap = fabs(a) > fabs(e.r0);
-  double p0, p1, p2, pd, o0, o1, o2, od;
-  if (swap) { p0 = a; p1 = b; p2 = cc; pd = d; o0 = e.r0; o1 = e.r1; o2 = 0.0; od = e.rb; }
-  else      { p0 = e.r0; p1 = e.r1; p2 = 0.0; pd = e.rb; o0 = a; o1 = b; o2 = cc; od = d; }
-  bool sing = false;
-  if (p0 != 0.0) {
-    const double rp = 1.0 / p0;
-    const double l = rp * o0;
-    if (p1 != 0.0) o1 = o1 + l * (-p1);
-    if (p2 != 0.0) o2 = o2 + l * (-p2);
-    if (pd != 0.0) od = od + l * (-pd);
-  } else {
-    sing = true;
-  }
-  put2(q, sj, SU0, p0); put2(q, sj, SU1, p1); put2(q, sj, SU2, p2); put2(q, sj, SY, pd);
-  if (real) {
-    e.singular = e.singular || sing;
-    e.r0 = o1; e.r1 = o2; e.rb = od;
-  }
-  return swap;
+// a grid array at a wave-uniform index, by a scalar load (a vector load would be the newest
+// vector memory operation, and waiting for it would wait for every kept row in flight)
+__device__ __forceinline__ double ld_row(const double* p, int i) {
+  return ((const __attribute__((address_space(4))) double*)p)[i];
 }
 
-// The same step on the matrix alone (the BDF2 factorisation): stores the pivot row, the
-// multiplier l and the interchange bit that the right-hand side will need in pass 3 (a
-// word of 32 steps' bits, stored once its last step, or step N-1, has run).
-struct Fact {
-  double r0, r1;
+// a pointer to HBM that is the same for the whole wave, in scalar registers
+typedef __attribute__((address_space(1))) double gdouble;
+__device__ __forceinline__ gdouble* uniform_ptr(double* p) {
+  const unsigned long a = (unsigned long)p;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+  return (gdouble*)(((unsigned long)hi << 32) | lo);
+}
+
+// State of the pivoted elimination between steps: the row at pivot position j holds
+// (r0, r1) in columns j, j+1 (column j+2 is always zero there) and right-hand side rb.
+struct Elim {
+  double r0, r1, rb;
   bool singular;
-  int word, bits;              // interchange bits of steps 32*word .. 32*word+31
+};
+struct Pivot {
+  double u0, u1, u2, y;
 };
 
-__device__ __forceinline__ void elim_mat(const Group& q, Fact& f, int j, int sj, bool real,
-                                         double a, double b, double cc) {
-  const bool swap = fabs(a) > fabs(f.r0);
-  double p0, p1, p2, o0, o1, o2;
-  if (swap) { p0 = a; p1 = b; p2 = cc; o0 = f.r0; o1 = f.r1; o2 = 0.0; }
-  else      { p0 = f.r0; p1 = f.r1; p2 = 0.0; o0 = a; o1 = b; o2 = cc; }
-  bool sing = false;
-  double l = 0.0;
-  if (p0 != 0.0) {
-    const double rp = 1.0 / p0;
-    l = rp * o0;
-    if (p1 != 0.0) o1 = o1 + l * (-p1);
-    if (p2 != 0.0) o2 = o2 + l * (-p2);
-  } else {
-    sing = true;
-  }
-  put2(q, sj, SV0, p0); put2(q, sj, SV1, p1); put2(q, sj, SV2, p2); put2(q, sj, SL, l);
-  if (real) {
-    f.singular = f.singular || sing;
-    f.r0 = o1; f.r1 = o2;
-    const int w = j >> 5;
-    f.bits = (w == f.word ? f.bits : 0) | ((swap ? 1 : 0) << (j & 31));
-    f.word = w;
-  }
-  if ((j & 31) == 31 || j >= q.N - 1) q.swb[f.word * 64] = f.bits;   // the word is complete
+// Pivoted elimination step (dgbtf2 with dgbtrs's forward solve) bringing in the row
+// (a, b, cc | d): returns the pivot row, advances the state.  A zero pivot leaves the other
+// row as it is, a zero entry of the pivot row its column (dger skips it).  Written without
+// branches: a step under a branch could not overlap the next row's independent work.
+__device__ __forceinline__ Pivot elim_step(Elim& e, double a, double b, double cc, double d,
+                                           bool& swap) {
+  swap = fabs(a) > fabs(e.r0);
+  Pivot p;
+  p.u0 = swap ? a : e.r0;
+  p.u1 = swap ? b : e.r1;
+  p.u2 = swap ? cc : 0.0;
+  p.y = swap ? d : e.rb;
+  const double o0 = swap ? e.r0 : a, o1 = swap ? e.r1 : b, o2 = swap ? 0.0 : cc,
+               od = swap ? e.rb : d;
+  const bool live = p.u0 != 0.0;
+  const double rp = 1.0 / p.u0;
+  const double l = rp * o0;
+  const double n1 = o1 + l * (-p.u1), n2 = o2 + l * (-p.u2), nd = od + l * (-p.y);
+  e.r0 = live & (p.u1 != 0.0) ? n1 : o1;
+  e.r1 = live & (p.u2 != 0.0) ? n2 : o2;
+  e.rb = live & (p.y != 0.0) ? nd : od;
+  e.singular = e.singular | !live;
+  return p;
 }
 
-template <int R, bool BE, bool ELEC, int PH, bool EXT>
-__device__ __forceinline__ void diffusion_group(const DevGrid& g, const DevState& s,
-                                                double* scratch, int* swbits, int* lst,
-                                                const Coef& k1,
-                                                const Coef& bdf, double Teinf, int isp,
-                                                long cg, long gps, double (*sT)[LP],
-                                                double (*sC)[LP], double (*sB)[LP],
-                                                double (*sD)[LP]) {
-  const long ncol = (long)g.lx2 * g.lx3;
+// one row of dtbsv, column-oriented: x(i+2) U2 comes off first, then x(i+1) U1; a zero x(j)
+// contributes nothing, a zero row stays zero
+__device__ __forceinline__ double back_step(const Pivot& p, double x1, double x2) {
+  const double a2 = p.y - x2 * p.u2;
+  double acc = x2 != 0.0 ? a2 : p.y;
+  const double a1 = acc - x1 * p.u1;
+  acc = x1 != 0.0 ? a1 : acc;
+  const double q = acc / p.u0;
+  return acc != 0.0 ? q : acc;
+}
+
+template <int R, bool BE, bool ELEC, bool EXT>
+__device__ __forceinline__ void diffusion_unit(const DevGrid& g, const DevState& s,
+                                               double* scratch, const Coef& k1, const Coef& bdf,
+                                               double Teinf, long cg, int half, int pair,
+                                               double (*sT)[LP], double (*sC)[LP],
+                                               double (*sB)[LP], double (*sD)[LP]) {
+  constexpr int NC = ELEC ? 64 : 32;                 // columns of the wave
+  constexpr int NSP = ELEC ? 1 : 2;                  // species of the wave
+  constexpr int CPI = 64 / R;                        // columns per load instruction
+  constexpr int NK = NC / CPI;                       // and cells per lane of a chunk
+  constexpr int NS = ELEC ? 4 : 3;
   const int lane = threadIdx.x;
-  const int col = group_column(g, cg, lane);
   const int N = g.lx1;
-  const long grp = (long)(isp - 1) * gps + cg;
-  Group q;
-  q.N = N;
-  q.scr = scratch + grp * (long)N * NSLOT * 64 + lane;
-  q.swb = swbits + grp * (long)((N + 31) / 32) * 64 + lane;
-  const long so = (long)(isp - 1) * g.N;
+  const int isp0 = ELEC ? LSP : 2 * pair + 1;
+  const int isp = ELEC ? LSP : isp0 + (lane >> 5);
+  const int l0 = ELEC ? 0 : half * 32;               // the wave's first lane in the group
+  const int col = group_column(g, cg, l0 + (lane & (NC - 1)));
+  const long gps = diffusion_groups(g);
+  gdouble* row0 = uniform_ptr(
+      scratch + (ELEC ? cg * unit_doubles(g, true)
+                      : gps * unit_doubles(g, true) +
+                            ((cg * 2 + half) * 3 + pair) * unit_doubles(g, false)));
+  gdouble* ck0 = row0 + (long)N * NS * 64;
+  // Kept rows are non-temporal (the nt bit: streamed through L2 at low priority): each is
+  // written once and read a pass later, and as ordinary accesses they evicted the input
+  // lines that the cooperative loads of the next chunk still needed.
+  // (addresses: a wave-uniform row pointer plus the lane)
+  const unsigned ln = lane;
+  auto put = [&](int i, int k, double v) { __builtin_nontemporal_store(v, row0 + ((long)(i - 1) * NS + k) * 64 + ln); };
+  auto get = [&](int i, int k) { return __builtin_nontemporal_load(row0 + ((long)(i - 1) * NS + k) * 64 + ln); };
+  auto keep_state = [&](int m, const Elim& e) {
+    gdouble* c = ck0 + (long)m * NCK * 64;
+    __builtin_nontemporal_store(e.r0, c + ln);
+    __builtin_nontemporal_store(e.r1, c + 64 + ln);
+    __builtin_nontemporal_store(e.rb, c + 128 + ln);
+  };
   const long ni = (long)g.lx1 * g.lx2 * g.lx3;
   const long kb = (long)g.lx1 * col;
-  const double gm1kB = (gammas(isp) - 1.0) / kB;
   const double* dx1 = g.dx1;
   const double* dx1i = g.dx1i - 1;
   double Tmin, Tmax;
@@ -214,347 +215,394 @@ __device__ __forceinline__ void diffusion_group(const DevGrid& g, const DevState
   double aN = 0.0, bN = 1.0;
   if (EXT && ELEC && s.qtop) {
     CellIn<ELEC> top;
-    cell_load<ELEC, EXT>(g, s, so, gix(g, 0, col % g.lx2 + 1, col / g.lx2 + 1), kb, ni, N, top,
-                         hcol_index(g, col, N), col);
+    cell_load<ELEC, EXT>(g, s, (long)(LSP - 1) * g.N, gix(g, 0, col % g.lx2 + 1, col / g.lx2 + 1),
+                         kb, ni, N, top, hcol_index(g, col, N), col);
     aN = -1.0 / dx1[N];
     bN = 1.0 / dx1[N];
     Tmax = (s.qtop[col] * top.h1) / cell_lambda<ELEC, EXT>(top, isp);
   }
-  // cooperative mapping of a chunk: lane -> (row lr, column sub-index cs); R loads per lane
+  // cooperative mapping of a chunk: lane -> (row lr, column sub-index cs)
   const int lr = lane % R, cs = lane / R;
-  constexpr int CPI = 64 / R;                        // columns per load instruction
-  constexpr int BATCH = ELEC ? DIFF_BATCH_E : DIFF_BATCH_I;
-  static_assert(R % BATCH == 0 || R < BATCH, "chunk and batch sizes");
-  constexpr int NB = R < BATCH ? R : BATCH;
   // Row phase of the chunk windows: a column's row 1 sits 2 cells into its stride, so
   // windows of R rows from row 1 straddle 64-byte sectors, and a sector's other part is
   // fetched again a chunk later (long after the L2 dropped it).  The wave's windows start
   // ph rows early instead, which puts the windows of lane 0's column, and of every column
   // that shares its sector phase (all of an interleaved group's), on sector boundaries.
-  // The steps before row 1 are not real.  The electrons' neutral densities are stored without
-  // ghosts and are aligned at row 1, so their waves keep phase 0 in pass 1.
+  // The steps before row 1 are not real.  Blocks of kept state use the same windows.
   int c2, c3;
-  column_of(g, group_column(g, cg, 0), c2, c3);
-  const int pos1 = (int)(((unsigned long)(s.Ts + so + gix(g, 0, c2, c3) + 1) >> 3) & 7);
+  column_of(g, group_column(g, cg, l0), c2, c3);
   constexpr int RA = R < 8 ? R : 8;                  // (R a power of two)
-  const int ph1 = ELEC ? 0 : pos1 % RA;              // pass 1: windows from row 1 - ph1
-  const int ph3 = (pos1 + 1) % RA;                   // pass 3: windows from row 2 - ph3
-  const int pho = pos1 % RA;                         // output chunks from row 1 - pho
-  int cbk[R];                                        // gix(0, i2, i3) of the columns this lane loads
-  int kbk[R];                                        // and their interior offsets lx1*(column)
-  int gck[R];                                        // and column numbers (extension only)
+  const double* Ts0 = s.Ts + (long)(isp0 - 1) * g.N;
+  const int ph = __builtin_amdgcn_readfirstlane(
+      (int)(((unsigned long)(Ts0 + gix(g, 0, c2, c3) + 1) >> 3) & 7) % RA);
+  const int mb = (N - 1 + ph) / R;                   // block and chunk of row N
+  int cbk[NK];                                       // gix(0, i2, i3) of the columns this lane loads
+  int kbk[ELEC ? NK : 1];                            // and their interior offsets lx1*(column)
+  int gck[EXT && ELEC ? NK : 1];                     // and column numbers (extension only)
 #pragma unroll
-  for (int k = 0; k < R; ++k) {
-    const int gcol = group_column(g, cg, k * CPI + cs);
+  for (int k = 0; k < NK; ++k) {
+    const int gcol = group_column(g, cg, l0 + k * CPI + cs);
     int a2, a3;
     column_of(g, gcol, a2, a3);
     cbk[k] = (int)gix(g, 0, a2, a3);
-    kbk[k] = g.lx1 * gcol;
-    gck[k] = gcol;
+    if (ELEC) kbk[k % (ELEC ? NK : 1)] = g.lx1 * gcol;
+    if (EXT && ELEC) gck[k % (EXT && ELEC ? NK : 1)] = gcol;
   }
 
-  // load and convert the rows r0..r0+R-1 of the 64 columns into LDS (rows past N repeat N)
-  auto load_chunk = [&](int r0) {
+  // inputs of a chunk: rows r0..r0+R-1 (clamped to 1..N) of the wave's columns.  The electrons
+  // (nine values a cell) load theirs in batches, the first a chunk ahead.
+  constexpr int NB = ELEC ? (NK < DIFF_BATCH_E ? NK : DIFF_BATCH_E) : NK;
+  CellIn<ELEC> in[NB][NSP];
+  auto issue = [&](int r0, int k0, CellIn<ELEC> (*c)[NSP]) {
     const int r = clampi(r0 + lr, 1, N);
     // hcol slot of this lane's first column at row r: the group's 64 columns are contiguous
     // (slots past the last column repeat it, as these lanes do)
-    const long hrow = ((long)cg * N + (r - 1)) * 64 + cs;
+    const long hrow = ((long)cg * N + (r - 1)) * 64 + l0 + cs;
 #pragma unroll
-    for (int k0 = 0; k0 < R; k0 += NB) {
-      CellIn<ELEC> in[NB];
+    for (int k = 0; k < NB; ++k) {
+      const int kk = k0 + k;
+      if (ELEC) {
+        cell_load<ELEC, EXT>(g, s, (long)(LSP - 1) * g.N, cbk[kk], kbk[kk % (ELEC ? NK : 1)], ni, r,
+                             c[k][0], hrow + kk * CPI, gck[kk % (EXT && ELEC ? NK : 1)]);
+      } else {
+        const long hc = hrow + kk * CPI;
+        const double h1 = g.hcol[hc], h2 = g.hcol[g.hstride + hc], h3 = g.hcol[2 * g.hstride + hc];
 #pragma unroll
-      for (int k = 0; k < NB; ++k)
-        cell_load<ELEC, EXT>(g, s, so, cbk[k0 + k], kbk[k0 + k], ni, r, in[k],
-                             hrow + (k0 + k) * CPI, gck[k0 + k]);
+        for (int q = 0; q < NSP; ++q) {
+          const long so = (long)(isp0 + q - 1) * g.N;
+          c[k][q].T = s.Ts[so + cbk[kk] + r];
+          c[k][q].n = s.ns[so + cbk[kk] + r];
+          c[k][q].h1 = h1; c[k][q].h2 = h2; c[k][q].h3 = h3;
+        }
+      }
+    }
+  };
+  auto convert = [&](int k0, CellIn<ELEC> (*c)[NSP]) {
 #pragma unroll
-      for (int k = 0; k < NB; ++k) {
+    for (int k = 0; k < NB; ++k) {
+#pragma unroll
+      for (int q = 0; q < NSP; ++q) {
         double C_, B_, D_;
-        cell_coeffs<ELEC, EXT>(in[k], isp, gm1kB, C_, B_, D_);
-        const int cc = (k0 + k) * CPI + cs;
-        sT[lr][cc] = in[k].T; sC[lr][cc] = C_; sB[lr][cc] = B_; sD[lr][cc] = D_;
+        cell_coeffs<ELEC, EXT>(c[k][q], isp0 + q, (gammas(isp0 + q) - 1.0) / kB, C_, B_, D_);
+        const int cc = q * 32 + (k0 + k) * CPI + cs;
+        sT[lr][cc] = c[k][q].T; sC[lr][cc] = C_; sD[lr][cc] = D_;
+        if (ELEC) sB[lr][cc] = B_;
       }
     }
   };
 
-  // walk the rows in chunks; row r's arrival completes the coefficients of row ro = r-1
-  // (2..N-1), handed to `row(ro, real, t1f, t2f, t3f, Tm, Tc, Tp)`; rows before 3 and rows
-  // past N are not real and the handler must leave its state alone for them
-  auto rows = [&](auto row) {
+  // a row of each matrix from its parabolic terms (PDEparabolic.f90:19-145 TR half step,
+  // :146-216 BDF2, :221-346 backward Euler); the ions' drift term is an exact zero
+  auto first_row = [&](double t1f, double t2f, double t3f, double Tm, double Tc, double Tp,
+                       double& a, double& b, double& c, double& d) {
+    if (BE) {
+      a = -t1f + t2f; b = (k1.K + t3f) + t1f; c = -t3f - t2f;
+      d = div_rcp(Tc, k1.dt, k1.K);
+    } else {
+      const double t1 = t1f / 2.0, t2 = t2f / 2.0, t3 = t3f / 2.0;
+      a = -t1 + t2; b = (k1.K + t3) + t1; c = -t3 - t2;
+      d = ((div_rcp(Tc, k1.dt2, k1.K) - a * Tm) - (t3 + t1) * Tc) - c * Tp;
+    }
+  };
+
+  // the record of the electron columns' interchanges (fitting extension, adjoint tapes)
+  const int nw = (N + 31) / 32;
+  int* prec = (EXT && ELEC && s.pivrec) ? s.pivrec + (long)col * 2 * nw : nullptr;
+  int sbits = 0;
+  auto record = [&](int stage, int j, bool swap) {   // step j (1..N-1) of the TR or BDF2 solve
+    if (!(EXT && ELEC) || !prec) return;
+    sbits |= (swap ? 1 : 0) << (j & 31);
+    if ((j & 31) == 31 || j == N - 1) {
+      prec[stage * nw + (j >> 5)] = sbits;
+      sbits = 0;
+    }
+  };
+
+  // ---- pass 1
+  Elim e{1.0, 0.0, Tmin, false};
+  {
     double Tm = 0.0, Tc = 0.0, Cc = 0.0, Bc = 0.0, Dm = 0.0, Dc = 1.0;
-    for (int r0 = 1 - ph1; r0 <= N; r0 += R) {
+    issue(1 - ph, 0, in);
+    for (int m = 0; m <= mb; ++m) {
+      const int r0 = m * R + 1 - ph;
       __builtin_amdgcn_wave_barrier();
-      load_chunk(r0);
+#pragma unroll
+      for (int k0 = 0; k0 < NK; k0 += NB) {
+        CellIn<ELEC> nxt[NB][NSP];
+        if (k0 + NB < NK) issue(r0, k0 + NB, nxt);
+        convert(k0, in);
+        if (k0 + NB < NK) {
+#pragma unroll
+          for (int k = 0; k < NB; ++k) in[k][0] = nxt[k][0];
+        }
+      }
+      issue(r0 + R, 0, in);
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int k = 0; k < R; ++k) {
-        const int r = r0 + k;
-        const double Tp = sT[k][lane], Cp = sC[k][lane], Bp = sB[k][lane], Dp = sD[k][lane];
-        const int ro = r - 1;
-        const int rc = clampi(ro, 2, N - 1);
+        // row r's arrival completes the terms of row ro = r-1 (2..N-1)
+        const int r = r0 + k, ro = r - 1, rc = clampi(ro, 2, N - 1), rs = clampi(ro, 1, N);
+        const double Tp = sT[k][lane], Cp = sC[k][lane], Dp = sD[k][lane];
+        const double Bp = ELEC ? sB[k][lane] : 0.0;
+        const double dxi = ld_row(dx1i, rc), dxl = ld_row(dx1, rc), dxr = ld_row(dx1, rc + 1);
+        const double ydxi = ld_row(g.rdx1i, rc), ydxl = ld_row(g.rdx1, rc), ydxr = ld_row(g.rdx1, rc + 1);
         const double Dhr = 0.5 * (Dm + Dc), Dhr1 = 0.5 * (Dc + Dp);
-        const double t1f = ((Cc * Dhr) / dx1i[rc]) / dx1[rc];
-        const double t3f = ((Cc * Dhr1) / dx1i[rc]) / dx1[rc + 1];
-        const double t2f = Bc / (dx1[rc + 1] + dx1[rc]);
-        row(ro, r >= 3 && r <= N, t1f, t2f, t3f, Tm, Tc, Tp);
+        const double t1f = div_rcp(div_rcp(Cc * Dhr, dxi, ydxi), dxl, ydxl);
+        const double t3f = div_rcp(div_rcp(Cc * Dhr1, dxi, ydxi), dxr, ydxr);
+        const double t2f = ELEC ? div_rcp(Bc, dxr + dxl, ld_row(g.rdx1s, rc)) : 0.0;
+        put(rs, ST1, t1f);
+        put(rs, ST3, t3f);
+        put(rs, STV, Tc);
+        if (ELEC) put(rs, ST2, t2f);
+        if (k == 2) keep_state(m, e);                // before the step of position r0 = r - 2
+        if (r >= 3 && r <= N) {
+          double a, b, c, d;
+          bool sw;
+          first_row(t1f, t2f, t3f, Tm, Tc, Tp, a, b, c, d);
+          elim_step(e, a, b, c, d, sw);
+          record(0, r - 2, sw);
+        }
         Tm = Tc; Tc = Tp;
         Cc = Cp; Bc = Bp;
         Dm = Dc; Dc = Dp;
       }
     }
-  };
+    put(N, STV, Tc);                                 // (the window may end on row N)
+    bool sw;
+    elim_step(e, aN, bN, 0.0, Tmax, sw);             // boundary row N
+    record(0, N - 1, sw);
+    if (mb * R + 1 - ph == N) keep_state(mb, e);     // position N starts its block
+    if (e.r0 == 0.0) e.singular = true;
+  }
 
-  // rows of the first solve (PDEparabolic.f90:19-145 TR half step, :221-346 backward Euler)
-  auto first_row = [&](double t1f, double t2f, double t3f, double Tm, double Tc, double Tp,
-                       double& a, double& b, double& c, double& d) {
-    if (BE) {
-      a = -t1f + t2f; b = (k1.K + t3f) + t1f; c = -t3f - t2f; d = Tc / k1.dt;
-    } else {
-      const double t1 = t1f / 2.0, t2 = t2f / 2.0, t3 = t3f / 2.0;
-      a = -t1 + t2; b = (k1.K + t3) + t1; c = -t3 - t2;
-      d = ((Tc / k1.dt2 - a * Tm) - (t3 + t1) * Tc) - c * Tp;
-    }
+  // The rows of a block's steps: terms of row r = position + 1, reloaded for the next block
+  // as soon as a step has used them.
+  double t1[R], t3[R], t2[ELEC ? R : 1], v[R], ckn[NCK];
+  auto load_terms = [&](int r, int u) {
+    const int rr = clampi(r, 1, N);
+    t1[u] = get(rr, ST1);
+    t3[u] = get(rr, ST3);
+    if (ELEC) t2[u % (ELEC ? R : 1)] = get(rr, ST2);
   };
-
-  // dtbsv over stored pivot rows (slots s0 s1 s2, rhs sy), column-oriented: row i takes
-  // x(i+2)*U2 off first, then x(i+1)*U1, and divides by U0; a zero x(j) contributes
-  // nothing.  Rows are taken in the chunks [kR+1-ph, kR+R-ph] from the top; each chunk's
-  // results go to `put` (rows past N and before 1 too, which must land nowhere that
-  // matters: rows past N come first and are put on row N), then `flush(k)` runs.
-  auto backsub = [&](int s0, int s1, int s2, int sy, bool singular, int ph, auto put,
-                     auto flush) {
-    double pu0[R], pu1[R], pu2[R], py[R];
-    const int kt = (N - 1 + ph) / R;                 // top chunk
-    auto fetch = [&](int i, int u) {
-      const int ic = clampi(i, 1, N);
-      pu0[u] = get2(q, ic, s0); pu1[u] = get2(q, ic, s1); pu2[u] = get2(q, ic, s2);
-      py[u] = get2(q, ic, sy);
-    };
+  auto load_state = [&](int m) {
 #pragma unroll
-    for (int u = 0; u < R; ++u) fetch(kt * R + 1 - ph + u, u);  // row i: slot (i-1+ph) % R
-    double x1 = 0.0, x2 = 0.0;
-    auto row = [&](int i, int u, bool live) {
-      const double u0 = pu0[u], u1 = pu1[u], u2 = pu2[u], y = py[u];
-      fetch(i - R, u);
-      double acc = y;
-      if (!singular) {
-        if (i + 2 <= N && x2 != 0.0) acc = acc - x2 * u2;
-        if (i + 1 <= N && x1 != 0.0) acc = acc - x1 * u1;
-        if (acc != 0.0) acc = acc / u0;
-      }
-      if (live) {
-        x2 = x1;
-        x1 = acc;
-      }
-      put(min(i, N), u, acc);
-    };
-    // top chunk: rows above N are skipped (their put lands on row N before row N's own)
-#pragma unroll
-    for (int u = 0; u < R; ++u) {
-      const int i = kt * R + R - u - ph;
-      row(i, R - 1 - u, i <= N);
-    }
-    flush(kt);
-    for (int k = kt - 1; k >= 0; --k) {
-#pragma unroll
-      for (int u = 0; u < R; ++u) row(k * R + R - u - ph, R - 1 - u, true);
-      flush(k);
-    }
+    for (int q = 0; q < NCK; ++q) ckn[q] = __builtin_nontemporal_load(ck0 + ((long)(m < 0 ? 0 : m) * NCK + q) * 64 + ln);
   };
-
-  // final temperatures go out through LDS, one chunk of R rows (phase pho) at a time; the
-  // slots of rows past N and before 1 are never stored (those lanes store row N or 1 again)
-  auto put_out = [&](int, int u, double x) { sT[u][lane] = fmax_f(x, 100.0); };
-  auto flush_out = [&](int k) {
+  // Final temperatures go out through LDS, one block of R rows at a time (rows past N and
+  // before 1 are never stored: those lanes store row N or 1 again).
+  auto flush_out = [&](int j0) {
     __builtin_amdgcn_wave_barrier();
-    const int r0 = k * R + 1 - pho;
-    const int rr = clampi(r0 + lr, 1, N);
+    const int rr = clampi(j0 + lr, 1, N);
 #pragma unroll
-    for (int kk = 0; kk < R; ++kk) {
-      const int cc = kk * CPI + cs;
-      s.Ts[so + cbk[kk] + rr] = sT[rr - r0][cc];
+    for (int q = 0; q < NSP; ++q) {
+      double* To = s.Ts + (long)(isp0 + q - 1) * g.N;
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) To[cbk[kk] + rr] = sT[rr - j0][q * 32 + kk * CPI + cs];
     }
     __builtin_amdgcn_wave_barrier();
   };
 
-  // the BDF2 factorisation's singular flag, kept between the launches of a split solve
-  int* mysing = lst + (((long)(isp - 1) * gps + cg) * 64 + lane);
-  Elim e{1.0, 0.0, Tmin, false};
-  Fact f{1.0, 0.0, false, 0, 0};
-  if (PH == 2) {
-    f.singular = *mysing != 0;
-  } else {
-  // the record of the electron columns' interchanges (fitting extension, adjoint tapes)
-  const int nw = (N + 31) / 32;
-  int* prec = (EXT && ELEC && s.pivrec) ? s.pivrec + (long)col * 2 * nw : nullptr;
-  int tbits = 0;
-  auto record_tr = [&](int j, bool swap) {   // TR step j (1..N-1)
-    tbits |= (swap ? 1 : 0) << (j & 31);
-    if ((j & 31) == 31 || j == N - 1) {
-      prec[j >> 5] = tbits;
-      tbits = 0;
-    }
+  // A TR factorisation that is singular leaves dgbsv's right-hand side as the solution: the
+  // lanes concerned put the BDF2 right-hand side of that solution in place now (a slow pass
+  // that never runs on physical inputs) and pass 2 leaves it there.
+  const bool tr_sing = __any(e.singular);
+  auto bdf_rhs = [&](double T, double x) {
+    return -div_rcp(bdf.c13 * T, bdf.dt3, bdf.K) + div_rcp(bdf.c43 * x, bdf.dt3, bdf.K);
   };
-  // pass 1
-  rows([&](int ro, bool real, double t1f, double t2f, double t3f, double Tm, double Tc,
-           double Tp) {
-    const int j = ro - 1, sj = clampi(j, 1, N - 1);
-    double a, b, c, d;
-    first_row(t1f, t2f, t3f, Tm, Tc, Tp, a, b, c, d);
-    const bool sw = elim_rhs(q, e, j, sj, real, a, b, c, d);
-    if (EXT && ELEC && prec && real) record_tr(j, sw);
-    if (!BE) {                                       // PDEparabolic.f90:146-216 matrix
-      elim_mat(q, f, j, sj, real, -t1f + t2f, (bdf.K + t3f) + t1f, -t3f - t2f);
-    }
-  });
-  {
-    const bool sw = elim_rhs(q, e, N - 1, N - 1, true, aN, bN, 0.0, Tmax);   // boundary row N
-    if (EXT && ELEC && prec) record_tr(N - 1, sw);
-  }
-  if (e.r0 == 0.0) e.singular = true;
-  S2(q, N, SU0) = e.r0; S2(q, N, SU1) = 0.0; S2(q, N, SU2) = 0.0; S2(q, N, SY) = e.rb;
-  if (!BE) {
-    elim_mat(q, f, N - 1, N - 1, true, aN, bN, 0.0);
-    if (f.r0 == 0.0) f.singular = true;
-    S2(q, N, SV0) = f.r0; S2(q, N, SV1) = 0.0; S2(q, N, SV2) = 0.0;
-    if (EXT && ELEC && prec)                         // the BDF2 interchanges, as stored
-      for (int w = 0; w < nw; ++w) prec[nw + w] = q.swb[w * 64];
-  }
-  // a singular factorisation leaves dgbsv's right-hand side as the solution: for the
-  // lanes concerned, store the first solve's right-hand side in the y slot (a slow pass
-  // that never runs on physical inputs)
-  if (__any(e.singular)) {
-    const bool mine = e.singular;
-    if (mine) S2(q, 1, SY) = Tmin;
-    rows([&](int ro, bool real, double t1f, double t2f, double t3f, double Tm, double Tc,
-             double Tp) {
+  if (!BE && tr_sing && e.singular) {
+    double Tm = get(1, STV), Tc = get(2, STV);
+    for (int r = 2; r <= N - 1; ++r) {
+      const double Tp = get(r + 1, STV);
       double a, b, c, d;
-      first_row(t1f, t2f, t3f, Tm, Tc, Tp, a, b, c, d);
-      if (mine && real) S2(q, ro, SY) = d;
-    });
-    if (mine) S2(q, N, SY) = Tmax;
-  }
-
-  // pass 2
-  __builtin_amdgcn_wave_barrier();
-  if (BE) {
-    backsub(SU0, SU1, SU2, SY, e.singular, pho, put_out, flush_out);
-    return;
-  }
-  backsub(SU0, SU1, SU2, SY, e.singular, 0, [&](int i, int u, double x) { put2(q, i, STR, x); },
-          [&](int) {});
-
-  if (PH == 1) {
-    *mysing = f.singular ? 1 : 0;
-    return;
-  }
-  }  // passes 1 and 2
-
-  // pass 3: d(r) = AT(r) + ((4/3) TR(r))/(dt/3) for rows 2..N-1 (Tmin, Tmax at the ends),
-  // with AT(r) = -((1/3) T(r))/(dt/3) from the input temperature (its column of Ts, which
-  // only pass 4 overwrites), through the interchanges and multipliers of pass 1; singular
-  // lanes keep d itself.  The input temperatures come in R-row chunks loaded by the wave
-  // cooperatively (as pass 1 loads its inputs) into two alternating LDS buffers, the next
-  // chunk's loads in flight while a chunk is used.
-  {
-    constexpr int PF = R;
-    double ptr[PF], pl[PF];
-    double tv[R];
-    auto issue_T = [&](int r0) {                     // rows r0..r0+R-1 (clamped to 1..N)
-      const int rr = clampi(r0 + lr, 1, N);
-#pragma unroll
-      for (int kk = 0; kk < R; ++kk) tv[kk] = s.Ts[so + cbk[kk] + rr];
-    };
-    auto store_T = [&](double (*buf)[LP]) {
-#pragma unroll
-      for (int kk = 0; kk < R; ++kk) buf[lr][kk * CPI + cs] = tv[kk];
-    };
-    const int t0 = 2 - ph3;                          // first row of chunk 0
-    __builtin_amdgcn_wave_barrier();
-    issue_T(t0);
-    store_T(sT);
-    __builtin_amdgcn_wave_barrier();
-    issue_T(t0 + R);
-    auto fetch = [&](int r, int u) {                 // inputs of step j = r-1
-      const int rc = clampi(r, 1, N), jc = clampi(r - 1, 1, N - 1);
-      ptr[u] = get2(q, rc, STR); pl[u] = get2(q, jc, SL);
-    };
-    // the interchange words of a chunk's steps j0 .. j0+PF-1 (at most two), a chunk ahead
-    auto words = [&](int j0, int& w0, int& w1) {
-      w0 = q.swb[(clampi(j0, 1, N - 1) >> 5) * 64];
-      w1 = q.swb[(clampi(j0 + PF - 1, 1, N - 1) >> 5) * 64];
-    };
-#pragma unroll
-    for (int u = 0; u < PF; ++u) fetch(t0 + u, u);
-    const bool fs = f.singular;
-    S2(q, 1, SY) = Tmin;
-    double rb = Tmin;
-    int cw0, cw1, nw0, nw1;
-    words(t0 - 1, cw0, cw1);
-    int ch = 0;                                      // chunk of rows t0 + ch R ..
-    for (int j0 = t0 - 1; j0 <= N - 1; j0 += PF, ++ch) {
-      double (*tb)[LP] = (ch & 1) ? sC : sT;
-      words(j0 + PF, nw0, nw1);
-      const int jw0 = clampi(j0, 1, N - 1) >> 5;
-#pragma unroll
-      for (int u = 0; u < PF; ++u) {
-        const int j = j0 + u, r = j + 1;
-        const double at = -((bdf.c13 * tb[u][lane]) / bdf.dt3), trr = ptr[u], l = pl[u];
-        const int bits = (clampi(j, 1, N - 1) >> 5) == jw0 ? cw0 : cw1;
-        fetch(r + PF, u);
-        const bool live = j >= 1 && j <= N - 1;
-        const double d = r >= N ? Tmax : at + (bdf.c43 * trr) / bdf.dt3;
-        const bool swap = (bits >> (j & 31)) & 1;
-        const double pd = swap ? d : rb;
-        double od = swap ? rb : d;
-        if (!fs && pd != 0.0) od = od + l * (-pd);
-        // steps past N-1 store on row N, which the store after the loop overwrites
-        put2(q, live ? (fs ? r : j) : N, SY, fs ? d : pd);
-        rb = live ? od : rb;
-      }
-      cw0 = nw0;
-      cw1 = nw1;
-      __builtin_amdgcn_wave_barrier();
-      store_T((ch & 1) ? sT : sC);                   // chunk ch + 1
-      __builtin_amdgcn_wave_barrier();
-      issue_T(t0 + (ch + 2) * R);
+      first_row(get(r, ST1), ELEC ? get(r, ST2) : 0.0, get(r, ST3), Tm, Tc, Tp, a, b, c, d);
+      put(r, STV, bdf_rhs(Tc, d));
+      Tm = Tc; Tc = Tp;
     }
-    S2(q, N, SY) = fs ? Tmax : rb;
   }
 
-  // pass 4
-  backsub(SV0, SV1, SV2, SY, f.singular, pho, put_out, flush_out);
+  // ---- pass 2
+  {
+    double x1 = 0.0, x2 = 0.0, va = 0.0, vb = 0.0;   // va, vb: temperatures of the two rows above
+    auto block = [&](auto edge_, int m) {
+      constexpr bool EDGE = decltype(edge_)::value;
+      const int j0 = m * R + 1 - ph;
+      Elim q{ckn[0], ckn[1], ckn[2], false};
+      double w[R + 2];
+      Pivot P[R];
+#pragma unroll
+      for (int u = 0; u < R; ++u) w[u] = v[u];
+      w[R] = va; w[R + 1] = vb;
+      va = w[0]; vb = w[1];
+      load_state(m - 1);
+#pragma unroll
+      for (int u = 0; u < R; ++u) v[u] = get(clampi(j0 - R + u, 1, N), STV);
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int j = j0 + u;                        // row j+1 comes in
+        double a, b, c, d;
+        bool sw;
+        first_row(t1[u], ELEC ? t2[u % (ELEC ? R : 1)] : 0.0, t3[u], w[u], w[u + 1], w[u + 2], a, b, c, d);
+        load_terms(j + 1 - R, u);
+        if (EDGE && j >= N - 1) { a = aN; b = bN; c = 0.0; d = Tmax; }
+        if (EDGE && j >= N) P[u] = Pivot{q.r0, 0.0, 0.0, q.rb};
+        else if (!EDGE || j >= 1) P[u] = elim_step(q, a, b, c, d, sw);
+        else P[u] = Pivot{1.0, 0.0, 0.0, 0.0};
+      }
+#pragma unroll
+      for (int u = R - 1; u >= 0; --u) {
+        const int i = j0 + u;
+        if (EDGE && (i > N || i < 1)) continue;
+        double x = back_step(P[u], x1, x2);
+        if (BE) {
+          if (tr_sing && e.singular) x = i == 1 ? Tmin : i == N ? Tmax : div_rcp(w[u], k1.dt, k1.K);
+          sT[u][lane] = fmax_f(x, 100.0);
+        } else {
+          double d = bdf_rhs(w[u], x);
+          if (tr_sing && e.singular) d = w[u];       // (already the right-hand side)
+          put(i, STV, d);
+        }
+        x2 = x1;
+        x1 = x;
+      }
+      if (BE) flush_out(j0);
+    };
+    load_state(mb);
+    {
+      const int j0 = mb * R + 1 - ph;
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        v[u] = get(clampi(j0 + u, 1, N), STV);
+        load_terms(j0 + u + 1, u);
+      }
+    }
+    for (int m = mb; m >= 0; --m) {
+      const int j0 = m * R + 1 - ph;
+      if (j0 >= 1 && j0 + R <= N - 1) block(std::false_type{}, m);
+      else block(std::true_type{}, m);
+    }
+  }
+  if (BE) return;
+
+  // ---- pass 3: the BDF2 elimination; v holds the right-hand sides of the steps' rows
+  Elim f{1.0, 0.0, Tmin, false};
+  auto load_row = [&](int r, int u) {
+    load_terms(r, u);
+    v[u] = get(clampi(r, 1, N), STV);
+  };
+  auto bdf_row = [&](int u, double& a, double& b, double& c, double& d) {
+    const double t2f = ELEC ? t2[u % (ELEC ? R : 1)] : 0.0;
+    a = -t1[u] + t2f; b = (bdf.K + t3[u]) + t1[u]; c = -t3[u] - t2f; d = v[u];
+  };
+  {
+#pragma unroll
+    for (int u = 0; u < R; ++u) load_row(2 - ph + u, u);
+    auto block = [&](auto edge_, int m) {
+      constexpr bool EDGE = decltype(edge_)::value;
+      const int j0 = m * R + 1 - ph;
+      keep_state(m, f);
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int j = j0 + u;
+        double a, b, c, d;
+        bool sw;
+        bdf_row(u, a, b, c, d);
+        load_row(j + 1 + R, u);
+        if (EDGE && (j < 1 || j > N - 1)) continue;
+        if (EDGE && j == N - 1) { a = aN; b = bN; c = 0.0; d = Tmax; }
+        elim_step(f, a, b, c, d, sw);
+        record(1, j, sw);
+      }
+    };
+    for (int m = 0; m <= mb; ++m) {
+      const int j0 = m * R + 1 - ph;
+      if (j0 >= 1 && j0 + R <= N - 1) block(std::false_type{}, m);
+      else block(std::true_type{}, m);
+    }
+    if (f.r0 == 0.0) f.singular = true;
+  }
+
+  // ---- pass 4
+  {
+    double x1 = 0.0, x2 = 0.0;
+    auto block = [&](auto edge_, int m) {
+      constexpr bool EDGE = decltype(edge_)::value;
+      const int j0 = m * R + 1 - ph;
+      Elim q{ckn[0], ckn[1], ckn[2], false};
+      Pivot P[R];
+      load_state(m - 1);
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int j = j0 + u;
+        double a, b, c, d;
+        bool sw;
+        bdf_row(u, a, b, c, d);
+        load_row(j + 1 - R, u);
+        if (EDGE && j >= N - 1) { a = aN; b = bN; c = 0.0; d = Tmax; }
+        if (EDGE && j >= N) P[u] = Pivot{q.r0, 0.0, 0.0, q.rb};
+        else if (!EDGE || j >= 1) P[u] = elim_step(q, a, b, c, d, sw);
+        else P[u] = Pivot{1.0, 0.0, 0.0, 0.0};
+      }
+#pragma unroll
+      for (int u = R - 1; u >= 0; --u) {
+        if (EDGE && (j0 + u > N || j0 + u < 1)) continue;
+        const double x = back_step(P[u], x1, x2);
+        sT[u][lane] = fmax_f(x, 100.0);
+        x2 = x1;
+        x1 = x;
+      }
+      flush_out(j0);
+    };
+    load_state(mb);
+    {
+      const int j0 = mb * R + 1 - ph;
+#pragma unroll
+      for (int u = 0; u < R; ++u) load_row(j0 + u + 1, u);
+    }
+    for (int m = mb; m >= 0; --m) {
+      const int j0 = m * R + 1 - ph;
+      if (j0 >= 1 && j0 + R <= N - 1) block(std::false_type{}, m);
+      else block(std::true_type{}, m);
+    }
+  }
+  // a singular BDF2 factorisation likewise (slow, never on physical inputs): the right-hand
+  // sides, which pass 4 left in place, are the solution
+  if (__any(f.singular) && f.singular) {
+    int a2, a3;
+    column_of(g, col, a2, a3);
+    double* To = s.Ts + (long)(isp - 1) * g.N + gix(g, 0, a2, a3);
+    for (int r = 1; r <= N; ++r) {
+      const double d = r == 1 ? Tmin : r == N ? Tmax : get(r, STV);
+      To[r] = fmax_f(d, 100.0);
+    }
+  }
 }
 
-// PH 0: the whole solve; for a solve split in two launches, PH 1 runs passes 1-2 and
-// PH 2 passes 3-4 (shorter waves, so the last wave round leaves less of the GPU idle)
-template <int R, bool BE, int PH, bool EXT = false>
-__global__ __launch_bounds__(64) void k_diffusion(DevGrid g, DevState s, double* scratch,
-                                                  int* swbits, int* lst, Coef k1, Coef bdf,
-                                                  double Teinf) {
-  __shared__ double sT[R][LP], sC[R][LP], sB[R][LP], sD[R][LP];
-  const long ncol = (long)g.lx2 * g.lx3;
-  const long gps = (ncol + 63) / 64;                 // column groups per species
-  // the electron groups first (their waves are the longest, so the last wave round is
-  // shorter), then the six ion species of each run of 8 groups; block b runs on XCD b % 8,
-  // and every species of column group cg on XCD cg % 8
-  const long ne = (gps + 7) / 8 * 8;
-  long cg;
-  int isp;
-  if ((long)blockIdx.x < ne) {
-    cg = blockIdx.x;
-    isp = LSP;
-  } else {
-    const long b = blockIdx.x - ne, slot = b / 8;
-    cg = (slot / (LSP - 1)) * 8 + b % 8;
-    isp = (int)(slot % (LSP - 1)) + 1;
+// Unit v of a launch: the electron groups first (their waves are the longest, so the last
+// wave round is shorter), then the six ion units of each run of 8 groups; unit v runs on XCD
+// v % 8, and every unit of column group cg on XCD cg % 8.
+template <int R, bool BE, bool EXT>
+__device__ __forceinline__ void diffusion_block(const DevGrid& g, const DevState& s, long v,
+                                                double* scratch, const Coef& k1, const Coef& bdf,
+                                                double Teinf, double (*sT)[LP], double (*sC)[LP],
+                                                double (*sB)[LP], double (*sD)[LP]) {
+  const long gps = diffusion_groups(g), ne = (gps + 7) / 8 * 8;
+  if (v < ne) {
+    if (v < gps)
+      diffusion_unit<R, BE, true, EXT>(g, s, scratch, k1, bdf, Teinf, v, 0, 0, sT, sC, sB, sD);
+    return;
   }
-  if (cg >= gps) return;
-  if (isp == LSP)
-    diffusion_group<R, BE, true, PH, EXT>(g, s, scratch, swbits, lst, k1, bdf, Teinf, isp, cg,
-                                          gps, sT, sC, sB, sD);
-  else
-    diffusion_group<R, BE, false, PH, EXT>(g, s, scratch, swbits, lst, k1, bdf, Teinf, isp, cg,
-                                           gps, sT, sC, sB, sD);
+  const long b = v - ne, slot = b / 8, cg = slot / 6 * 8 + b % 8;
+  const int half = (int)(slot % 6) / 3, pair = (int)(slot % 6) % 3;
+  // (a half past the last column has none of its own)
+  if (cg >= gps || (!group_interleaved(g, cg) && cg * 64 + half * 32 >= (long)g.lx2 * g.lx3)) return;
+  diffusion_unit<R, BE, false, EXT>(g, s, scratch, k1, bdf, Teinf, cg, half, pair, sT, sC, sB, sD);
+}
+
+template <int R, bool BE, bool EXT = false>
+__global__ __launch_bounds__(64, 2) void k_diffusion(DevGrid g, DevState s, double* scratch,
+                                                     Coef k1, Coef bdf, double Teinf) {
+  __shared__ double sT[R][LP], sC[R][LP], sB[R][LP], sD[R][LP];
+  diffusion_block<R, BE, EXT>(g, s, blockIdx.x, scratch, k1, bdf, Teinf, sT, sC, sB, sD);
 }
 
 }  // namespace
@@ -562,60 +610,50 @@ __global__ __launch_bounds__(64) void k_diffusion(DevGrid g, DevState s, double*
 void launch_floor_ghosts(const DevGrid& g, double* Ts, hipStream_t st);
 
 namespace {
-// layout of a grid's diffusion work space: the pivot-row slots of every column group, the
-// BDF2 interchange words, one singular flag per lane
-__host__ __device__ inline long diffusion_groups(const DevGrid& g) {
-  return ((long)g.lx2 * g.lx3 + 63) / 64 * LSP;
+__host__ __device__ inline Coef tr_coef(double dt) {
+  Coef c{};
+  c.dt2 = dt / 2.0; c.K = 1.0 / c.dt2; c.dt = dt;
+  return c;
 }
-__host__ __device__ inline size_t factor_bytes(const DevGrid& g) {
-  return (size_t)diffusion_groups(g) * (size_t)g.lx1 * NSLOT * 64 * sizeof(double);
+__host__ __device__ inline Coef bdf_coef(double dt) {
+  Coef c{};
+  c.dt3 = dt / 3.0; c.K = 1.0 / c.dt3; c.dt = dt;
+  c.c13 = 1.0 / 3.0; c.c43 = 4.0 / 3.0;
+  return c;
 }
-__host__ __device__ inline size_t swap_bytes(const DevGrid& g) {
-  return (size_t)diffusion_groups(g) * ((g.lx1 + 31) / 32) * 64 * sizeof(int);
+
+__device__ __forceinline__ double uniform_double(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ BatchMember load_uniform(const BatchMember* p) {
+  BatchMember b;
+  static_assert(sizeof(BatchMember) % 4 == 0, "copied by words");
+  const auto* w = (const __attribute__((address_space(4))) int*)p;
+#pragma unroll
+  for (unsigned k = 0; k < sizeof(BatchMember) / 4; ++k) ((int*)&b)[k] = w[k];
+  return b;
 }
 
 // The TRBDF2 solve of every member of a batched step: a persistent grid of one-wave blocks
-// taking the members' column groups in turn, numbered as each member's own launch numbers
-// them (every member's count is a multiple of 8, so a group keeps its XCD).  The
-// coefficients are formed from each member's dt as launch_energy_diffusion forms them.
+// taking the members' units in turn, numbered as each member's own launch numbers them
+// (every member's count is a multiple of 8, so a group keeps its XCD).  The coefficients are
+// formed from each member's dt as launch_energy_diffusion forms them.
 template <int R>
 __global__ __launch_bounds__(64, 2) void kb_diffusion(const BatchMember* M, const long* pre, int n,
-                                                   long total) {
+                                                      long total) {
   __shared__ double sT[R][LP], sC[R][LP], sB[R][LP], sD[R][LP];
   const long* p = pre + (long)BK_DIFF * (n + 1);
   for (long t = blockIdx.x; t < total; t += gridDim.x) {
-    const int m = batch_member(p, n, t);
-    const DevGrid& g = M[m].g;
-    const DevState& s = M[m].s;
-    const long v = t - p[m];
-    const long ncol = (long)g.lx2 * g.lx3;
-    const long gps = (ncol + 63) / 64;
-    const long ne = (gps + 7) / 8 * 8;               // (k_diffusion's numbering)
-    long cg;
-    int isp;
-    if (v < ne) {
-      cg = v;
-      isp = LSP;
-    } else {
-      const long b = v - ne, slot = b / 8;
-      cg = (slot / (LSP - 1)) * 8 + b % 8;
-      isp = (int)(slot % (LSP - 1)) + 1;
-    }
-    if (cg >= gps) continue;
-    const double dt = M[m].dt;
-    Coef tr{}, bdf{};
-    tr.dt2 = dt / 2.0; tr.K = 1.0 / tr.dt2; tr.dt = dt;
-    bdf.dt3 = dt / 3.0; bdf.K = 1.0 / bdf.dt3; bdf.dt = dt;
-    bdf.c13 = 1.0 / 3.0; bdf.c43 = 4.0 / 3.0;
-    double* scratch = M[m].scratch;
-    int* swbits = (int*)((char*)scratch + factor_bytes(g));
-    int* lst = (int*)((char*)swbits + swap_bytes(g));
-    if (isp == LSP)
-      diffusion_group<R, false, true, 0, false>(g, s, scratch, swbits, lst, tr, bdf, M[m].Teinf,
-                                                isp, cg, gps, sT, sC, sB, sD);
-    else
-      diffusion_group<R, false, false, 0, false>(g, s, scratch, swbits, lst, tr, bdf, M[m].Teinf,
-                                                 isp, cg, gps, sT, sC, sB, sD);
+    // (the member's table entry by scalar loads: as vector loads its 60 uniform values took
+    // vector registers, and the kernel spilled)
+    const int m = __builtin_amdgcn_readfirstlane(batch_member(p, n, t));
+    const BatchMember b = load_uniform(M + m);
+    Coef tr = tr_coef(b.dt), bdf = bdf_coef(b.dt);
+    tr.dt2 = uniform_double(tr.dt2); tr.K = uniform_double(tr.K);
+    bdf.dt3 = uniform_double(bdf.dt3); bdf.K = uniform_double(bdf.K);
+    diffusion_block<R, false, false>(b.g, b.s, t - p[m], b.scratch, tr, bdf, b.Teinf, sT, sC, sB, sD);
   }
 }
 }  // namespace
@@ -637,20 +675,39 @@ __global__ void k_fill_hcol(DevGrid g, double* hcol) {
     hcol[2 * g.hstride + t] = g.h3[cb + r];
   }
 }
+// the correctly rounded reciprocals of the row divisors (DevGrid::rdx1, rdx1i, rdx1s, each
+// indexed as its divisor, 0..lx1+2)
+__global__ void k_fill_rdx(DevGrid g, double* r) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, L = g.lx1 + 3;
+  if (i >= L) return;
+  r[i] = 1.0 / g.dx1[i];
+  r[L + i] = 1.0 / g.dx1i[clampi(i - 1, 0, g.lx1 - 1)];
+  r[2 * L + i] = 1.0 / (g.dx1[min(i + 1, g.lx1 + 2)] + g.dx1[i]);
+}
 
 long pivot_record_ints(const DevGrid& g) { return (long)g.lx2 * g.lx3 * 2 * ((g.lx1 + 31) / 32); }
 
 long diffusion_hcol_doubles(const DevGrid& g) {
   return 3 * (((long)g.lx2 * g.lx3 + 63) / 64) * g.lx1 * 64;
 }
+long diffusion_rdx_doubles(const DevGrid& g) { return 3L * (g.lx1 + 3); }
 
-void launch_fill_hcol(const DevGrid& g, double* hcol, hipStream_t st) {
+void launch_fill_hcol(const DevGrid& g, double* hcol, double* rdx, hipStream_t st) {
   hipLaunchKernelGGL(k_fill_hcol, dim3(4096), dim3(256), 0, st, g, hcol);
+  hipLaunchKernelGGL(k_fill_rdx, dim3((g.lx1 + 3 + 255) / 256), dim3(256), 0, st, g, rdx);
 }
 
-// pivot rows, right-hand sides and solutions, the BDF2 interchange bits, one flag per lane
+// the kept rows and elimination states of every unit
 size_t diffusion_scratch_bytes(const DevGrid& g) {
-  return factor_bytes(g) + swap_bytes(g) + (size_t)diffusion_groups(g) * 64 * sizeof(int);
+  const size_t gps = (size_t)diffusion_groups(g);
+  return gps * (size_t)(unit_doubles(g, true) + 6 * unit_doubles(g, false)) * sizeof(double);
+}
+
+// the size a grid is held to by the allocation-free entry point, whose limit is part of its
+// interface: nine doubles, an interchange bit and a flag per row and system of 64-column groups
+size_t diffusion_noalloc_bytes(const DevGrid& g) {
+  const size_t sys = (size_t)diffusion_groups(g) * LSP * 64;
+  return sys * ((size_t)g.lx1 * 9 * sizeof(double) + (size_t)((g.lx1 + 31) / 32 + 1) * sizeof(int));
 }
 
 namespace {
@@ -658,27 +715,13 @@ template <int R>
 void diffusion_launch(const DevGrid& g, const DevState& s, int diffsolvetype, double Teinf,
                       double* scratch, const Coef& tr, const Coef& bdf, const Coef& be,
                       hipStream_t st) {
-  const long ncol = (long)g.lx2 * g.lx3;
-  const long blocks = ((ncol + 63) / 64 + 7) / 8 * 8 * LSP;   // XCD-major numbering
-  int* swbits = (int*)((char*)scratch + factor_bytes(g));
-  int* lst = (int*)((char*)swbits + swap_bytes(g));
-  const dim3 grd((unsigned)blocks), blk(64);
-  if (diffsolvetype == 1) {
-    hipLaunchKernelGGL((k_diffusion<R, true, 0>), grd, blk, 0, st, g, s, scratch, swbits, lst, be,
-                       bdf, Teinf);
-  } else if (s.kappa || s.qtop) {                     // fitting extension (TRBDF2 only; the
-    // 4-row chunk keeps two waves per SIMD with the extension's extra registers)
-    hipLaunchKernelGGL((k_diffusion<4, false, 0, true>), grd, blk, 0, st, g, s, scratch, swbits,
-                       lst, tr, bdf, Teinf);
-  } else if (DIFF_SPLIT) {
-    hipLaunchKernelGGL((k_diffusion<R, false, 1>), grd, blk, 0, st, g, s, scratch, swbits, lst, tr,
-                       bdf, Teinf);
-    hipLaunchKernelGGL((k_diffusion<R, false, 2>), grd, blk, 0, st, g, s, scratch, swbits, lst, tr,
-                       bdf, Teinf);
-  } else {
-    hipLaunchKernelGGL((k_diffusion<R, false, 0>), grd, blk, 0, st, g, s, scratch, swbits, lst, tr,
-                       bdf, Teinf);
-  }
+  const dim3 grd((unsigned)((diffusion_groups(g) + 7) / 8 * 8 * LSP)), blk(64);
+  if (diffsolvetype == 1)
+    hipLaunchKernelGGL((k_diffusion<R, true>), grd, blk, 0, st, g, s, scratch, be, bdf, Teinf);
+  else if (s.kappa || s.qtop)                         // fitting extension (TRBDF2 only)
+    hipLaunchKernelGGL((k_diffusion<R, false, true>), grd, blk, 0, st, g, s, scratch, tr, bdf, Teinf);
+  else
+    hipLaunchKernelGGL((k_diffusion<R, false>), grd, blk, 0, st, g, s, scratch, tr, bdf, Teinf);
 }
 }  // namespace
 
@@ -697,14 +740,13 @@ void launch_batch_diffusion(const BatchTable& t, int diff_chunk, hipStream_t st)
 void launch_energy_diffusion(const DevGrid& g, const DevState& s, double dt, int diffsolvetype,
                              double Teinf, double* scratch, hipStream_t st, const Tuning& tune,
                              bool floor_ghosts) {
-  Coef tr{}, bdf{}, be{};
-  tr.dt2 = dt / 2.0; tr.K = 1.0 / tr.dt2; tr.dt = dt;
-  bdf.dt3 = dt / 3.0; bdf.K = 1.0 / bdf.dt3; bdf.dt = dt;
-  bdf.c13 = 1.0 / 3.0; bdf.c43 = 4.0 / 3.0;
+  Coef be{};
   be.dt = dt; be.K = 1.0 / dt;
   timing_begin("trbdf2", st);
-  if (tune.diff_chunk == 4) diffusion_launch<4>(g, s, diffsolvetype, Teinf, scratch, tr, bdf, be, st);
-  else diffusion_launch<DIFF_CHUNK>(g, s, diffsolvetype, Teinf, scratch, tr, bdf, be, st);
+  if (tune.diff_chunk == 4)
+    diffusion_launch<4>(g, s, diffsolvetype, Teinf, scratch, tr_coef(dt), bdf_coef(dt), be, st);
+  else
+    diffusion_launch<DIFF_CHUNK>(g, s, diffsolvetype, Teinf, scratch, tr_coef(dt), bdf_coef(dt), be, st);
   timing_end("trbdf2", st);
   if (!floor_ghosts) return;
   timing_begin("floor_ghosts", st);

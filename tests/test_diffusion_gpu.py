@@ -1,0 +1,56 @@
+"""GPU: the energy diffusion at the edges of its tiling, bit for bit against the oracle (with
+the GPU's correctly rounded x**2.5): lines a block of kept rows shorter or longer by one,
+column counts around a half group of 32, a group of 64 and an interleaved block of 128, both
+solvers and both chunk heights; and x**2.5 outside the range of its fast form."""
+import numpy as np
+import pytest
+
+import gemini_amd as ga
+import oracle
+from gemini_amd.transport import Transport
+from helpers import compare
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [(4, 1, 1), (5, 7, 3), (7, 8, 4), (8, 31, 1), (9, 32, 1), (10, 33, 1),
+                                   (15, 9, 7), (16, 13, 5), (17, 8, 16), (18, 43, 3), (23, 3, 43),
+                                   (24, 16, 17), (33, 20, 13), (40, 14, 14)])
+@pytest.mark.parametrize("solver", [2, 1])
+def test_diffusion_tiles_match_oracle(shape, solver):
+    print(f"case {shape} solver {solver}", flush=True)
+    grid = ga.dipole_grid if shape[1] > 1 and shape[2] % 2 else ga.cartesian_grid
+    g = grid(*shape)
+    st = ga.synthetic_state(g, seed=sum(shape))
+    # temperatures that vary from row to row, so that rows interchange in both solves
+    st.Ts[...] *= np.random.default_rng(1).uniform(0.5, 2.0, st.Ts.shape)
+    np.maximum(st.Ts, 100.0, out=st.Ts)
+    ref = st.copy()
+    with oracle.pow_mode(1):
+        oracle.op(g, ref, "energy_diffusion", dt=0.3, diffsolvetype=solver)
+    tr = Transport(g, st.nn, st.Tn, own_context=True, diffsolvetype=solver)
+    for chunk in (8, 4):
+        tr.set_tuning("diff_chunk", chunk)
+        got = st.copy()
+        tr.energy_diffusion(got, 0.3)
+        compare(got, ref, exact=("Ts", "ns"))
+    tr.close()
+
+
+def test_pow25_outside_its_fast_range():
+    g = ga.cartesian_grid(8, 4, 3)
+    st = ga.synthetic_state(g)
+    tr = Transport(g, st.nn, st.Tn, own_context=True)
+    m = np.random.default_rng(2).uniform(1.0, 4.0, 4096)
+    core = tr.eval_math(0, m)
+    for k in (-280, -205, 201, 202):               # results stay normal numbers
+        x = np.ldexp(m, 2 * k)
+        x[::3] = m[::3]                            # waves that hold both kinds
+        want = np.ldexp(core, 5 * k)
+        want[::3] = core[::3]
+        fin = np.isfinite(want) & (np.abs(want) >= 2.0 ** -1022)
+        assert np.array_equal(tr.eval_math(0, x)[fin], want[fin])
+    x = np.array([0.0, -0.0, np.inf, np.nan, -1.0, 1e300, 1e-300, 5e-324, 1.0, 4.0])
+    want = np.array([0.0, 0.0, np.inf, np.nan, np.nan, np.inf, 0.0, 0.0, 1.0, 32.0])
+    assert np.array_equal(tr.eval_math(0, x), want, equal_nan=True)
+    tr.close()
