@@ -504,7 +504,7 @@ int gemhip_register_grid(int xtype, int gridflag, int flagper, const int* isglob
   c.d_geom = nullptr;
   // every array starts 256-byte aligned (the sweeps' DMA loads read 16-byte pairs)
   if (!hipok(hipMalloc((void**)&c.d_geom, (total + 20 * 32 + 3 * g.hstride +
-                                             diffusion_rdx_doubles(g)) * sizeof(double)),
+                                             rdx_doubles(g)) * sizeof(double)),
              "geometry"))
     return 5;
   const double** dst[] = {&g.h1, &g.h2, &g.h3, &g.h1x1i, &g.h2x1i, &g.h3x1i, &g.h1x2i, &g.h2x2i,
@@ -520,11 +520,8 @@ int gemhip_register_grid(int xtype, int gridflag, int flagper, const int* isglob
   }
   off = (off + 31) & ~31L;                     // 256-byte aligned rows of 64 columns
   g.hcol = c.d_geom + off;                     // the diffusion's copy of h1, h2, h3
-  double* rdx = c.d_geom + off + 3 * g.hstride;
-  g.rdx1 = rdx;
-  g.rdx1i = rdx + (c.lx1 + 3);
-  g.rdx1s = rdx + 2 * (c.lx1 + 3);
-  launch_fill_hcol(g, c.d_geom + off, rdx, c.stream);
+  launch_fill_hcol(g, c.d_geom + off, c.stream);
+  launch_fill_rdx(g, c.d_geom + off + 3 * g.hstride, c.stream);
   if (!hipok(hipStreamSynchronize(c.stream), "geometry reorder")) return 6;
   g.gridflag = gridflag;
   g.flagper = flagper ? 1 : 0;
@@ -704,7 +701,7 @@ int run_step(double dt, double* tape) {
   launch_sweep(g, s, 1, F_ALL, dt, true, st, c.tune);   // :178-180
   halo_fields({NS, RHOVS1, RHOES});                      // :181
   if (tape) keep(3, s.rhoes);
-  if (!tape && postconvert_fusable(g)) {                 // :183-186 with the conversions
+  if (!tape && postconvert_fusable(g) && postconvert_pays(g)) {                 // :183-186 with the conversions
     launch_sweep2_postconvert(g, s, dt, st, c.tune);     // folded into the x2 sweep
   } else {
     launch_sweep(g, s, 2, F_ALL, dt, true, st, c.tune);  // :183-185

@@ -26,8 +26,8 @@ struct DevGrid {
   // lane) the column's group and lane (hcol_index in diffusion_cell.h)
   const double* hcol;
   long hstride;
-  // correctly rounded reciprocals of dx1(i), dx1i(i) and dx1(i+1) + dx1(i) at index i
-  const double *rdx1, *rdx1i, *rdx1s;
+  // correctly rounded reciprocals of dx(i), dxi(i) and dx(i+1) + dx(i), at index i (0..lx+2)
+  const double *rdx1, *rdx1i, *rdx1s, *rdx2, *rdx2i, *rdx2s, *rdx3, *rdx3i, *rdx3s;
 };
 
 // State pointers in HBM.  ns..Ts point into one fluidvars block of 35 fields,
@@ -97,6 +97,7 @@ void launch_sweep3_preconvert(const DevGrid& g, const DevState& s, double dt, hi
                               const Tuning& tune);
 // the fused step's x2 sweep with rhov12v1 + rhoe2T folded in (x2 not a single cell)
 bool postconvert_fusable(const DevGrid& g);
+bool postconvert_pays(const DevGrid& g);
 void launch_sweep2_postconvert(const DevGrid& g, const DevState& s, double dt, hipStream_t st,
                                const Tuning& tune);
 void launch_halo_periodic(const DevGrid& g, double* const* fields, int nfields, int lhalo,
@@ -114,8 +115,9 @@ void launch_sweep(const DevGrid& g, const DevState& s, int dir, int fields, doub
 // ---- launchers (kernels_diffusion.hip) ----
 size_t diffusion_scratch_bytes(const DevGrid& g);
 long diffusion_hcol_doubles(const DevGrid& g);              // size of DevGrid::hcol
-long diffusion_rdx_doubles(const DevGrid& g);               // and of rdx1, rdx1i, rdx1s together
-void launch_fill_hcol(const DevGrid& g, double* hcol, double* rdx, hipStream_t st);
+void launch_fill_hcol(const DevGrid& g, double* hcol, hipStream_t st);
+long rdx_doubles(const DevGrid& g);                         // size of rdx1 .. rdx3s together
+void launch_fill_rdx(DevGrid& g, double* rdx, hipStream_t st);   // fills and points at them
 size_t diffusion_noalloc_bytes(const DevGrid& g);           // the allocation-free entry's measure
 
 // ---- batched ensemble steps (kernels_advec.hip, kernels_diffusion.hip) ----
@@ -135,9 +137,9 @@ enum BatchKernel : int {
   BK_BC2,    // x2 ghost fill: threads, L1 L3 lsp (times 4 fields in blockIdx.y)
   BK_BC3,    // x3 ghost fill: threads, L1 L2 lsp (times 4 fields in blockIdx.y)
   BK_V1B,    // x1 boundary interface velocities: threads, lx2 lx3 lsp
-  BK_SW3,    // x3 sweep with the conversions: blocks (64 x 7), sweep_blocks(ceil(lx1/64), lx2)
+  BK_SW3,    // x3 sweep with the conversions: blocks (64 x 8), sweep_blocks(ceil(lx1/64), lx2)
   BK_SW1,    // x1 sweep (the electron wave: energy only): blocks (64 x 7), lx2 lx3
-  BK_SW2,    // x2 sweep with rhov12v1 + rhoe2T: blocks (64 x 7), sweep_blocks(.., lx3)
+  BK_SW2,    // x2 sweep with rhov12v1 + rhoe2T: blocks (64 x 8), sweep_blocks(.., lx3)
   BK_POST,   // rhov12v1 + rhoe2T outside the interior box: threads, surface cells
   BK_DIFF,   // TRBDF2: blocks (64), 8 ceil(ceil(lx2 lx3/64)/8) lsp (a multiple of 8)
   BK_FLOOR,  // Ts ghost floor: threads, surface cells lsp

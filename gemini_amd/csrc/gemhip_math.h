@@ -54,15 +54,12 @@ GEMHIP_HD double fmax_f(double a, double b) { return (b > a) ? b : a; }
 
 // x / b from y = RN(1/b), correctly rounded: q0 = RN(x y) is within a few ulps of x/b,
 // the FMA residual x - b q0 is exact, and one correction step q0 + r y, rounded once,
-// gives RN(x/b) (Markstein's theorem for a correctly rounded reciprocal).  Where the
-// residual is zero (exact quotients, zero numerators: q0 has the sign IEEE division gives)
-// or not a number (infinite numerators) or infinite (a quotient past the largest double) q0
-// is the quotient.
+// gives RN(x/b) (Markstein's theorem for a correctly rounded reciprocal).  v_div_fixup_f64
+// gives the quotients of zeros (with their sign), infinities and NaN.
 __device__ __forceinline__ double div_rcp(double x, double b, double y) {
   const double q0 = x * y;
   const double r = __builtin_fma(-b, q0, x);
-  const double q1 = __builtin_fma(r, y, q0);
-  return __builtin_amdgcn_class(r, 0x267) ? q0 : q1;   // sNaN qNaN -inf -0 +0 +inf
+  return __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q0), b, x);
 }
 
 // advec.f90:438-447

@@ -640,12 +640,6 @@ __global__ __launch_bounds__(448) void k_sweep1(DevGrid g, DevState s, SweepFiel
 #ifndef SWEEP1_RCP
 #define SWEEP1_RCP 1          // x1 sweep: divisions through the line's reciprocals where they fit
 #endif
-#ifndef SWEEP1_E7_IN_BLOCK
-#define SWEEP1_E7_IN_BLOCK 1  // x1: electrons as a seventh wave of the species block
-#endif
-#ifndef SWEEP_E7_IN_BLOCK
-#define SWEEP_E7_IN_BLOCK 1   // x2/x3: electrons as a seventh wave of the species block
-#endif
 #ifndef SWEEP23_WAVES
 #define SWEEP23_WAVES         // e.g. __attribute__((amdgpu_waves_per_eu(3))) to cap registers
 #endif
@@ -675,13 +669,23 @@ template <int PF>
 constexpr int sweep_xch_doubles() { return 2 * PF * (LSP - 1) * 2 * 64; }
 
 // block (bx, by): i1 = 64 bx + lane + 1 (lanes past lx1 redo column lx1), line by + 1
-// The fused step's sweeps (CONV or POST: blocks of the 7 species waves) share the metric
-// factors of each step through LDS: waves 0-5 each load one of hI, hA, hB (interface k)
-// and h1, h2, h3 (cell k-1) two groups of steps ahead and store them one group ahead into
-// met[group parity][step][factor][lane]; every wave reads them there.
-#ifndef SWEEP_SHARE_METRICS
-#define SWEEP_SHARE_METRICS 1
-#endif
+// Three-field launches with interface velocities on the fly (SHM): blocks of the seven
+// species waves and an eighth, which loads the six metric factors of each step (hI, hA, hB
+// at interface k; h1, h2, h3 at cell k-1) three groups ahead and leaves in LDS what the
+// species waves make of them: the products, and the correctly rounded reciprocals of the
+// three divisors that vary along the line, so that their divisions are div_rcp.  The steps
+// were bound by instruction issue, not by memory (a lone block took as long per step,
+// 1.84 us, as a full GPU's worth): fourteen to eighteen IEEE divisions, the products formed
+// again by every wave.  The divisors that depend on the step alone (dx, dx + dx, dxi) have
+// their reciprocals in the grid (scalar loads).  An eighth wave rather than work for the
+// seven: they sit two to a SIMD on three of the CU's four, and it takes the free place.
+// met[group parity][step][row][lane], rows below.
+enum : int {
+  M_HI = 0, M_YI = 1,                    // h1i and its reciprocal
+  M_H2A = 2, M_HA = 3, M_YA = 4,         // area product, volume and its reciprocal, rank 0
+  M_H2B = 5, M_HB = 6, M_YB = 7,         // and rank 1
+  M_ROWS = 8
+};
 
 // The fused step's sweeps load each step's three fields and cell velocity by LDS DMA
 // (global_load_lds_dwordx4, which holds no registers while in flight) SWEEP_DMA steps
@@ -699,11 +703,8 @@ constexpr int sweep_xch_doubles() { return 2 * PF * (LSP - 1) * 2 * 64; }
 #endif
 template <int D>
 constexpr int sweep_ring_doubles() { return LSP * (D + 1) * 4 * 64; }
-// metric-factor slots: two groups in registers-then-LDS, or four DMA slots
-template <bool DMAV, int PF>
-constexpr int sweep_met_slots() { return DMAV && SWEEP_DMA > 0 ? 4 : 2; }
-template <int PF, bool DMAV = false>
-constexpr int sweep_met_doubles() { return sweep_met_slots<DMAV, PF>() * PF * 6 * 64; }
+template <int PF>
+constexpr int sweep_met_doubles() { return 2 * PF * M_ROWS * 64; }
 // vector memory operations issued after the loads of step k: two per step at least; from
 // the first step whose D - 1 predecessors all store (k > D), also the step's stores
 template <int D>
@@ -736,19 +737,23 @@ __device__ __forceinline__ void ring_read4(const double* p, double& a, double& b
       : "v"(ad)
       : "memory");
 }
-// six rows 1 KiB apart (the metric factors of one step in their DMA slot), likewise
-__device__ __forceinline__ void lds_read6(const double* p, double* v) {
+// a step's metric rows, 512 B apart, likewise: the first five at p, the last three at pb
+__device__ __forceinline__ void lds_read8(const double* p, const double* pb, double* v) {
   const unsigned ad = (unsigned)(unsigned long)(__attribute__((address_space(3))) const double*)p;
+  const unsigned bd = (unsigned)(unsigned long)(__attribute__((address_space(3))) const double*)pb;
   __asm__ volatile(
-      "ds_read_b64 %0, %6\n\t"
-      "ds_read_b64 %1, %6 offset:1024\n\t"
-      "ds_read_b64 %2, %6 offset:2048\n\t"
-      "ds_read_b64 %3, %6 offset:3072\n\t"
-      "ds_read_b64 %4, %6 offset:4096\n\t"
-      "ds_read_b64 %5, %6 offset:5120\n\t"
+      "ds_read_b64 %0, %8\n\t"
+      "ds_read_b64 %1, %8 offset:512\n\t"
+      "ds_read_b64 %2, %8 offset:1024\n\t"
+      "ds_read_b64 %3, %8 offset:1536\n\t"
+      "ds_read_b64 %4, %8 offset:2048\n\t"
+      "ds_read_b64 %5, %9\n\t"
+      "ds_read_b64 %6, %9 offset:512\n\t"
+      "ds_read_b64 %7, %9 offset:1024\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5])
-      : "v"(ad)
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]),
+        "=&v"(v[7])
+      : "v"(ad), "v"(bd)
       : "memory");
 }
 // a read-only grid array (dx, dxi) at a wave-uniform index, by a scalar load: a vector load
@@ -771,20 +776,96 @@ __device__ __forceinline__ bool sweep_block(int nbx, int nlines, int& bx, int& b
   return by < nlines;
 }
 
+// (launches of fewer fields, or with stored interface velocities, have no eighth wave)
+template <int NQ, bool OTF>
+constexpr bool sweep_shm() { return NQ == 3 && OTF; }
+template <int NQ, bool OTF>
+constexpr int sweep_threads() { return 64 * (sweep_shm<NQ, OTF>() ? LSP + 1 : LSP); }
+
+// LDS stores of one group are visible to the other waves after this barrier.  With DMA, the
+// fences would also wait for the ring's loads: this wave's LDS accesses are complete
+// (lgkmcnt) before the barrier, and nothing moves across it.
+template <bool DMA>
+__device__ __forceinline__ void sweep_barrier() {
+  if (DMA) {
+    __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+}
+
+// The eighth wave of an SHM block: the metric rows of group G + 1 (steps 2 + (G+1) PF ..) are
+// formed while the species waves run group G, from factors loaded three groups before.
+template <int DIR, int PF, bool POST, bool DMA>
+__device__ __forceinline__ void sweep23_metrics(const DevGrid& g, int bx, int by, double* met) {
+  const int lane = threadIdx.x, lx = DIR == 2 ? g.lx2 : g.lx3, other = by + 1;
+  const int i1 = min(bx * 64 + lane, g.lx1 - 1) + 1;
+  const long cs_ = DIR == 2 ? (long)g.L1 : (long)g.L1 * g.L2;
+  const long c0 = DIR == 2 ? gix(g, i1, 0, other) : gix(g, i1, other, 0);
+  const long istr = DIR == 2 ? (long)g.lx1 : (long)g.lx1 * g.lx2;
+  const long if0 = DIR == 2 ? (long)(i1 - 1) + (long)g.lx1 * ((long)(g.lx2 + 1) * (other - 1)) - istr
+                            : (long)(i1 - 1) + (long)g.lx1 * (other - 1) - istr;
+  const double* hA = DIR == 2 ? g.h1x2i : g.h1x3i;
+  const double* hB = DIR == 2 ? g.h3x2i : g.h2x3i;
+  const double* hI = DIR == 2 ? g.h2x2i : g.h3x3i;
+  struct Raw { double i, a, b, h1, h2, h3; };
+  auto load = [&](int G, Raw* r) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      const int k = 2 + G * PF + u;
+      const long ik = if0 + (long)clampi(k, 1, lx + 1) * istr;
+      const long cm = c0 + (long)clampi(k - 1, 1, lx) * cs_;
+      r[u] = Raw{hI[ik], hA[ik], hB[ik], g.h1[cm], g.h2[cm], g.h3[cm]};
+    }
+  };
+  auto form = [&](int G, const Raw* r) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      double* m = met + ((G & 1) * PF + u) * M_ROWS * 64 + lane;
+      const double ha = (r[u].h1 * r[u].h2) * r[u].h3, hb = ((r[u].h1 * r[u].h1) * r[u].h2) * r[u].h3;
+      m[M_HI * 64] = r[u].i;
+      m[M_YI * 64] = 1.0 / r[u].i;
+      m[M_H2A * 64] = r[u].a * r[u].b;
+      m[M_H2B * 64] = (r[u].a * r[u].a) * r[u].b;
+      m[M_HA * 64] = ha;
+      m[M_YA * 64] = 1.0 / ha;
+      m[M_HB * 64] = hb;
+      m[M_YB * 64] = 1.0 / hb;
+    }
+  };
+  Raw r0[PF], r1[PF], r2[PF];
+  load(0, r0);
+  load(1, r1);
+  load(2, r2);
+  form(0, r0);
+  sweep_barrier<DMA>();
+  const int groups = lx / PF;
+  for (int G = 0; G < groups; ++G) {
+    form(G + 1, r1);
+#pragma unroll
+    for (int u = 0; u < PF; ++u) { r1[u] = r2[u]; }
+    load(G + 3, r2);
+    sweep_barrier<DMA>();
+  }
+  if (POST) sweep_barrier<DMA>();
+}
+
 template <int DIR, int PF, int NQ, bool OTF, bool CONV = false, bool POST = false,
           bool DMAV = false>
 __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s,
                                              const SweepFields& F, int isp0, double dt, int bx,
                                              int by, double* xch, double* met, double* ring) {
   static_assert(!(CONV || POST) || NQ == 3, "the conversions come with all three fields");
-  constexpr bool SHM = SWEEP_SHARE_METRICS && (CONV || POST);
-  static_assert(!DMAV || (OTF && NQ == 3 && (CONV || POST)), "DMA: the fused sweeps only");
+  constexpr bool SHM = sweep_shm<NQ, OTF>();
+  static_assert(!DMAV || (SHM && (CONV || POST)), "DMA: the fused sweeps only");
   constexpr bool DMA = DMAV && SWEEP_DMA > 0;
   constexpr int D = DMA ? SWEEP_DMA : 1;
-  constexpr bool MDMA = DMA && SHM;           // metric factors by DMA as well
-  constexpr int MS = sweep_met_slots<DMAV, PF>();
-  static_assert(!MDMA || PF == 2, "one DMA instruction loads a factor's two steps");
-  static_assert(!MDMA || 3 * PF >= D, "the factors are loaded at least as far ahead as the rows");
+  if (SHM && threadIdx.y == blockDim.y - 1) {
+    sweep23_metrics<DIR, PF, POST, DMA>(g, bx, by, met);
+    return;
+  }
   const int lx = DIR == 2 ? g.lx2 : g.lx3;
   // lanes past lx1 redo column lx1's work: same inputs, same values written to the same cells
   const int i1 = min((int)(bx * 64 + threadIdx.x), g.lx1 - 1) + 1;
@@ -800,6 +881,10 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
   const double* hI = DIR == 2 ? g.h2x2i : g.h3x3i;   // h1i of advec1D_MC_curv
   const double* dx = DIR == 2 ? g.dx2 : g.dx3;
   const double* dxi = DIR == 2 ? g.dx2i : g.dx3i;
+  // reciprocals of dx(i), dx(i) + dx(i+1), dxi(i)
+  const double* rdx = DIR == 2 ? g.rdx2 : g.rdx3;
+  const double* rdxs = DIR == 2 ? g.rdx2s : g.rdx3s;
+  const double* rdxi = DIR == 2 ? g.rdx2i : g.rdx3i;
   const long so = (long)(isp - 1) * g.N;
   const double* w = (DIR == 2 ? s.vs2 : s.vs3) + so + c0;
   const double* vi = (DIR == 2 ? s.vs2i : s.vs3i) +
@@ -815,7 +900,7 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
     fr1[q] = !e7 && F.frank[q] == 1;
     lp[q] = fp[q];
   }
-  const double msp = ms(isp), gm1 = gammas(isp) - 1.0;
+  const double msp = ms(isp), gm1 = gammas(isp) - 1.0, rgm1 = CONV ? 1.0 / gm1 : 0.0;
   if (CONV) {
     if (e7) {                                  // density and momentum: converted, not advected
       fp[0] = s.ns + so + c0;
@@ -830,7 +915,7 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
     if (CONV) {
       const double n = v[0];
       v[1] = (n * msp) * v[1];
-      v[2] = ((n * kB) * v[2]) / gm1;
+      v[2] = div_rcp((n * kB) * v[2], gm1, rgm1);
     }
   };
   // pipeline registers of the steps in flight
@@ -869,64 +954,6 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
     dma16(a + dc + (long)kf * cs_, sl);
     dma16(b + dc + (long)kf * cs_, sl + 128);
   };
-  // SHM: this wave's metric factor (wave wy < 6 loads factor wy) at step k, and a group's
-  // PF steps into registers or from registers into LDS
-  const int wy = threadIdx.y;
-  auto met_at = [&](int k) -> double {
-    const int ki = clampi(k, 1, lx + 1);
-    const long ik = if0 + (long)ki * istr;
-    const long cm = c0 + (long)clampi(k - 1, 1, lx) * cs_;
-    if (wy == 0) return hI[ik];
-    if (wy == 1) return hA[ik];
-    if (wy == 2) return hB[ik];
-    if (wy == 3) return g.h1[cm];
-    if (wy == 4) return g.h2[cm];
-    return g.h3[cm];
-  };
-  auto met_load = [&](int G, double* r) {            // group G: steps 2 + G PF ..
-#pragma unroll
-    for (int u = 0; u < PF; ++u) r[u] = wy < 6 ? met_at(2 + G * PF + u) : 0.0;
-  };
-  auto met_store = [&](int G, const double* r) {
-    if (wy < 6) {
-#pragma unroll
-      for (int u = 0; u < PF; ++u) met[(((G & 1) * PF + u) * 6 + wy) * 64 + threadIdx.x] = r[u];
-    }
-  };
-  auto met_get = [&](int G, int u, int m) -> double {
-    return met[(((G & 1) * PF + u) * 6 + m) * 64 + threadIdx.x];
-  };
-  // MDMA: the factors by DMA into a ring of MS group slots [slot][factor][step][64], three
-  // groups ahead; wave wy < 6 loads factor wy of a group's two steps with one instruction
-  // (lanes 0-31 the first step's row, lanes 32-63 the second's)
-  auto met_ptr = [&](int k) -> const double* {
-    const int ki = clampi(k, 1, lx + 1);
-    const long ik = if0 + (long)ki * istr;
-    const long cm = c0 + (long)clampi(k - 1, 1, lx) * cs_;
-    if (wy == 0) return hI + ik;
-    if (wy == 1) return hA + ik;
-    if (wy == 2) return hB + ik;
-    if (wy == 3) return g.h1 + cm;
-    if (wy == 4) return g.h2 + cm;
-    return g.h3 + cm;
-  };
-  auto met_dma = [&](int G) {
-    if (wy < 6) dma16(met_ptr(2 + G * PF + (hi ? 1 : 0)) + dc, met + ((G % MS) * 6 + wy) * PF * 64);
-  };
-  // before the barrier that ends group G, this wave's load of group G+1's factors has
-  // landed: it was followed by the loads and stores of the steps of groups G-2 .. G (or,
-  // for G < 2, by the ring's prologue loads and steps 0 and 1)
-  auto met_wait = [&](int G) {
-    if (wy >= 6) return;
-    if (G < 2) wait_vmcnt<2 * D + 4>();
-    else if (POST && !e7) wait_vmcnt<3 * PF * (2 + NQ + 2)>();
-    else wait_vmcnt<3 * PF * (2 + NQ)>();
-  };
-  if (MDMA) {
-    met_dma(0);
-    met_dma(1);
-    met_dma(2);
-  }
   double fa[NQ], fb[NQ], fc[NQ], rsp[NQ], slp[NQ], php[NQ];
   double dxcur = dx[0];
   double wprev = w[0];         // vs(0) for the on-the-fly interface velocity
@@ -992,51 +1019,68 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
 #pragma unroll
       for (int q = 0; q < NQ; ++q) nxt[q] = pf[q][u];
     }
-    double hIv, a, b, h1, h2, h3;
-    if (!SHM) {
-      hIv = pI[u]; a = pA[u]; b = pB[u]; h1 = p1[u]; h2 = p2[u]; h3 = p3[u];
-    } else if (mode == 2 && MDMA) {
-      double m6[6];
-      lds_read6(met + ((G % MS) * 6 * PF + slot) * 64 + rel, m6);
-      hIv = m6[0]; a = m6[1]; b = m6[2]; h1 = m6[3]; h2 = m6[4]; h3 = m6[5];
-    } else if (mode == 2) {
-      hIv = met_get(G, slot, 0); a = met_get(G, slot, 1); b = met_get(G, slot, 2);
-      h1 = met_get(G, slot, 3); h2 = met_get(G, slot, 4); h3 = met_get(G, slot, 5);
-    } else {                                   // step 1 (step 0 uses none)
-      const long ik = if0 + (long)clampi(k, 1, lx + 1) * istr;
-      hIv = hI[ik]; a = hA[ik]; b = hB[ik];
-      h1 = h2 = h3 = 1.0;
+    // h1i of the interface, the two ranks' area products there and volumes of the cell, and
+    // (SHM) the reciprocals of the divisors
+    double hIv, h2f0, h2f1, ha1f0 = 1.0, ha1f1 = 1.0, yI = 0.0, y0 = 0.0, y1 = 0.0;
+    if (SHM && mode == 2) {
+      // (the electron wave's middle slot is not of rank 1: it reads the rank-0 rows twice)
+      double m8[M_ROWS];
+      const double* m = met + ((G & 1) * PF + slot) * M_ROWS * 64 + threadIdx.x;
+      const double* mb = m + (e7 ? M_H2A : M_H2B) * 64;
+      if (DMA) {
+        lds_read8(m, mb, m8);
+      } else {
+#pragma unroll
+        for (int r = 0; r < M_H2B; ++r) m8[r] = m[r * 64];
+#pragma unroll
+        for (int r = M_H2B; r < M_ROWS; ++r) m8[r] = mb[(r - M_H2B) * 64];
+      }
+      hIv = m8[M_HI]; yI = m8[M_YI]; h2f0 = m8[M_H2A]; h2f1 = m8[M_H2B];
+      ha1f0 = m8[M_HA]; y0 = m8[M_YA]; ha1f1 = m8[M_HB]; y1 = m8[M_YB];
+    } else {
+      double a, b;
+      if (SHM) {                               // step 1 (step 0 uses none)
+        const long ik = if0 + (long)clampi(k, 1, lx + 1) * istr;
+        hIv = hI[ik]; a = hA[ik]; b = hB[ik];
+      } else {
+        hIv = pI[u]; a = pA[u]; b = pB[u];
+        ha1f0 = (p1[u] * p2[u]) * p3[u];
+        ha1f1 = ((p1[u] * p1[u]) * p2[u]) * p3[u];
+      }
+      h2f0 = a * b;
+      h2f1 = SHM && e7 ? h2f0 : (a * a) * b;
     }
     if (!DMA) issue(k + PF, u);                // (after this step's slot u was read)
     if (CONV && min(k + 2, lx + 2) <= lx) convert(nxt);
-    double v = 0.0, vq = 0.0, h2f0 = 0.0, h2f1 = 0.0, ha1f0 = 1.0, ha1f1 = 1.0, dxim = 1.0;
+    double v = 0.0, vq = 0.0, dxim = 1.0, ydxim = 1.0;
     double newv[NQ];
     if (mode >= 1) {
       if (OTF) { v = 0.5 * (wprev + wv); wprev = wv; }
       else v = wv;
-      vq = v / hIv;
-      h2f0 = a * b;
-      h2f1 = (a * a) * b;
+      vq = SHM && mode == 2 ? div_rcp(v, hIv, yI) : v / hIv;
     }
     if (mode == 2) {
-      ha1f0 = (h1 * h2) * h3;
-      ha1f1 = ((h1 * h1) * h2) * h3;
       dxim = ld_uniform(dxi + k - 2);
+      ydxim = ld_uniform(rdxi + k - 1);
     }
+    const double dxs = dxk + dxk1, ydx = ld_uniform(rdx + k + 1), ydxs = ld_uniform(rdxs + k);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      const double rs = (fc[q] - fb[q]) / dxk1;
-      const double csl = (fc[q] - fa[q]) / (dxk + dxk1);
+      const double rs = div_rcp(fc[q] - fb[q], dxk1, ydx);
+      const double csl = div_rcp(fc[q] - fa[q], dxs, ydxs);
       const double sl = minmod(csl, minmod(2.0 * rsp[q], 2.0 * rs));
       if (mode >= 1) {
         const double phn = fb[q] * v - ((0.5 * v) * (dxk + vq * dt)) * sl;
         const double phv = fa[q] * v + ((0.5 * v) * (dxk - vq * dt)) * slp[q];
         const double ph = v < 0.0 ? phn : phv;
         if (mode == 2) {
-          const double h2k = fr1[q] ? h2f1 : h2f0;
-          const double h2m = fr1[q] ? h2p1 : h2p0;
-          const double ha1 = fr1[q] ? ha1f1 : ha1f0;
-          const double out = fa[q] - ((dt * (h2k * ph - h2m * php[q])) / dxim) / ha1;
+          // (SHM: slot 1's values carry its rank)
+          const bool r1 = SHM ? q == 1 : fr1[q];
+          const double h2k = r1 ? h2f1 : h2f0;
+          const double h2m = r1 ? h2p1 : h2p0;
+          const double ha1 = r1 ? ha1f1 : ha1f0;
+          const double dfl = div_rcp(dt * (h2k * ph - h2m * php[q]), dxim, ydxim);
+          const double out = fa[q] - (SHM ? div_rcp(dfl, ha1, r1 ? y1 : y0) : dfl / ha1);
           // CONV: the electron wave's density and momentum go back unchanged
           fp[q][(long)(k - 1) * cs_] = (CONV && q < 2 && e7) ? fa[q] : out;
           if (POST) newv[q] = out;
@@ -1065,56 +1109,24 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
     }
     if (DMA) dma_issue(k + D);                // into the slot step k - 1 read
   };
-  // POST: LDS stores of one group are visible to the electron wave after this barrier; no
-  // fence on global memory, so loads issued ahead stay in flight
-  auto lds_barrier = [&]() {
-    if (DMA) {
-      // the fences would also wait for the ring's loads: this wave's LDS accesses are
-      // complete (lgkmcnt) before the barrier, and nothing moves across it
-      __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    } else {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    }
-  };
-  double rmA[PF], rmB[PF];                    // SHM: factors of two groups ahead
-  if (MDMA) {
-    // (the ring's prologue loads are issued after these: see met_wait)
-  } else if (SHM) {
-    met_load(0, rmA);
-    met_store(0, rmA);
-    met_load(1, rmB);
-    lds_barrier();
-  }
   step(0, 0, 0);
   step(1, 1 % PF, 1);
-  if (MDMA) {                                 // group 0's factors published
-    wait_vmcnt<2 * D + 4>();
-    lds_barrier();
-  }
+  if (SHM) sweep_barrier<DMA>();              // group 0's metric rows published
   int kb = 2;
   int groups = 0;
-  // group G (steps kb..kb+PF-1): SHM loads the factors of group G+2 into rl and stores
-  // those of group G+1 from rw before the barrier (MDMA: loads those of group G+3 into
-  // their slot and waits for its load of group G+1's before the barrier)
-  auto group = [&](double* rl, double* rw) {
-    if (MDMA) met_dma(groups + 3);
-    else if (SHM) met_load(groups + 2, rl);
+  while (kb + PF - 1 <= lx + 1) {              // group `groups`: steps kb..kb+PF-1
 #pragma unroll
     for (int u = 0; u < PF; ++u) step(kb + u, (2 + u) % PF, 2, u, groups);
-    if (MDMA) met_wait(groups);
-    else if (SHM) met_store(groups + 1, rw);
     if (POST) {
       // the electron wave finishes the previous group (its LDS parity is not written in
       // this group), then the ion waves may write that parity again after the barrier
       if (e7 && groups > 0) finalize(xbuf ^ 1, kb - PF, PF, eprev);
 #pragma unroll
       for (int u = 0; u < PF; ++u) eprev[u] = eout[u];
-      lds_barrier();
+      sweep_barrier<DMA>();
       xbuf ^= 1;
     } else if (SHM) {
-      lds_barrier();
+      sweep_barrier<DMA>();
     } else {
       // keep the species waves of the block in step so the metric factors they all read
       // are still cached when the slower waves reach them (no memory fence: nothing is
@@ -1123,11 +1135,6 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
     }
     ++groups;
     kb += PF;
-  };
-  while (kb + PF - 1 <= lx + 1) {              // two groups a turn: rmA and rmB alternate
-    group(rmA, rmB);
-    if (kb + PF - 1 > lx + 1) break;
-    group(rmB, rmA);
   }
   int tail = 0;
 #pragma unroll
@@ -1138,7 +1145,7 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
   }
   if (POST) {
     if (e7 && groups > 0) finalize(xbuf ^ 1, kb - PF, PF, eprev);
-    lds_barrier();
+    sweep_barrier<DMA>();
     if (e7 && tail > 0) finalize(xbuf, kb, tail, eout);
   }
   if (DMA) wait_vmcnt<0>();                   // no load still writing the ring on exit
@@ -1147,13 +1154,19 @@ __device__ __forceinline__ void sweep23_body(const DevGrid& g, const DevState& s
 // (a 1-D grid of sweep_blocks(nbx, lines) blocks, see sweep_block)
 template <int DIR, int PF, int NQ, bool OTF, bool CONV = false, bool POST = false,
           bool DMAV = false>
-__global__ __launch_bounds__(448) SWEEP23_WAVES void k_sweep23(DevGrid g, DevState s,
+__global__ __launch_bounds__((sweep_threads<NQ, OTF>())) SWEEP23_WAVES void k_sweep23(DevGrid g, DevState s,
                                                                SweepFields F, int isp0, double dt) {
   __shared__ double xch[POST ? sweep_xch_doubles<PF>() : 1];
-  __shared__ double met[(CONV || POST) ? sweep_met_doubles<PF, DMAV>() : 1];
+  __shared__ double met[sweep_shm<NQ, OTF>() ? sweep_met_doubles<PF>() : 1];
   __shared__ double ring[DMAV && SWEEP_DMA > 0 ? sweep_ring_doubles<SWEEP_DMA>() : 1];
   int bx, by;
   if (!sweep_block((g.lx1 + 63) / 64, DIR == 2 ? g.lx3 : g.lx2, bx, by)) return;
+  if (sweep_shm<NQ, OTF>() && !POST) {
+    // a block of a launch with fewer than seven species waves (sweep_species): the last
+    // block row's waves past the seventh species leave (a barrier does not count them)
+    isp0 += blockIdx.y * (blockDim.y - 1);
+    if (threadIdx.y < blockDim.y - 1 && isp0 + (int)threadIdx.y > LSP) return;
+  }
   sweep23_body<DIR, PF, NQ, OTF, CONV, POST, DMAV>(g, s, F, isp0, dt, bx, by, xch, met, ring);
 }
 
@@ -1216,9 +1229,9 @@ __global__ __launch_bounds__(TPB) void kb_threads(const BatchMember* M, const lo
 }
 
 // the x2/x3 sweeps of all fields (x3 with the conversions folded in, x2 with rhov12v1 and
-// rhoe2T); blocks of 64 x 7
+// rhoe2T); blocks of 64 x 8
 template <int DIR, int PF>
-__global__ __launch_bounds__(448) void kb_sweep23(const BatchMember* M, const long* pre, int n,
+__global__ __launch_bounds__(512) void kb_sweep23(const BatchMember* M, const long* pre, int n,
                                                   long total) {
   __shared__ double xch[sweep_xch_doubles<PF>()];
   __shared__ double met[sweep_met_doubles<PF>()];
@@ -1287,7 +1300,7 @@ long batch_units(const DevGrid& g, int kernel) {
 // ghost fill (with v12rhov1, T2rhoe), x1 boundary interface velocities, x3 sweep
 // (converting), x1 sweep, x2 sweep (with rhov12v1, rhoe2T), the surface conversions.
 void launch_batch_advection(const BatchTable& t, int sweep_pf, hipStream_t st) {
-  const dim3 thr(TPB), s7(64, LSP);
+  const dim3 thr(TPB), s7(64, LSP), s8(64, LSP + 1);
   auto tb = [&](long total) { return (unsigned)std::max(1L, std::min<long>(total, t.blocks_sweep)); };
   auto th = [&](long total) {
     return (unsigned)std::max(1L, std::min<long>((total + TPB - 1) / TPB, t.blocks_thread));
@@ -1301,18 +1314,18 @@ void launch_batch_advection(const BatchTable& t, int sweep_pf, hipStream_t st) {
   hipLaunchKernelGGL(kb_threads<BK_V1B>, dim3(th(t.total[BK_V1B])), thr, 0, st, t.m, t.pre, t.n,
                      t.total[BK_V1B]);
   if (sweep_pf == 1)
-    hipLaunchKernelGGL((kb_sweep23<3, 1>), dim3(tb(t.total[BK_SW3])), s7, 0, st, t.m, t.pre, t.n,
+    hipLaunchKernelGGL((kb_sweep23<3, 1>), dim3(tb(t.total[BK_SW3])), s8, 0, st, t.m, t.pre, t.n,
                        t.total[BK_SW3]);
   else
-    hipLaunchKernelGGL((kb_sweep23<3, 2>), dim3(tb(t.total[BK_SW3])), s7, 0, st, t.m, t.pre, t.n,
+    hipLaunchKernelGGL((kb_sweep23<3, 2>), dim3(tb(t.total[BK_SW3])), s8, 0, st, t.m, t.pre, t.n,
                        t.total[BK_SW3]);
   hipLaunchKernelGGL(kb_sweep1, dim3(tb(t.total[BK_SW1])), s7, 0, st, t.m, t.pre, t.n,
                      t.total[BK_SW1]);
   if (sweep_pf == 1)
-    hipLaunchKernelGGL((kb_sweep23<2, 1>), dim3(tb(t.total[BK_SW2])), s7, 0, st, t.m, t.pre, t.n,
+    hipLaunchKernelGGL((kb_sweep23<2, 1>), dim3(tb(t.total[BK_SW2])), s8, 0, st, t.m, t.pre, t.n,
                        t.total[BK_SW2]);
   else
-    hipLaunchKernelGGL((kb_sweep23<2, 2>), dim3(tb(t.total[BK_SW2])), s7, 0, st, t.m, t.pre, t.n,
+    hipLaunchKernelGGL((kb_sweep23<2, 2>), dim3(tb(t.total[BK_SW2])), s8, 0, st, t.m, t.pre, t.n,
                        t.total[BK_SW2]);
   hipLaunchKernelGGL(kb_threads<BK_POST>, dim3(th(t.total[BK_POST])), thr, 0, st, t.m, t.pre, t.n,
                      t.total[BK_POST]);
@@ -1415,6 +1428,21 @@ void launch_save_v1_boundaries(const DevGrid& g, const DevState& s, hipStream_t 
 // The DMA ring loads 16-byte pairs of cells: every pair must be 16-byte aligned, so rows of
 // an even length (lx1 + 4) and fields at 16-byte aligned addresses; otherwise the sweeps
 // prefetch through registers.
+// Species waves of a block of the x2/x3 sweeps (SHM), seven unless the grid leaves CUs idle:
+// a march is a serial chain, and two species waves on a SIMD take each step in turns.  So
+// while the (x1 block, line) pairs times the groups fit the 256 CUs, the species go to
+// blocks of their own, in fours up to 128 pairs, in twos up to 64.  Such launches load four
+// steps ahead (their registers are free, and the latency of two did not cover a step).
+// Measured, seven in a block -> this rule: x2 of 128x64x1 (2 pairs) 86 -> 39 us, x3 and x2 of
+// 96x24x20 (48, 40) 29 -> 20 and 40 -> 20, of 98x40x36 (80, 72) 45 -> 30 and 42 -> 30; at
+// 192x64x48 (192, 144) fours take 78 and 86 against 69 and 78.
+constexpr int SWEEP_CUS = 256;
+constexpr int SWEEP_PFS = 4;
+static int sweep_species(const DevGrid& g, int dir) {
+  const long pairs = (long)((g.lx1 + 63) / 64) * (dir == 2 ? g.lx3 : g.lx2);
+  return pairs * 4 <= SWEEP_CUS ? 2 : pairs * 2 <= SWEEP_CUS ? 4 : LSP;
+}
+
 static bool sweep_dma_ok(const DevGrid& g, std::initializer_list<const double*> fields) {
   if (SWEEP_DMA <= 0 || g.L1 % 2 != 0) return false;
   for (const double* f : fields)
@@ -1423,12 +1451,15 @@ static bool sweep_dma_ok(const DevGrid& g, std::initializer_list<const double*> 
 }
 
 namespace {
+bool sweep_shm_of(int nq, bool otf) { return nq == 3 && otf; }
+
 template <int NQ, int PFM = SWEEP_PF>
 void sweep_launch(const DevGrid& g, const DevState& s, int dir, const SweepFields& F, int isp0,
-                  int nsp, double dt, bool otf, hipStream_t st) {
-  const dim3 blk(64, nsp);
-  const dim3 grd = dir == 1 ? dim3(g.lx2, g.lx3)
-                            : dim3(sweep_blocks((g.lx1 + 63) / 64, dir == 2 ? g.lx3 : g.lx2));
+                  int nsp, double dt, bool otf, hipStream_t st, int nsb_shm = LSP) {
+  const int nbx = (g.lx1 + 63) / 64, nl = dir == 2 ? g.lx3 : g.lx2;
+  const int nsb = dir != 1 && sweep_shm_of(NQ, otf) ? nsb_shm : nsp;
+  const dim3 blk(64, nsb + (dir != 1 && sweep_shm_of(NQ, otf) ? 1 : 0));
+  const dim3 grd = dir == 1 ? dim3(g.lx2, g.lx3) : dim3(sweep_blocks(nbx, nl), (nsp + nsb - 1) / nsb);
   if (dir == 1) {
     if (otf) hipLaunchKernelGGL((k_sweep1<NQ, true>), grd, blk, 0, st, g, s, F, isp0, dt);
     else hipLaunchKernelGGL((k_sweep1<NQ, false>), grd, blk, 0, st, g, s, F, isp0, dt);
@@ -1458,7 +1489,7 @@ void launch_sweep(const DevGrid& g, const DevState& s, int dir, int fields, doub
   timing_begin(name, st);
   if (na == 1 && fields == F_ENERGY) {       // energy alone: all seven species in one launch
     sweep_launch<1>(g, s, dir, A, 1, LSP, dt, onthefly, st);
-  } else if (na == 3 && dir == 1 && SWEEP1_E7_IN_BLOCK) {
+  } else if (na == 3 && dir == 1) {
     // x1, all fields: the electron wave joins the block and sweeps its energy only
     A.elec_energy = 1;
     if (onthefly && SWEEP1_RCP && sweep1_lm_bytes(g.lx1, 2) <= SWEEP1_LM_MAX) {
@@ -1470,15 +1501,16 @@ void launch_sweep(const DevGrid& g, const DevState& s, int dir, int fields, doub
     } else {
       sweep_launch<3>(g, s, dir, A, 1, LSP, dt, onthefly, st);
     }
-  } else if (na == 3 && dir != 1 && SWEEP_E7_IN_BLOCK) {
+  } else if (na == 3) {
     // x2/x3, all fields: the electron wave joins the block and does energy only
     A.elec_energy = 1;
-    if (tune.sweep_pf == 1) sweep_launch<3, 1>(g, s, dir, A, 1, LSP, dt, onthefly, st);
+    const int nsb = onthefly ? sweep_species(g, dir) : LSP;
+    if (nsb < LSP) sweep_launch<3, SWEEP_PFS>(g, s, dir, A, 1, LSP, dt, onthefly, st, nsb);
+    else if (tune.sweep_pf == 1) sweep_launch<3, 1>(g, s, dir, A, 1, LSP, dt, onthefly, st);
     else sweep_launch<3, 2>(g, s, dir, A, 1, LSP, dt, onthefly, st);
   } else {                                   // fewer fields: ions, then the electrons
     if (na == 1) sweep_launch<1>(g, s, dir, A, 1, LSP - 1, dt, onthefly, st);
-    else if (na == 2) sweep_launch<2>(g, s, dir, A, 1, LSP - 1, dt, onthefly, st);
-    else sweep_launch<3>(g, s, dir, A, 1, LSP - 1, dt, onthefly, st);
+    else sweep_launch<2>(g, s, dir, A, 1, LSP - 1, dt, onthefly, st);
     if (fields & F_ENERGY) {                 // electrons: energy only
       SweepFields E{};
       E.f[0] = s.rhoes;
@@ -1498,11 +1530,13 @@ void launch_sweep3_preconvert(const DevGrid& g, const DevState& s, double dt, hi
   A.f[1] = s.rhovs1; A.frank[1] = 1;
   A.f[2] = s.rhoes; A.frank[2] = 0;
   A.elec_energy = 1;
-  const dim3 blk(64, LSP), grd(sweep_blocks((g.lx1 + 63) / 64, g.lx2));
-  const bool dma = sweep_dma_ok(g, {s.ns, s.rhovs1, s.rhoes, s.vs1, s.Ts, s.vs3, g.h1, g.h2,
-                                    g.h3, g.h1x3i, g.h2x3i, g.h3x3i});
+  const int nbx = (g.lx1 + 63) / 64, nsb = sweep_species(g, 3);
+  const dim3 blk(64, nsb + 1), grd(sweep_blocks(nbx, g.lx2), (LSP + nsb - 1) / nsb);
+  const bool dma = nsb == LSP && sweep_dma_ok(g, {s.ns, s.rhovs1, s.rhoes, s.vs1, s.Ts, s.vs3});
   timing_begin("sweep3", st);
-  if (tune.sweep_pf == 1) {
+  if (nsb < LSP) {
+    hipLaunchKernelGGL((k_sweep23<3, SWEEP_PFS, 3, true, true>), grd, blk, 0, st, g, s, A, 1, dt);
+  } else if (tune.sweep_pf == 1) {
     hipLaunchKernelGGL((k_sweep23<3, 1, 3, true, true>), grd, blk, 0, st, g, s, A, 1, dt);
   } else {
     if (dma) hipLaunchKernelGGL((k_sweep23<3, 2, 3, true, true, false, true>), grd, blk, 0, st, g, s, A, 1, dt);
@@ -1520,9 +1554,8 @@ void launch_sweep2_postconvert(const DevGrid& g, const DevState& s, double dt, h
   A.f[1] = s.rhovs1; A.frank[1] = 1;
   A.f[2] = s.rhoes; A.frank[2] = 0;
   A.elec_energy = 1;
-  const dim3 blk(64, LSP), grd(sweep_blocks((g.lx1 + 63) / 64, g.lx3));
-  const bool dma = sweep_dma_ok(g, {s.ns, s.rhovs1, s.rhoes, s.vs1, s.Ts, s.vs2, g.h1, g.h2,
-                                    g.h3, g.h1x2i, g.h2x2i, g.h3x2i});
+  const dim3 blk(64, LSP + 1), grd(sweep_blocks((g.lx1 + 63) / 64, g.lx3));
+  const bool dma = sweep_dma_ok(g, {s.ns, s.rhovs1, s.rhoes, s.vs1, s.Ts, s.vs2});
   timing_begin("sweep2", st);
   if (tune.sweep_pf == 1) {
     hipLaunchKernelGGL((k_sweep23<2, 1, 3, true, false, true>), grd, blk, 0, st, g, s, A, 1, dt);
@@ -1538,6 +1571,9 @@ void launch_sweep2_postconvert(const DevGrid& g, const DevState& s, double dt, h
 }
 
 bool postconvert_fusable(const DevGrid& g) { return g.lx2 > 1; }
+// a small grid's x2 sweep is faster without the conversions, which need its seven species
+// in one block (see sweep_species)
+bool postconvert_pays(const DevGrid& g) { return sweep_species(g, 2) == LSP; }
 
 void launch_floor_ghosts(const DevGrid& g, double* Ts, hipStream_t st) {
   hipLaunchKernelGGL(k_floor_ghosts, dim3(blocks_for(surface_cells(g)), LSP), dim3(TPB), 0, st, g,

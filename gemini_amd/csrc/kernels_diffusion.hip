@@ -675,14 +675,13 @@ __global__ void k_fill_hcol(DevGrid g, double* hcol) {
     hcol[2 * g.hstride + t] = g.h3[cb + r];
   }
 }
-// the correctly rounded reciprocals of the row divisors (DevGrid::rdx1, rdx1i, rdx1s, each
-// indexed as its divisor, 0..lx1+2)
-__global__ void k_fill_rdx(DevGrid g, double* r) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, L = g.lx1 + 3;
+// the correctly rounded reciprocals of one axis' divisors (DevGrid::rdx1, rdx1i, rdx1s)
+__global__ void k_fill_rdx(const double* dx, const double* dxi, int lx, double* r) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, L = lx + 3;
   if (i >= L) return;
-  r[i] = 1.0 / g.dx1[i];
-  r[L + i] = 1.0 / g.dx1i[clampi(i - 1, 0, g.lx1 - 1)];
-  r[2 * L + i] = 1.0 / (g.dx1[min(i + 1, g.lx1 + 2)] + g.dx1[i]);
+  r[i] = 1.0 / dx[i];
+  r[L + i] = 1.0 / dxi[clampi(i - 1, 0, lx - 1)];
+  r[2 * L + i] = 1.0 / (dx[min(i + 1, lx + 2)] + dx[i]);
 }
 
 long pivot_record_ints(const DevGrid& g) { return (long)g.lx2 * g.lx3 * 2 * ((g.lx1 + 31) / 32); }
@@ -690,11 +689,24 @@ long pivot_record_ints(const DevGrid& g) { return (long)g.lx2 * g.lx3 * 2 * ((g.
 long diffusion_hcol_doubles(const DevGrid& g) {
   return 3 * (((long)g.lx2 * g.lx3 + 63) / 64) * g.lx1 * 64;
 }
-long diffusion_rdx_doubles(const DevGrid& g) { return 3L * (g.lx1 + 3); }
+long rdx_doubles(const DevGrid& g) { return 3L * (g.lx1 + g.lx2 + g.lx3 + 9); }
 
-void launch_fill_hcol(const DevGrid& g, double* hcol, double* rdx, hipStream_t st) {
+void launch_fill_hcol(const DevGrid& g, double* hcol, hipStream_t st) {
   hipLaunchKernelGGL(k_fill_hcol, dim3(4096), dim3(256), 0, st, g, hcol);
-  hipLaunchKernelGGL(k_fill_rdx, dim3((g.lx1 + 3 + 255) / 256), dim3(256), 0, st, g, rdx);
+}
+
+void launch_fill_rdx(DevGrid& g, double* rdx, hipStream_t st) {
+  const double* dx[] = {g.dx1, g.dx2, g.dx3};
+  const double* dxi[] = {g.dx1i, g.dx2i, g.dx3i};
+  const double** out[] = {&g.rdx1, &g.rdx1i, &g.rdx1s, &g.rdx2, &g.rdx2i, &g.rdx2s, &g.rdx3, &g.rdx3i,
+                          &g.rdx3s};
+  const int lx[] = {g.lx1, g.lx2, g.lx3};
+  for (int a = 0; a < 3; ++a) {
+    const int L = lx[a] + 3;
+    hipLaunchKernelGGL(k_fill_rdx, dim3((L + 255) / 256), dim3(256), 0, st, dx[a], dxi[a], lx[a], rdx);
+    for (int k = 0; k < 3; ++k) *out[3 * a + k] = rdx + k * L;
+    rdx += 3 * L;
+  }
 }
 
 // the kept rows and elimination states of every unit
