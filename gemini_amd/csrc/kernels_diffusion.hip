@@ -132,7 +132,7 @@ struct Pivot {
 // row as it is, a zero entry of the pivot row its column (dger skips it).  Written without
 // branches: a step under a branch could not overlap the next row's independent work.
 __device__ __forceinline__ Pivot elim_step(Elim& e, double a, double b, double cc, double d,
-                                           bool& swap) {
+                                           bool& swap, double* mult = nullptr) {
   swap = fabs(a) > fabs(e.r0);
   Pivot p;
   p.u0 = swap ? a : e.r0;
@@ -144,6 +144,7 @@ __device__ __forceinline__ Pivot elim_step(Elim& e, double a, double b, double c
   const bool live = p.u0 != 0.0;
   const double rp = 1.0 / p.u0;
   const double l = rp * o0;
+  if (mult) *mult = live ? l : 0.0;
   const double n1 = o1 + l * (-p.u1), n2 = o2 + l * (-p.u2), nd = od + l * (-p.y);
   e.r0 = live & (p.u1 != 0.0) ? n1 : o1;
   e.r1 = live & (p.u2 != 0.0) ? n2 : o2;
@@ -605,6 +606,243 @@ __global__ __launch_bounds__(64, 2) void k_diffusion(DevGrid g, DevState s, doub
   diffusion_block<R, BE, EXT>(g, s, blockIdx.x, scratch, k1, bdf, Teinf, sT, sC, sB, sD);
 }
 
+// ---------------------------------------------------------------- small grids
+// A grid with few columns leaves most of the GPU idle under the kernel above, whose waves then
+// take 1.5 us a row: four passes of a serial chain, the cells' conductivity and factors formed
+// by the same wave.  Here a workgroup of four waves owns W columns of one species and keeps
+// everything in LDS (nine doubles a row and column): all four form the parabolic terms, then
+// one wave eliminates both systems at once (lanes 0-31 the first solve, 32-63 the BDF2
+// matrix, one instruction stream) and keeps the pivot rows in the place of the terms it has
+// used, so nothing is formed twice and each pass is one chain of a few dozen instructions.
+// Same operations and order as above.  Wave kernel -> this one: 128x64x1 188 -> 66 us,
+// 96x24x20 148 -> 58, 64x24x16 103 -> 41, 24x12x8 48 -> 18, 500x10x10 699 -> 243.
+//
+// LDS rows of Q_SLOTS x W doubles and one more (which spreads the rows over the banks for the
+// threads of the first phase, which run along x1): row r at r RS.  Rows 0, N+1 and N+2 exist
+// and hold nothing: the walks read a row or two ahead.
+enum : int { Q_T1 = 0, Q_T3 = 1, Q_T2 = 2, Q_Y = 3,      // terms, then U0 U1 U2 and the rhs
+             Q_T = 4,                                    // temperature, then the BDF2 rhs, x
+             Q_V = 5, Q_SLOTS = 9 };                     // C B D, then V0 V1 V2 and multiplier
+__host__ __device__ inline size_t small_lds_bytes(int N, int W) {
+  return (size_t)(N + 3) * (Q_SLOTS * W + 1) * sizeof(double) +
+         (size_t)((N + 31) / 32) * W * sizeof(int);
+}
+
+template <int W, bool BE, bool EXT>
+__global__ __launch_bounds__(256) void k_diffusion_small(DevGrid g, DevState s, Coef k1, Coef bdf,
+                                                         double Teinf) {
+  extern __shared__ double lds[];
+  const int N = g.lx1, tid = threadIdx.x;
+  const int ncol = g.lx2 * g.lx3;
+  const int c0 = blockIdx.x * W;                       // first column
+  const int isp = LSP - (int)blockIdx.y;               // (electrons first: the longer blocks)
+  const bool elec = isp == LSP;
+  const long so = (long)(isp - 1) * g.N, ni = (long)g.lx1 * ncol;
+  constexpr int RS = Q_SLOTS * W + 1;                  // doubles of a row
+  int* swb = (int*)(lds + (N + 3) * RS);               // BDF2 interchange words [word][W]
+  auto at = [&](int q, int r, int c) -> double& { return lds[r * RS + q * W + c]; };
+  const double gm1kB = (gammas(isp) - 1.0) / kB;
+  // temperature and the factors C, B, D of one cell, from HBM
+  auto cell = [&](int r, int col, double& T, double& C, double& B, double& D) {
+    const int i2 = col % g.lx2 + 1, i3 = col / g.lx2 + 1;
+    const long cb = gix(g, r, i2, i3), kb = (long)g.lx1 * col + r - 1;
+    const double h1 = g.h1[cb], h2 = g.h2[cb], h3 = g.h3[cb];
+    if (elec) {
+      CellIn<true> in;
+      in.T = s.Ts[so + cb]; in.n = s.ns[so + cb];
+      in.h1 = h1; in.h2 = h2; in.h3 = h3;
+      in.n1 = s.nn[kb]; in.n2 = s.nn[ni + kb]; in.n3 = s.nn[2 * ni + kb];
+      in.J = s.J1[cb];
+      in.kap = EXT && s.kappa ? s.kappa[col] : 1.0;
+      cell_coeffs<true, EXT>(in, isp, gm1kB, C, B, D);
+      T = in.T;
+    } else {
+      CellIn<false> in;
+      in.T = s.Ts[so + cb]; in.n = s.ns[so + cb];
+      in.h1 = h1; in.h2 = h2; in.h3 = h3;
+      cell_coeffs<false, false>(in, isp, gm1kB, C, B, D);
+      T = in.T;
+    }
+  };
+  const double* dx1i = g.dx1i - 1;
+  // the parabolic terms of row r from C(r), B(r), D(r-1..r+1)
+  auto terms = [&](int r, double C, double B, double Dm, double D, double Dp, double& t1, double& t2,
+                   double& t3) {
+    const double dxi = dx1i[r], dxl = g.dx1[r], dxr = g.dx1[r + 1], yi = g.rdx1i[r];
+    t1 = div_rcp(div_rcp(C * (0.5 * (Dm + D)), dxi, yi), dxl, g.rdx1[r]);
+    t3 = div_rcp(div_rcp(C * (0.5 * (D + Dp)), dxi, yi), dxr, g.rdx1[r + 1]);
+    t2 = elec ? div_rcp(B, dxr + dxl, g.rdx1s[r]) : 0.0;
+  };
+  // ---- terms: threads along x1 (columns past the last repeat it)
+  for (int t = tid; t < N * W; t += 256) {
+    const int c = t / N, r = t - c * N + 1;
+    double T, C, B, D;
+    cell(r, min(c0 + c, ncol - 1), T, C, B, D);
+    at(Q_T, r, c) = T;
+    at(Q_V, r, c) = C; at(Q_V + 1, r, c) = B; at(Q_V + 2, r, c) = D;
+  }
+  __syncthreads();
+  for (int t = tid; t < N * W; t += 256) {
+    const int c = t / N, r = t - c * N + 1;
+    if (r == 1 || r == N) continue;
+    double t1, t2, t3;
+    terms(r, at(Q_V, r, c), at(Q_V + 1, r, c), at(Q_V + 2, r - 1, c), at(Q_V + 2, r, c),
+          at(Q_V + 2, r + 1, c), t1, t2, t3);
+    at(Q_T1, r, c) = t1; at(Q_T3, r, c) = t3; at(Q_T2, r, c) = t2;
+  }
+  __syncthreads();
+  // ---- the solves: one wave; lanes past W repeat the last column
+  if ((tid >> 6) == (int)((blockIdx.x >> 8) & 3)) {    // (blocks of one CU on different SIMDs)
+    const int lane = tid & 63, c = min(lane & 31, W - 1);
+    const bool second = !BE && lane >= 32;             // the BDF2 factorisation
+    const int col = min(c0 + c, ncol - 1);
+    double Tmin, Tmax, aN = 0.0, bN = 1.0;
+    {
+      const long kb = (long)g.lx1 * col;
+      const double Tn1 = s.Tn[kb], TnN = s.Tn[kb + N - 1];
+      if (g.gridflag == 0) { Tmin = Tn1; Tmax = TnN; }
+      else if (g.gridflag == 1) { Tmax = TnN; Tmin = Teinf; }
+      else { Tmin = Tn1; Tmax = Teinf; }
+    }
+    if (EXT && elec && s.qtop) {                       // (see diffusion_unit)
+      const int i2 = col % g.lx2 + 1, i3 = col / g.lx2 + 1;
+      CellIn<true> top;
+      cell_load<true, true>(g, s, so, gix(g, 0, i2, i3), (long)g.lx1 * col, ni, N, top,
+                            hcol_index(g, col, N), col);
+      aN = -1.0 / g.dx1[N];
+      bN = 1.0 / g.dx1[N];
+      Tmax = (s.qtop[col] * top.h1) / cell_lambda<true, true>(top, isp);
+    }
+    const int nw = (N + 31) / 32;
+    int* prec = (EXT && elec && s.pivrec) ? s.pivrec + ((long)col * 2 + (second ? 1 : 0)) * nw : nullptr;
+    // first solve: TR takes half of each term; backward Euler and BDF2 the whole
+    const double half = BE || second ? 1.0 : 0.5, K = second ? bdf.K : k1.K;
+    const int out = second ? Q_V : Q_T1;
+    auto rhs1 = [&](double a, double tsum, double cc, double Tm, double Tc, double Tp) {
+      if (BE) return div_rcp(Tc, k1.dt, k1.K);
+      return ((div_rcp(Tc, k1.dt2, k1.K) - a * Tm) - tsum * Tc) - cc * Tp;
+    };
+    Elim e{1.0, 0.0, Tmin, false};
+    double Tm = at(Q_T, 1, c), Tc = at(Q_T, 2, c);
+    double n1 = at(Q_T1, 2, c), n2 = at(Q_T2, 2, c), n3 = at(Q_T3, 2, c), nT = at(Q_T, 3, c);
+    double* in = &at(0, 3, c);                         // the next row's terms
+    double* po = &at(out, 1, c);                       // pivot rows
+    // step j brings row j+1 in; the bits of its interchanges, 32 steps a word
+    auto step = [&](bool last) -> bool {
+      const double t1 = n1 * half, t2 = n2 * half, t3 = n3 * half, Tp = nT;
+      n1 = in[Q_T1 * W]; n2 = in[Q_T2 * W]; n3 = in[Q_T3 * W]; nT = in[Q_T * W + RS];
+      in += RS;
+      double a = -t1 + t2, b = (K + t3) + t1, cc = -t3 - t2, l;
+      double d = rhs1(a, t3 + t1, cc, Tm, Tc, Tp);
+      if (last) { a = aN; b = bN; cc = 0.0; d = Tmax; }
+      bool sw;
+      const Pivot p = elim_step(e, a, b, cc, d, sw, &l);
+      po[0] = p.u0; po[W] = p.u1; po[2 * W] = p.u2;
+      po[3 * W] = second ? l : p.y;
+      po += RS;
+      Tm = Tc; Tc = Tp;
+      return sw;
+    };
+    auto word = [&](int j, int bits) {
+      if (second) swb[(j >> 5) * W + c] = bits;
+      if (EXT && prec) prec[j >> 5] = bits;
+    };
+    for (int j0 = 0; j0 < N - 1; j0 += 32) {
+      int bits = 0;
+      const int je = min(j0 + 32, N - 1);              // row N's step comes after the loops
+#pragma unroll 4
+      for (int j = max(j0, 1); j < je; ++j) bits |= (step(false) ? 1 : 0) << (j & 31);
+      if (je == N - 1 && (je & 31)) bits |= (step(true) ? 1 : 0) << (je & 31);
+      word(j0, bits);
+    }
+    if (((N - 1) & 31) == 0) word(N - 1, step(true) ? 1 : 0);
+    if (e.r0 == 0.0) e.singular = true;
+    at(out, N, c) = e.r0; at(out + 1, N, c) = 0.0; at(out + 2, N, c) = 0.0;
+    if (!second) at(out + 3, N, c) = e.rb;
+    const int sing = e.singular ? 1 : 0;
+    const bool s1 = __shfl(sing, lane & 31) != 0, s2 = __shfl(sing, (lane & 31) + 32) != 0;
+    __builtin_amdgcn_wave_barrier();
+    // dgbsv leaves the right-hand side where a factorisation is singular (never on physical
+    // inputs): formed again from HBM, in the place of the eliminated one
+    if (__any(s1) && s1) {
+      at(Q_Y, 1, c) = Tmin;
+      at(Q_Y, N, c) = Tmax;
+      double T0, T1, T2, C0, C1, C2, B0, B1, B2, D0, D1, D2;
+      cell(1, col, T0, C0, B0, D0);
+      cell(2, col, T1, C1, B1, D1);
+      for (int r = 2; r < N; ++r) {
+        cell(r + 1, col, T2, C2, B2, D2);
+        double t1, t2, t3;
+        terms(r, C1, B1, D0, D1, D2, t1, t2, t3);
+        const double h = BE ? 1.0 : 0.5;
+        t1 *= h; t2 *= h; t3 *= h;
+        at(Q_Y, r, c) = rhs1(-t1 + t2, t3 + t1, -t3 - t2, T0, T1, T2);
+        T0 = T1; D0 = D1; T1 = T2; C1 = C2; B1 = B2; D1 = D2;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    // back substitution through the pivot rows at slots q0.., rhs in Q_Y
+    auto back = [&](int q0, bool singular, auto put) {
+      double x1 = 0.0, x2 = 0.0;
+      const double* pq = &at(0, N, c);
+      Pivot n{pq[q0 * W], pq[(q0 + 1) * W], pq[(q0 + 2) * W], pq[Q_Y * W]};
+      double* pT = &at(Q_T, N, c);
+#pragma unroll 4
+      for (int i = N; i >= 1; --i) {
+        const Pivot p = n;
+        pq -= RS;
+        n = Pivot{pq[q0 * W], pq[(q0 + 1) * W], pq[(q0 + 2) * W], pq[Q_Y * W]};
+        const double v = back_step(p, x1, x2), x = singular ? p.y : v;
+        *pT = put(*pT, x);
+        pT -= RS;
+        x2 = x1;
+        x1 = x;
+      }
+    };
+    auto floor100 = [&](double, double x) { return fmax_f(x, 100.0); };
+    if (BE) {
+      back(Q_T1, s1, floor100);
+    } else {
+      back(Q_T1, s1, [&](double T, double x) {
+        return -div_rcp(bdf.c13 * T, bdf.dt3, bdf.K) + div_rcp(bdf.c43 * x, bdf.dt3, bdf.K);
+      });
+      __builtin_amdgcn_wave_barrier();
+      // BDF2 forward solve through the kept interchanges and multipliers
+      const double* pi = &at(0, 1, c);                 // row j: multiplier; row j+1: rhs
+      double* py = &at(Q_Y, s2 ? 2 : 1, c);
+      double rb = Tmin, nd = pi[Q_T * W + RS], nl = pi[(Q_V + 3) * W];
+      if (s2) at(Q_Y, 1, c) = Tmin;
+      auto fwd = [&](int w, int j, bool last) {
+        const double d = last ? Tmax : nd, l = nl;
+        pi += RS;
+        nd = pi[Q_T * W + RS];
+        nl = pi[(Q_V + 3) * W];
+        const bool sw = (w >> (j & 31)) & 1;
+        const double pd = sw ? d : rb, od = sw ? rb : d;
+        const double nod = od + l * (-pd);
+        rb = pd != 0.0 ? nod : od;
+        *py = s2 ? d : pd;
+        py += RS;
+      };
+      for (int j0 = 0; j0 < N - 1; j0 += 32) {
+        const int w = swb[(j0 >> 5) * W + c], je = min(j0 + 32, N - 1);
+#pragma unroll 4
+        for (int j = max(j0, 1); j < je; ++j) fwd(w, j, false);
+        if (je == N - 1 && (je & 31)) fwd(w, je, true);
+      }
+      if (((N - 1) & 31) == 0) fwd(swb[((N - 1) >> 5) * W + c], N - 1, true);
+      if (!s2) at(Q_Y, N, c) = rb;
+      __builtin_amdgcn_wave_barrier();
+      back(Q_V, s2, floor100);
+    }
+  }
+  __syncthreads();
+  for (int t = tid; t < N * W; t += 256) {
+    const int c = t / N, r = t - c * N + 1, col = c0 + c;
+    if (col < ncol) s.Ts[so + gix(g, r, col % g.lx2 + 1, col / g.lx2 + 1)] = at(Q_T, r, c);
+  }
+}
+
 }  // namespace
 
 void launch_floor_ghosts(const DevGrid& g, double* Ts, hipStream_t st);
@@ -723,10 +961,52 @@ size_t diffusion_noalloc_bytes(const DevGrid& g) {
 }
 
 namespace {
+// Columns per block of the small-grid kernel, 0 where the wave kernel is faster: the fewest
+// that leave at most one block per CU (the solving waves of two would share a SIMD), else the
+// most that fit the LDS, if that takes at most two rounds of blocks: a round takes 0.5-0.7 us
+// a row, the wave kernel 1.4-1.6 at these sizes (98x40x36, 2.46 rounds: 160 by waves, 167
+// here; 300x20x20, 2.73: 435 and 437; 64x64x64, 3.5: 125 and 170).
+#ifndef SMALL_ROUNDS
+#define SMALL_ROUNDS 2.0
+#endif
+int small_columns(const DevGrid& g) {
+  constexpr size_t LDS = 160 * 1024;
+  constexpr long CUS = 256;
+  const long ncol = (long)g.lx2 * g.lx3;
+  int best = 0;
+  for (int W = 2; W <= 16; W *= 2) {
+    const size_t b = small_lds_bytes(g.lx1, W);
+    if (b > LDS) break;
+    const long blocks = (ncol + W - 1) / W * LSP;
+    if (blocks <= CUS) return W;
+    best = (double)blocks <= SMALL_ROUNDS * CUS * (double)(LDS / b) ? W : 0;
+  }
+  return best;
+}
+
+template <int W>
+void small_launch(const DevGrid& g, const DevState& s, int diffsolvetype, double Teinf,
+                  const Coef& tr, const Coef& bdf, const Coef& be, hipStream_t st) {
+  const dim3 grd((unsigned)(((long)g.lx2 * g.lx3 + W - 1) / W), LSP), blk(256);
+  const size_t b = small_lds_bytes(g.lx1, W);
+  if (diffsolvetype == 1)
+    hipLaunchKernelGGL((k_diffusion_small<W, true, false>), grd, blk, b, st, g, s, be, bdf, Teinf);
+  else if (s.kappa || s.qtop)
+    hipLaunchKernelGGL((k_diffusion_small<W, false, true>), grd, blk, b, st, g, s, tr, bdf, Teinf);
+  else
+    hipLaunchKernelGGL((k_diffusion_small<W, false, false>), grd, blk, b, st, g, s, tr, bdf, Teinf);
+}
+
 template <int R>
 void diffusion_launch(const DevGrid& g, const DevState& s, int diffsolvetype, double Teinf,
                       double* scratch, const Coef& tr, const Coef& bdf, const Coef& be,
                       hipStream_t st) {
+  switch (R == 4 ? 0 : small_columns(g)) {             // (the 4-row variant: waves always)
+    case 16: return small_launch<16>(g, s, diffsolvetype, Teinf, tr, bdf, be, st);
+    case 8: return small_launch<8>(g, s, diffsolvetype, Teinf, tr, bdf, be, st);
+    case 4: return small_launch<4>(g, s, diffsolvetype, Teinf, tr, bdf, be, st);
+    case 2: return small_launch<2>(g, s, diffsolvetype, Teinf, tr, bdf, be, st);
+  }
   const dim3 grd((unsigned)((diffusion_groups(g) + 7) / 8 * 8 * LSP)), blk(64);
   if (diffsolvetype == 1)
     hipLaunchKernelGGL((k_diffusion<R, true>), grd, blk, 0, st, g, s, scratch, be, bdf, Teinf);

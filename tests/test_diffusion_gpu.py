@@ -1,7 +1,9 @@
 """GPU: the energy diffusion at the edges of its tiling, bit for bit against the oracle (with
 the GPU's correctly rounded x**2.5): lines a block of kept rows shorter or longer by one,
 column counts around a half group of 32, a group of 64 and an interleaved block of 128, both
-solvers and both chunk heights; and x**2.5 outside the range of its fast form."""
+solvers, both chunk heights (4 always takes the wave kernel) and the small-grid kernel at each
+of its block widths; singular columns in the wave kernel; the fitting extension in both; and
+x**2.5 outside the range of its fast form."""
 import numpy as np
 import pytest
 
@@ -15,7 +17,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("shape", [(4, 1, 1), (5, 7, 3), (7, 8, 4), (8, 31, 1), (9, 32, 1), (10, 33, 1),
                                    (15, 9, 7), (16, 13, 5), (17, 8, 16), (18, 43, 3), (23, 3, 43),
-                                   (24, 16, 17), (33, 20, 13), (40, 14, 14)])
+                                   (24, 16, 17), (33, 20, 13), (40, 14, 14),
+                                   # more columns than the small-grid kernel takes
+                                   (9, 115, 113), (16, 92, 91), (24, 77, 78), (33, 60, 61),
+                                   # lines that take it from 16 columns a block to two
+                                   (110, 3, 5), (230, 3, 3), (440, 2, 3), (700, 1, 3), (1100, 1, 2)])
 @pytest.mark.parametrize("solver", [2, 1])
 def test_diffusion_tiles_match_oracle(shape, solver):
     print(f"case {shape} solver {solver}", flush=True)
@@ -33,6 +39,50 @@ def test_diffusion_tiles_match_oracle(shape, solver):
         tr.set_tuning("diff_chunk", chunk)
         got = st.copy()
         tr.energy_diffusion(got, 0.3)
+        compare(got, ref, exact=("Ts", "ns"))
+    tr.close()
+
+
+@pytest.mark.parametrize("solver", [2, 1])
+def test_singular_columns_in_both_kernels(solver):
+    """Zero temperature on five rows and an infinite step make exact zero pivots."""
+    g = ga.cartesian_grid(20, 40, 3)
+    st = ga.synthetic_state(g, seed=5)
+    st.J1[...] = 0.0
+    for isp, i2, i3 in ((1, 2, 1), (3, 39, 2), (6, 7, 2)):
+        st.Ts[8:13, i2 + 1, i3 + 1, isp] = 0.0
+    ref = st.copy()
+    with oracle.pow_mode(1):
+        oracle.op(g, ref, "energy_diffusion", dt=np.inf, diffsolvetype=solver)
+    tr = Transport(g, st.nn, st.Tn, own_context=True, diffsolvetype=solver)
+    for chunk in (8, 4):
+        tr.set_tuning("diff_chunk", chunk)
+        got = st.copy()
+        tr.energy_diffusion(got, np.inf)
+        compare(got, ref, exact=("Ts",))
+    tr.close()
+
+
+@pytest.mark.parametrize("shape", [(21, 5, 3), (64, 9, 8)])
+def test_fitting_extension_in_both_kernels(shape):
+    g = ga.cartesian_grid(*shape)
+    st = ga.synthetic_state(g, seed=6)
+    rng = np.random.default_rng(7)
+    kappa = rng.uniform(0.5, 1.5, (g.lx2, g.lx3))
+    qtop = rng.uniform(0.0, 1e-5, (g.lx2, g.lx3))
+    ref = st.copy()
+    with oracle.pow_mode(1):
+        oracle.transport_step(g, ref, 0.2, kappa=kappa, qtop=qtop)
+    tr = Transport(g, st.nn, st.Tn, own_context=True)
+    tr.set_conductivity_scale(kappa)
+    tr.set_top_heat_flux(qtop)
+    tr.set_residency(1)
+    for chunk in (8, 4):
+        tr.set_tuning("diff_chunk", chunk)
+        got = st.copy()
+        tr.push(got)
+        tr.transport_step(0.2)
+        tr.pull(got)
         compare(got, ref, exact=("Ts", "ns"))
     tr.close()
 
