@@ -8,27 +8,36 @@
 // every cell (ghosts included, as the reference's whole-array statements do) then converts
 // back to temperature / velocity / electron density.  The rates never touch HBM.
 //
-// Arithmetic follows the reference's expressions (-ffp-contract=off), with liberties that
-// cost a few ulp per operation: a divide by a compile-time constant (a mass sum, 3) is a
-// multiply by its correctly rounded reciprocal; within a Coulomb pair 1/Teff is formed once
-// and gives Teff**-1.5 and W**2, and exp(-W**2) below W = 0.1 is a Taylor series.  The
-// transcendental functions (exp, log, log10, erf, tanh, sin, and x**p for the fitted
-// exponents) are the device library's, which agree with glibc to about an ulp; x**0.5 is
-// the correctly rounded sqrt.  These passes therefore match the reference to rounding (the
-// tests hold them to 1e-12 of each field's magnitude) rather than bit for bit.
+// Arithmetic follows the reference's expressions, with liberties that cost a few ulp per
+// operation at most: products and sums contract into FMAs in this file, a divide by a
+// compile-time constant (a mass sum, 3) is a multiply by its correctly rounded reciprocal, a
+// Coulomb pair's powers of 1/Teff come from one reciprocal root and its drift functions from
+// their series.  The transcendental functions (exp, log, log10, erf, tanh, sin, and x**p for
+// the fitted exponents) are the device library's, which agree with glibc to about an ulp;
+// x**0.5 is the correctly rounded sqrt.  These passes therefore match the reference to
+// rounding (the tests hold them to 1e-12 of each field's magnitude) rather than bit for bit.
 //
 // Ion-ion (Coulomb) terms: Teff, Wsj, Phisj and Psisj of coulomb_colln are symmetric in
 // the species pair, so each unordered pair is evaluated once and feeds both species.  The
 // pairs run in lexicographic order, which adds each species' terms in the reference's
-// isp2 order; self-collision terms are exact zeros and are skipped.  The pair loop is
-// rolled in the energy kernel (one copy of exp and erf instead of 21, per-species values
-// selected by a wave-uniform index), which keeps it within 256 registers.
+// isp2 order; self-collision terms are exact zeros and are skipped.
+//
+// On 512x256x192 the energy pass moves 13.5 GB in 3.33 ms, the momentum pass 13.5 GB in
+// 3.79 ms, the mass pass 9.9 GB in 1.92 ms (a large copy takes 3.1, 3.1 and 2.3 ms for as
+// much).  The first two were bound by their instructions, some 8000 a cell, at 5.5 and
+// 6.5 ms: erf and exp in every pair; register arrays indexed by a rolled loop's pair, or 130
+// KB of unrolled code that misses the instruction cache; the edge logarithms of a gradient
+// inlined once per use.  Blocks of 128 threads are 2 to 4 % faster than 256.  Momentum is
+// held to 168 registers (3 waves per SIMD: 3.79 ms against 4.25); energy at 168 spills and
+// takes 5.1 ms against 3.33 at 223.
 #include "gemhip_internal.h"
+
+#pragma clang fp contract(fast)
 
 namespace gemhip {
 namespace {
 
-constexpr int TPB = 256;
+constexpr int TPB = 128;
 constexpr double PI = 3.141592653589793;   // 4*atan(1.0_wp), phys_consts.in.f90:20
 
 // collisions.f90:11-47: default-real literals widened to real64
@@ -90,109 +99,104 @@ __device__ __forceinline__ double maxwell(int isp, int isp2, double nn2, double 
   }
 }
 
-// Tables of the rolled pair loop.  The pair index is the same on every lane of a wave, so
-// these are scalar loads; each entry is the constant expression the unrolled form would
-// fold at compile time.  Pairs run (1,2), (1,3), .., (1,7), (2,3), .., (6,7).
-__constant__ int c_pair_a[21] = {1, 1, 1, 1, 1, 1, 2, 2, 2, 2, 2, 3, 3, 3, 3, 4, 4, 4, 5, 5, 6};
-__constant__ int c_pair_b[21] = {2, 3, 4, 5, 6, 7, 3, 4, 5, 6, 7, 4, 5, 6, 7, 5, 6, 7, 6, 7, 7};
-__constant__ double c_ms[7] = {
-    16.0 * amu, 30.0 * amu, 28.0 * amu, 32.0 * amu,
-    14.0 * amu, 1.0 * amu, 5.485799090e-4 * amu};
-__constant__ double c_ms3[7] = {
-    (16.0 * amu) / 3.0, (30.0 * amu) / 3.0, (28.0 * amu) / 3.0,
-    (32.0 * amu) / 3.0, (14.0 * amu) / 3.0, (1.0 * amu) / 3.0,
-    (5.485799090e-4 * amu) / 3.0};
-__constant__ double c_nkB_igm1[7] = {
-    kB * (1.0 / (5.0 / 3.0 - 1.0)), kB * (1.0 / (7.0 / 5.0 - 1.0)),
-    kB * (1.0 / (7.0 / 5.0 - 1.0)), kB * (1.0 / (7.0 / 5.0 - 1.0)),
-    kB * (1.0 / (5.0 / 3.0 - 1.0)), kB * (1.0 / (5.0 / 3.0 - 1.0)),
-    kB * (1.0 / (5.0 / 3.0 - 1.0))};
-__constant__ double c_igm1[7] = {
-    1.0 / (5.0 / 3.0 - 1.0), 1.0 / (7.0 / 5.0 - 1.0), 1.0 / (7.0 / 5.0 - 1.0),
-    1.0 / (7.0 / 5.0 - 1.0), 1.0 / (5.0 / 3.0 - 1.0), 1.0 / (5.0 / 3.0 - 1.0),
-    1.0 / (5.0 / 3.0 - 1.0)};
-__constant__ double c_two_msum[21] = {
-    2.0 / ((16.0 * amu) + (30.0 * amu)), 2.0 / ((16.0 * amu) + (28.0 * amu)),
-    2.0 / ((16.0 * amu) + (32.0 * amu)), 2.0 / ((16.0 * amu) + (14.0 * amu)),
-    2.0 / ((16.0 * amu) + (1.0 * amu)), 2.0 / ((16.0 * amu) + (5.485799090e-4 * amu)),
-    2.0 / ((30.0 * amu) + (28.0 * amu)), 2.0 / ((30.0 * amu) + (32.0 * amu)),
-    2.0 / ((30.0 * amu) + (14.0 * amu)), 2.0 / ((30.0 * amu) + (1.0 * amu)),
-    2.0 / ((30.0 * amu) + (5.485799090e-4 * amu)), 2.0 / ((28.0 * amu) + (32.0 * amu)),
-    2.0 / ((28.0 * amu) + (14.0 * amu)), 2.0 / ((28.0 * amu) + (1.0 * amu)),
-    2.0 / ((28.0 * amu) + (5.485799090e-4 * amu)), 2.0 / ((32.0 * amu) + (14.0 * amu)),
-    2.0 / ((32.0 * amu) + (1.0 * amu)), 2.0 / ((32.0 * amu) + (5.485799090e-4 * amu)),
-    2.0 / ((14.0 * amu) + (1.0 * amu)), 2.0 / ((14.0 * amu) + (5.485799090e-4 * amu)),
-    2.0 / ((1.0 * amu) + (5.485799090e-4 * amu))};
-__constant__ double c_inv_msum[21] = {
-    1.0 / ((30.0 * amu) + (16.0 * amu)), 1.0 / ((28.0 * amu) + (16.0 * amu)),
-    1.0 / ((32.0 * amu) + (16.0 * amu)), 1.0 / ((14.0 * amu) + (16.0 * amu)),
-    1.0 / ((1.0 * amu) + (16.0 * amu)), 1.0 / ((5.485799090e-4 * amu) + (16.0 * amu)),
-    1.0 / ((28.0 * amu) + (30.0 * amu)), 1.0 / ((32.0 * amu) + (30.0 * amu)),
-    1.0 / ((14.0 * amu) + (30.0 * amu)), 1.0 / ((1.0 * amu) + (30.0 * amu)),
-    1.0 / ((5.485799090e-4 * amu) + (30.0 * amu)), 1.0 / ((32.0 * amu) + (28.0 * amu)),
-    1.0 / ((14.0 * amu) + (28.0 * amu)), 1.0 / ((1.0 * amu) + (28.0 * amu)),
-    1.0 / ((5.485799090e-4 * amu) + (28.0 * amu)), 1.0 / ((14.0 * amu) + (32.0 * amu)),
-    1.0 / ((1.0 * amu) + (32.0 * amu)), 1.0 / ((5.485799090e-4 * amu) + (32.0 * amu)),
-    1.0 / ((1.0 * amu) + (14.0 * amu)), 1.0 / ((5.485799090e-4 * amu) + (14.0 * amu)),
-    1.0 / ((5.485799090e-4 * amu) + (1.0 * amu))};
-__constant__ double c_csj_1e6[7][7] = {
-    {(double)0.22f * 1e-6, (double)0.26f * 1e-6, (double)0.25f * 1e-6, (double)0.26f * 1e-6, (double)0.22f * 1e-6, (double)0.077f * 1e-6, (double)1.87e-3f * 1e-6},
-    {(double)0.14f * 1e-6, (double)0.16f * 1e-6, (double)0.16f * 1e-6, (double)0.17f * 1e-6, (double)0.13f * 1e-6, (double)0.042f * 1e-6, (double)9.97e-4f * 1e-6},
-    {(double)0.15f * 1e-6, (double)0.17f * 1e-6, (double)0.17f * 1e-6, (double)0.18f * 1e-6, (double)0.14f * 1e-6, (double)0.045f * 1e-6, (double)1.07e-3f * 1e-6},
-    {(double)0.13f * 1e-6, (double)0.16f * 1e-6, (double)0.15f * 1e-6, (double)0.16f * 1e-6, (double)0.12f * 1e-6, (double)0.039f * 1e-6, (double)9.347e-4f * 1e-6},
-    {(double)0.25f * 1e-6, (double)0.28f * 1e-6, (double)0.28f * 1e-6, (double)0.28f * 1e-6, (double)0.24f * 1e-6, (double)0.088f * 1e-6, (double)2.136e-3f * 1e-6},
-    {(double)1.23f * 1e-6, (double)1.25f * 1e-6, (double)1.25f * 1e-6, (double)1.25f * 1e-6, (double)1.23f * 1e-6, (double)0.90f * 1e-6, (double)29.7e-3f * 1e-6},
-    {(double)54.5f * 1e-6, (double)54.5f * 1e-6, (double)54.5f * 1e-6, (double)54.5f * 1e-6, (double)54.5f * 1e-6, (double)54.5f * 1e-6, (double)38.537f * 1e-6}};
-
-// mred/(2 kB) of each pair, so that W**2 = (dv**2) mred/(2 kB Teff)
-__constant__ double c_mred_2kB[21] = {
-#define GEMHIP_MRED_2KB(ma, mb) ((((ma) * amu) * ((mb) * amu)) / (((ma) * amu) + ((mb) * amu))) / (2.0 * kB)
-    GEMHIP_MRED_2KB(16.0, 30.0), GEMHIP_MRED_2KB(16.0, 28.0), GEMHIP_MRED_2KB(16.0, 32.0),
-    GEMHIP_MRED_2KB(16.0, 14.0), GEMHIP_MRED_2KB(16.0, 1.0), GEMHIP_MRED_2KB(16.0, 5.485799090e-4),
-    GEMHIP_MRED_2KB(30.0, 28.0), GEMHIP_MRED_2KB(30.0, 32.0), GEMHIP_MRED_2KB(30.0, 14.0),
-    GEMHIP_MRED_2KB(30.0, 1.0), GEMHIP_MRED_2KB(30.0, 5.485799090e-4), GEMHIP_MRED_2KB(28.0, 32.0),
-    GEMHIP_MRED_2KB(28.0, 14.0), GEMHIP_MRED_2KB(28.0, 1.0), GEMHIP_MRED_2KB(28.0, 5.485799090e-4),
-    GEMHIP_MRED_2KB(32.0, 14.0), GEMHIP_MRED_2KB(32.0, 1.0), GEMHIP_MRED_2KB(32.0, 5.485799090e-4),
-    GEMHIP_MRED_2KB(14.0, 1.0), GEMHIP_MRED_2KB(14.0, 5.485799090e-4),
-    GEMHIP_MRED_2KB(1.0, 5.485799090e-4)};
-#undef GEMHIP_MRED_2KB
-
-// exp(-x) for 0 <= x < 0.01: Taylor series to x**6 (the remainder is below x**7/5040, 2e-18)
-__device__ __forceinline__ double exp_neg_small(double x) {
-  double r = 1.0 / 720.0;
-  r = r * x - 1.0 / 120.0;
-  r = r * x + 1.0 / 24.0;
-  r = r * x - 1.0 / 6.0;
-  r = r * x + 0.5;
-  r = r * x - 1.0;
-  return r * x + 1.0;
+// collisions.f90:22-31 (Csj), times the 1e-6 of :146
+__device__ __forceinline__ double csj_1e6(int x, int y) {
+  constexpr float t[7][7] = {
+      {0.22f, 0.26f, 0.25f, 0.26f, 0.22f, 0.077f, 1.87e-3f}, {0.14f, 0.16f, 0.16f, 0.17f, 0.13f, 0.042f, 9.97e-4f},
+      {0.15f, 0.17f, 0.17f, 0.18f, 0.14f, 0.045f, 1.07e-3f}, {0.13f, 0.16f, 0.15f, 0.16f, 0.12f, 0.039f, 9.347e-4f},
+      {0.25f, 0.28f, 0.28f, 0.28f, 0.24f, 0.088f, 2.136e-3f}, {1.23f, 1.25f, 1.25f, 1.25f, 1.23f, 0.90f, 29.7e-3f},
+      {54.5f, 54.5f, 54.5f, 54.5f, 54.5f, 54.5f, 38.537f}};
+  return (double)t[x - 1][y - 1] * 1e-6;
 }
 
-// the pair-symmetric part of coulomb_colln (collisions.f90:138-157) for pair pr = (a, b),
-// a < b: 1/Teff**1.5, Phisj, Psisj.  1/Teff is formed once: Teff**-1.5 = (1/Teff)
-// sqrt(1/Teff) and W**2 = dv**2 (mred/(2 kB)) (1/Teff), each a few ulp from the
-// reference's forms.  Below W = 0.1 (W**2 = 0.01), where Phisj = 1, W itself is not needed
-// and Psisj = exp(-W**2) comes from its Taylor series.
-struct Pair { double iT15, Phi, Psi; };
-__device__ __forceinline__ Pair coulomb_pair(int pr, double Ta, double Tb, double va, double vb) {
-  const int a = c_pair_a[pr], b = c_pair_b[pr];
-  const double ma = c_ms[a - 1], mb = c_ms[b - 1];
-  const double Teff = (mb * Ta + ma * Tb) * c_inv_msum[pr];
-  const double iTeff = 1.0 / Teff;
+// Psi = exp(-x) and Phi = 3 int_0^1 t^2 exp(-x t^2) dt for x = W**2 in [0, 1]: their power
+// series, sum (-x)^k/k! and sum 3 (-x)^k/(k! (2k+3)), interpolated at Chebyshev points (off
+// by 8e-18 and 3e-17 at most).  A table in memory, so that it is read into scalar registers.
+__constant__ double c_drift[25] = {
+    1.0, -0.5999999999999948, 0.21428571428546575, -0.05555555555090525, 0.011363636318628153,
+    -0.0019230766656642064, 0.0002777768425337601, -3.5011761846027854e-05, 3.912431467016512e-06,
+    -3.898097348795919e-07, 3.327267488170533e-08, -1.9011473537307833e-09,
+    1.0, -0.999999999999999, 0.4999999999999427, -0.16666666666540417, 0.041666666652193346,
+    -0.008333333234481316, 0.0013888884549085943, -0.00019841141919339013, 2.4798998659720724e-05,
+    -2.7521178006932173e-06, 2.721363367981267e-07, -2.2905624278899246e-08, 1.2719039650810423e-09};
+template <int DEG>
+__device__ __forceinline__ double horner(const double* c, double x) {
+  double b = c[DEG];
+#pragma unroll
+  for (int k = DEG - 1; k >= 0; --k) b = __builtin_fma(b, x, c[k]);
+  return b;
+}
+
+// The pair-symmetric part of coulomb_colln (collisions.f90:138-157) for species a < b:
+// 1/Teff**1.5 and W**2.  1/Teff and its power come from one v_rsq_f64: two Newton steps give
+// the reciprocal root to about an ulp, one residual correction its square.
+struct Pair { double iT15, W2; };
+__device__ __forceinline__ Pair coulomb_pair(double ma, double mb, double Ta, double Tb, double va, double vb) {
+  const double x = __builtin_fma(mb, Ta, ma * Tb) * (1.0 / (mb + ma));
+  double y = __builtin_amdgcn_rsq(x);
+  y = __builtin_fma(0.5 * y, __builtin_fma(-(x * y), y, 1.0), y);
+  y = __builtin_fma(0.5 * y, __builtin_fma(-(x * y), y, 1.0), y);
+  const double q = y * y;
+  const double iTeff = __builtin_fma(q, __builtin_fma(-x, q, 1.0), q);
   const double dv = va - vb;
-  const double W2 = ((dv * dv) * c_mred_2kB[pr]) * iTeff;
-  Pair p;
-  p.iT15 = iTeff * sqrt(iTeff);
-  if (W2 < 0.01) {
-    p.Phi = 1.0;
-    p.Psi = exp_neg_small(W2);
-  } else {
-    const double W = sqrt(W2);
-    p.Psi = exp(-W2);
-    const double iW = 1.0 / W, iW2 = iW * iW;
-    p.Phi = (((3.0 / 4.0) * sqrt(PI)) * erf(W)) * (iW2 * iW) - ((3.0 / 2.0) * iW2) * p.Psi;
+  return {iTeff * y, ((dv * dv) * (((ma * mb) / (ma + mb)) / (2.0 * kB))) * iTeff};
+}
+
+// Phisj and Psisj above W**2 = 1 (the reference's closed form; Phisj is 1 below W = 0.1)
+__device__ __forceinline__ void drift_far(double W2, double& Phi, double& Psi) {
+  const double W = sqrt(W2), iW = 1.0 / W, iW2 = iW * iW;
+  Psi = exp(-W2);
+  Phi = (((3.0 / 4.0) * sqrt(PI)) * erf(W)) * (iW2 * iW) - ((3.0 / 2.0) * iW2) * Psi;
+}
+// the bit of the unordered pair a < b in a mask of the 21 pairs
+__device__ __forceinline__ constexpr int pair_bit(int a, int b) { return (a - 1) * (14 - a) / 2 + (b - a - 1); }
+constexpr double W2_NEAR = 1.0;
+
+// The Coulomb terms of all species pairs.  add(x, y, iT15 Phi, iT15 Psi, Ty, v1y, ny) takes
+// species x's share of its collisions with y.  Up to W**2 = 1 (a drift of 1.5 km/s between
+// heavy ions, hundreds of km/s between ions and electrons) Phi and Psi are the series: no
+// branch, so that the 21 unrolled pairs stay one run of instructions.  Pairs beyond enter
+// with zeros there, are marked in a mask, and lanes that hold any add them afterwards in a
+// rolled loop over the partner, whose values it reads again (it is never entered at ordinary
+// drifts, and its erf and exp would otherwise be part of every pair).
+template <bool PSI, int NX, typename ADD>
+__device__ __forceinline__ void coulomb_terms(const DevGrid& g, const DevState& s, long c, const double* n,
+                                              const double* T, const double* v1, ADD add) {
+  unsigned far = 0;
+#pragma unroll
+  for (int a = 1; a < LSP; ++a) {
+#pragma unroll
+    for (int b = a + 1; b <= LSP; ++b) {
+      const Pair p = coulomb_pair(ms(a), ms(b), T[a - 1], T[b - 1], v1[a - 1], v1[b - 1]);
+      const bool f = !(p.W2 <= W2_NEAR);
+      const double i = f ? 0.0 : p.iT15;
+      far |= f ? 1u << pair_bit(a, b) : 0u;
+      double phi = horner<11>(c_drift, p.W2);
+      phi = i * (p.W2 < 0.01 ? 1.0 : phi);
+      const double psi = PSI ? i * horner<12>(c_drift + 12, p.W2) : 0.0;
+      const double phi_f = f ? 0.0 : phi, psi_f = f ? 0.0 : psi;   // (0 times an infinity is no zero)
+      add(a, b, phi_f, psi_f, T[b - 1], v1[b - 1], n[b - 1], false);
+      if (b <= NX) add(b, a, phi_f, psi_f, T[a - 1], v1[a - 1], n[a - 1], false);
+      __builtin_amdgcn_sched_barrier(0);         // (keeps one pair's values in registers)
+    }
   }
-  return p;
+  if (far) {
+#pragma unroll
+    for (int x = 1; x <= NX; ++x) {
+#pragma unroll 1
+      for (int y = 1; y <= LSP; ++y) {
+        if (y == x) continue;
+        const int a = x < y ? x : y, b = x < y ? y : x;
+        if (!(far >> pair_bit(a, b) & 1u)) continue;
+        const long o = (long)(y - 1) * g.N + c;
+        const double Ty = s.Ts[o], vy = s.vs1[o], ny = s.ns[o];
+        const Pair p = coulomb_pair(ms(x), ms(y), T[x - 1], Ty, v1[x - 1], vy);
+        double Phi, Psi;
+        drift_far(p.W2, Phi, Psi);
+        add(x, y, p.iT15 * Phi, p.iT15 * Psi, Ty, vy, ny, true);
+      }
+    }
+  }
 }
 
 struct Cell {
@@ -236,48 +240,39 @@ __global__ __launch_bounds__(TPB) void k_src_energy(DevGrid g, DevState s, DevSo
     double nnk[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) nnk[j] = a.nn[j * ni + k];
-    // ion-neutral and electron-neutral: heat transfer and friction
+    // ion-neutral and electron-neutral: heat transfer and friction.  Every production term
+    // of species isp carries the factor ns ms/(gamma-1), which is applied at the end.
 #pragma unroll
     for (int isp = 1; isp <= LSP; ++isp) {
-      const double m = ms(isp), gm1 = gammas(isp) - 1.0, nm = n[isp - 1] * m;
+      const double m = ms(isp);
       const double d1 = v1[isp - 1] - vn1, d2 = v2[isp - 1] - vn2, d3 = v3[isp - 1] - vn3;
       const double dv2 = ((d1 * d1) + (d2 * d2)) + (d3 * d3);
-      const double heat = (nm * kB) * (1.0 / gm1), fric = (nm * (1.0 / gm1)) * dv2;
       double Pp = 0.0, Ll = 0.0;
 #pragma unroll
       for (int isp2 = 1; isp2 <= 4; ++isp2) {
         const double nu = maxwell(isp, isp2, nnk[isp2 - 1], Tn, T[isp - 1]);
-        double fact = nu * (2.0 / (m + mn(isp2)));
-        Pp = Pp + (heat * fact) * Tn;
-        Ll = Ll + m * fact;
-        fact = fact * (mn(isp2) / 3.0);
-        Pp = Pp + fric * fact;
+        const double fact = nu * (2.0 / (m + mn(isp2)));
+        Pp = Pp + fact * (kB * Tn + (mn(isp2) / 3.0) * dv2);
+        Ll = Ll + fact;
       }
       P[isp - 1] = Pp;
-      L[isp - 1] = Ll;
+      L[isp - 1] = m * Ll;
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // ion-ion and ion-electron (Coulomb), one unordered pair per iteration
-#pragma unroll 1
-    for (int pr = 0; pr < 21; ++pr) {
-      const int ia = c_pair_a[pr], ib = c_pair_b[pr];
-      const Pair p = coulomb_pair(pr, T[ia - 1], T[ib - 1], v1[ia - 1], v1[ib - 1]);
-      const double d1 = v1[ia - 1] - v1[ib - 1], d2 = v2[ia - 1] - v2[ib - 1],
-                   d3 = v3[ia - 1] - v3[ib - 1];
-      const double dv2 = ((d1 * d1) + (d2 * d2)) + (d3 * d3);
-      const double psi2 = p.Psi * c_two_msum[pr], phi2 = p.Phi * c_two_msum[pr];
-      // species ia with partner ib, then ib with partner ia
+    // ion-ion and ion-electron (Coulomb)
+    coulomb_terms<true, LSP>(g, s, c, n, T, v1,
+        [&](int x, int y, double phi, double psi, double Ty, double v1y, double ny, bool again) {
+          const long o = (long)(y - 1) * g.N + c;
+          const double d1 = v1[x - 1] - v1y, d2 = v2[x - 1] - (again ? s.vs2[o] : v2[y - 1]),
+                       d3 = v3[x - 1] - (again ? s.vs3[o] : v3[y - 1]);
+          const double dv2 = ((d1 * d1) + (d2 * d2)) + (d3 * d3);
+          const double c2 = csj_1e6(x, y) * (2.0 / (ms(x) + ms(y)));
+          const double npsi = ny * psi;
+          P[x - 1] = P[x - 1] + (c2 * kB) * (npsi * Ty) + (c2 * (ms(y) / 3.0)) * (ny * (phi * dv2));
+          L[x - 1] = L[x - 1] + (c2 * ms(x)) * npsi;
+        });
 #pragma unroll
-      for (int side = 0; side < 2; ++side) {
-        const int x = side ? ib : ia, y = side ? ia : ib;
-        const double nm = n[x - 1] * c_ms[x - 1];
-        const double nu = (c_csj_1e6[x - 1][y - 1] * n[y - 1]) * p.iT15;
-        double fact = nu * psi2;
-        P[x - 1] = P[x - 1] + ((nm * c_nkB_igm1[x - 1]) * fact) * T[y - 1];
-        L[x - 1] = L[x - 1] + c_ms[x - 1] * fact;
-        fact = (nu * phi2) * c_ms3[y - 1];
-        P[x - 1] = P[x - 1] + ((nm * c_igm1[x - 1]) * dv2) * fact;
-      }
-    }
+    for (int i = 1; i <= LSP; ++i) P[i - 1] = (n[i - 1] * (ms(i) * (1.0 / (gammas(i) - 1.0)))) * P[i - 1];
     // inelastic electron-neutral collisions (sources.f90:350-373)
     const double sfact = (elchrg / kB) * (gammas(LSP) - 1.0);
     const double Te = T[LSP - 1], nn2 = nnk[1], nn3 = nnk[2];
@@ -312,34 +307,30 @@ __global__ __launch_bounds__(TPB) void k_src_energy(DevGrid g, DevState s, DevSo
   }
 }
 
-// d(log p)/dx1 / h1 of species isp at interior cell c (gradient.f90:136-146): centred over
-// the ghost cells when the subdomain touches neither x1 end, otherwise over the interior
-// with one-sided differences at i1 = 1 and lx1 (sources.f90:259-270).  lp holds log p of
-// the block's cells (x1 neighbours are neighbouring threads); cells outside the block are
-// evaluated directly, with the same expression.
-__device__ __forceinline__ double dlogp(const DevGrid& g, const DevState& s, const double* lp,
-                                        int isp, long c, int t, int i1, bool ghosted) {
-  const long o = (long)(isp - 1) * g.N;
-  auto at = [&](int dt_) -> double {
-    const int u = t + dt_;
-    if (u >= 0 && u < TPB) return lp[(isp - 1) * TPB + u];
-    return log((s.ns[o + c + dt_] * kB) * s.Ts[o + c + dt_]);
-  };
-  if (!ghosted) {
-    if (i1 == 1) return ((at(1) - at(0)) / g.dx1[1]) / g.h1[c];
-    if (i1 == g.lx1) return ((at(0) - at(-1)) / g.dx1[g.lx1]) / g.h1[c];
-  }
-  return ((at(1) - at(-1)) / (g.dx1[i1 + 1] + g.dx1[i1])) / g.h1[c];
-}
+// The divisors of an x1 gradient at cell i1 (centred, or one-sided at the ends: gradient.f90:
+// 136-146) and their correctly rounded reciprocals, for the gradients of a cell's seven log
+// pressures, six viscosities and two metric factors.
+struct Grad {
+  double d, yd, h, yh;
+  __device__ __forceinline__ double operator()(double diff) const { return div_rcp(div_rcp(diff, d, yd), h, yh); }
+};
 
 // ---- source_loss_momentum: srcsMomentum_curv (sources.f90:228-289), ETD, velocities ----
-__global__ __launch_bounds__(TPB) void k_src_momentum(DevGrid g, DevState s, DevSources a, double dt) {
-  __shared__ double lp[LSP * TPB];
+__global__ __launch_bounds__(TPB, 3) void k_src_momentum(DevGrid g, DevState s, DevSources a, double dt) {
+  // log p of the block's cells and of the one before and after them: x1 neighbours are
+  // neighbouring threads (a cell outside the grid is no interior cell's neighbour)
+  __shared__ double lp[LSP][TPB + 2];
   const int t = threadIdx.x;
-  const long c = (long)blockIdx.x * blockDim.x + t;
+  const long c0 = (long)blockIdx.x * TPB, c = c0 + t;
+  auto logp = [&](int i, long cc) { return log((s.ns[i * g.N + cc] * kB) * s.Ts[i * g.N + cc]); };
   if (c < g.N) {
 #pragma unroll
-    for (int i = 0; i < LSP; ++i) lp[i * TPB + t] = log((s.ns[i * g.N + c] * kB) * s.Ts[i * g.N + c]);
+    for (int i = 0; i < LSP; ++i) lp[i][t + 1] = logp(i, c);
+  }
+  if (t < 2 * LSP) {
+    const int i = t % LSP, u = t < LSP ? 0 : TPB + 1;
+    const long cc = c0 + u - 1;
+    if (cc >= 0 && cc < g.N) lp[i][u] = logp(i, cc);
   }
   __syncthreads();
   if (c >= g.N) return;
@@ -365,50 +356,49 @@ __global__ __launch_bounds__(TPB) void k_src_momentum(DevGrid g, DevState s, Dev
     for (int j = 0; j < 4; ++j) nnk[j] = a.nn[j * ni + k];
 #pragma unroll
     for (int isp = 1; isp <= LSP - 1; ++isp) {
-      const double nm = n[isp - 1] * ms(isp);
-      double Pp = 0.0, Ll = 0.0;
+      double Ll = 0.0;
 #pragma unroll
-      for (int isp2 = 1; isp2 <= 4; ++isp2) {
-        const double nu = maxwell(isp, isp2, nnk[isp2 - 1], Tn, T[isp - 1]);
-        Ll = Ll + nu;
-        Pp = Pp + (nm * nu) * vn1;
-      }
-      P[isp - 1] = Pp;
+      for (int isp2 = 1; isp2 <= 4; ++isp2) Ll = Ll + maxwell(isp, isp2, nnk[isp2 - 1], Tn, T[isp - 1]);
+      P[isp - 1] = Ll * vn1;                     // (times ns ms, applied at the end)
       L[isp - 1] = Ll;
+      __builtin_amdgcn_sched_barrier(0);
     }
+    coulomb_terms<false, LSP - 1>(g, s, c, n, T, v1,
+        [&](int x, int y, double phi, double, double, double v1y, double ny, bool) {
+          const double nphi = csj_1e6(x, y) * (ny * phi);
+          L[x - 1] = L[x - 1] + nphi;
+          P[x - 1] = P[x - 1] + nphi * v1y;
+        });
 #pragma unroll
-    for (int pr = 0; pr < 21; ++pr) {
-      const int ia = c_pair_a[pr], ib = c_pair_b[pr];
-      const Pair p = coulomb_pair(pr, T[ia - 1], T[ib - 1], v1[ia - 1], v1[ib - 1]);
-#pragma unroll
-      for (int side = 0; side < 2; ++side) {
-        const int x = side ? ib : ia, y = side ? ia : ib;
-        if (x == LSP) continue;
-        const double nu = (c_csj_1e6[x - 1][y - 1] * n[y - 1]) * p.iT15;
-        L[x - 1] = L[x - 1] + nu * p.Phi;
-        P[x - 1] = P[x - 1] + (((n[x - 1] * c_ms[x - 1]) * nu) * p.Phi) * v1[y - 1];
-      }
-    }
+    for (int i = 1; i < LSP; ++i) P[i - 1] = (n[i - 1] * ms(i)) * P[i - 1];
     // geometric factors, ambipolar field, gravity (sources.f90:248-288)
     const double h1 = g.h1[c], h2 = g.h2[c], h3 = g.h3[c];
     const double h1h2h3 = (h1 * h2) * h3;
-    const double dsum = g.dx1[i1 + 1] + g.dx1[i1];
-    const double dh2dx1 = ((g.h2[c + 1] - g.h2[c - 1]) / dsum) / h1;
-    const double dh3dx1 = ((g.h3[c + 1] - g.h3[c - 1]) / dsum) / h1;
+    // (sources.f90:259-270: centred over the ghost cells when the subdomain touches neither x1
+    // end, otherwise over the interior with one-sided differences at i1 = 1 and lx1)
+    const double dsum = g.dx1[i1 + 1] + g.dx1[i1], ysum = g.rdx1s[i1], yh1 = 1.0 / h1;
+    const Grad mid{dsum, ysum, h1, yh1};
+    const int lo = i1 == 1 ? 0 : -1, hi = i1 == g.lx1 ? 0 : 1;
+    const Grad one = i1 == 1 ? Grad{g.dx1[1], g.rdx1[1], h1, yh1}
+                   : i1 == g.lx1 ? Grad{g.dx1[g.lx1], g.rdx1[g.lx1], h1, yh1} : mid;
+    auto dlogp = [&](int isp) {
+      if (ghosted)
+        return mid(lp[isp - 1][t + 2] - lp[isp - 1][t]);
+      return one(lp[isp - 1][t + 1 + hi] - lp[isp - 1][t + 1 + lo]);
+    };
+    const double dh2dx1 = mid(g.h2[c + 1] - g.h2[c - 1]);
+    const double dh3dx1 = mid(g.h3[c + 1] - g.h3[c - 1]);
     const double Te = T[LSP - 1];
-    const double Epol1 = ((kB * Te) / qs(LSP)) * dlogp(g, s, lp, LSP, c, t, i1, ghosted);
+    const double Epol1 = ((kB * Te) / qs(LSP)) * dlogp(LSP);
     const double E1f = a.alt[c] < 100e3 ? 0.0 : a.E1[c];
     const double g1 = a.g1[k];
 #pragma unroll
     for (int isp = 1; isp <= LSP - 1; ++isp) {
       const double nsp = n[isp - 1], m = ms(isp);
       const double pr = (nsp * kB) * T[isp - 1];
-      const double ionpress = pr * dlogp(g, s, lp, isp, c, t, i1, ghosted);
+      const double ionpress = pr * dlogp(isp);
       const double* Qs = a.Q + (long)(isp - 1) * ni;
-      double gQ;
-      if (i1 == 1) gQ = ((Qs[k + 1] - Qs[k]) / g.dx1[1]) / h1;
-      else if (i1 == g.lx1) gQ = ((Qs[k] - Qs[k - 1]) / g.dx1[g.lx1]) / h1;
-      else gQ = ((Qs[k + 1] - Qs[k - 1]) / dsum) / h1;
+      const double gQ = one(Qs[k + hi] - Qs[k + lo]);
       const double w2 = s.vs2[(isp - 1) * g.N + c], w3 = s.vs3[(isp - 1) * g.N + c];
       const double geom = (((((w2 * w2) * h3) * dh2dx1 + ((w3 * w3) * h2) * dh3dx1) * nsp) * m) / h1h2h3;
       const double Pp = ((((P[isp - 1] + (nsp * qs(isp)) * (E1f + Epol1)) - ionpress) - gQ) + geom) +

@@ -84,6 +84,37 @@ def test_each_source_loss_entry_point(kind):
         assert max_rel(a, b, f) <= RTOL, f"allparams {f}"
 
 
+@pytest.mark.parametrize("lx1", [4, 59, 124])
+def test_drift_functions_over_their_branches(lx1):
+    """Species drifts from a small fraction to many times the thermal speed, mixed cell by
+    cell: the constant below W = 0.1, the series up to W**2 = 1 and the closed form beyond,
+    with grid rows shorter than, across and as long as a block of 128 cells."""
+    g = ga.cartesian_grid(lx1, 6, 5)
+    st = ga.synthetic_state(g, seed=8, perturb=True)
+    atm = ga.synthetic_atmosphere(g, st, seed=8)
+    rng = np.random.default_rng(lx1)
+    v = st.fluidvars[..., 7:14]
+    v[...] = rng.choice([-1.0, 1.0], v.shape) * 10.0 ** rng.uniform(0.0, 5.0, v.shape)
+    for name in ("v12rhov1", "T2rhoe"):
+        oracle.op(g, st, name)
+    # the pairs' W**2 fall on both sides of each limit
+    T = st.fluidvars[2:-2, 2:-2, 2:-2, 28:35]
+    u = v[2:-2, 2:-2, 2:-2]
+    Teff = (30 * T[..., 0] + 16 * T[..., 1]) / 46
+    W2 = (u[..., 0] - u[..., 1]) ** 2 * (16 * 30 / 46 * 1.66e-27) / (2 * 1.38e-23 * Teff)
+    assert (W2 < 0.01).any() and ((W2 > 0.01) & (W2 < 1)).any() and (W2 > 1).any()
+    tr = transport(g, st, atm)
+    Q = np.zeros((g.lx1, g.lx2, g.lx3, 7), order="F")
+    oracle.op(g, st.copy(), "VNRicht_artvisc", Q=Q)
+    tr.VNRicht_artvisc(st.copy())
+    for which, fields in {"energy": ("Ts", "rhoes"), "momentum": ("vs1", "rhovs1")}.items():
+        a, b = st.copy(), st.copy()
+        oracle.source_loss(g, a, atm, 0.01, which, Q=Q)
+        tr.source_loss(b, which, 0.01)
+        for f in fields:
+            assert max_rel(a, b, f) <= RTOL, f"{which} {f}"
+
+
 def null_cells(g, below):
     alt = np.asarray(g.planes["alt"][0])[2:-2, 2:-2].T          # (lx1, lx2)
     m = np.broadcast_to((alt < below)[:, :, None], (g.lx1, g.lx2, g.lx3))
