@@ -745,15 +745,16 @@ int run_block(double dt) {
   halo_fields({NS, RHOVS1, RHOES});                      // :181
   launch_sweep(g, s, 2, F_ALL, dt, true, st, c.tune);   // :183-185
   const int* nul = c.d_null;
-  launch_rhov12v1_clean_density(g, s, nul, st);          // :186-187, one pass
-  launch_clean_param(g, s, 2, nul, st);                  // :188
-  launch_artvisc(g, s, c.d_Q, st);                       // :191
+  if (!launch_rhov12v1_clean_artvisc(g, s, c.d_Q, nul, st)) {   // :186-191, one pass
+    launch_rhov12v1_clean_density(g, s, nul, st);        // :186-187
+    launch_clean_param(g, s, 2, nul, st);                // :188
+    launch_artvisc(g, s, c.d_Q, st);                     // :191
+  }
   halo_fields({NS, RHOVS1, RHOES, VS2, VS3});            // :199
-  launch_rk2_global_boundary(g, s, st);                  // :200
-  launch_compression_rhoe2T_clean(g, s, c.d_Q, dt, nul, st);   // :203-205, one pass
+  launch_compression_rhoe2T_clean(g, s, c.d_Q, dt, nul, st);   // :200-205, one pass
   if (!hipok(hipGetLastError(), "transport block launch")) return 3;
   c.vsi_current = false;
-  if (!run_energy_diffusion(dt)) return 4;               // :208
+  if (!run_energy_diffusion(dt, false)) return 4;        // :208 (every ghost cell is at 100 K)
   launch_clean_T2rhoe(g, s, nul, st);                    // :209-210, one pass
   return hipok(hipGetLastError(), "transport block launch") ? 0 : 3;
 }

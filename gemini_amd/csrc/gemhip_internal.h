@@ -200,11 +200,14 @@ void launch_artvisc(const DevGrid& g, const DevState& s, double* Q, hipStream_t 
 void launch_rk2_global_boundary(const DevGrid& g, const DevState& s, hipStream_t st);
 void launch_compression(const DevGrid& g, const DevState& s, const double* Q, double dt,
                         hipStream_t st);
-// the same passes fused per cell for the block step: compression + rhoe2T + clean_param(3),
-// and clean_param(3) + T2rhoe
+// the same passes fused for the block step: rhov12v1 + clean_param(1) (+ VNRicht_artvisc where
+// it says so), RK2_global_boundary + compression + rhoe2T + clean_param(3) without rhoes, which
+// clean_param(3) + T2rhoe sets at the end
 void launch_compression_rhoe2T_clean(const DevGrid& g, const DevState& s, const double* Q,
                                      double dt, const int* nul, hipStream_t st);
 void launch_clean_T2rhoe(const DevGrid& g, const DevState& s, const int* nul, hipStream_t st);
+bool launch_rhov12v1_clean_artvisc(const DevGrid& g, const DevState& s, double* Q, const int* nul,
+                                   hipStream_t st);
 void launch_rhov12v1_clean_density(const DevGrid& g, const DevState& s, const int* nul,
                                    hipStream_t st);
 

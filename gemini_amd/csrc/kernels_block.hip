@@ -237,13 +237,77 @@ __global__ void k_rhov12v1_clean_density(DevGrid g, double* ns, const double* rh
   }
 }
 
-// The tail of the compression substep fused per cell (src/libgemini.cpp:203-205):
-// compression of the interior energy density, rhoe2T over every cell, clean_param(3).
-// Ghost cells end at 100 K whatever rhoe2T gives them, and keep their energy density.
-__global__ void k_compression_rhoe2T_clean(DevGrid g, double dt, const double* ns,
-                                           const double* vs1, const double* vs2,
-                                           const double* vs3, const double* Q, double* rhoes,
-                                           double* Ts, const int* nul) {
+// The same without null cells, and VNRicht_artvisc with it (src/libgemini.cpp:186-191;
+// clean_param(2) between them changes nothing then).  A block owns whole columns, so that the
+// viscosity finds its x1 neighbours' velocities in LDS and no cell reads a density that
+// another block has cleaned: cols columns of L1 cells, a thread per cell.  Bound by HBM:
+// 1.29 ms at 512x256x192, 1.04 and 0.73 ms as two passes.
+__global__ __launch_bounds__(1024) void k_rhov12v1_clean_artvisc(DevGrid g, int cols, double* ns,
+                                                                 const double* rhovs1, double* vs1,
+                                                                 double* Q) {
+  extern __shared__ double lv[];
+  const int t = threadIdx.x, nt = blockDim.x;
+  const long ni = (long)g.lx1 * g.lx2 * g.lx3;
+  const long c = (long)blockIdx.x * cols * g.L1 + t;
+  const bool active = t < cols * g.L1 && c < g.N;
+  const int col = t / g.L1, i1 = t - col * g.L1 - 1;
+  const long r = (long)blockIdx.x * cols + col;
+  const int i2 = (int)(r % g.L2) - 1, i3 = (int)(r / g.L2) - 1;
+  const bool in = active && interior(g, i1, i2, i3);
+  double n[LSP - 1], v[LSP - 1];
+  if (active) {
+    double chrgflux = 0.0, sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < LSP - 1; ++i) {
+      n[i] = ns[i * g.N + c];
+      v[i] = rhovs1[i * g.N + c];
+    }
+#pragma unroll
+    for (int i = 0; i < LSP - 1; ++i) {
+      v[i] = v[i] / (ms(i + 1) * fmax_f(n[i], mindensdiv));
+      vs1[i * g.N + c] = v[i];
+      lv[i * nt + t] = v[i];
+      chrgflux = chrgflux + (n[i] * qs(i + 1)) * v[i];
+    }
+#pragma unroll
+    for (int i = 0; i < LSP - 1; ++i) sum = sum + n[i];
+    vs1[(LSP - 1) * g.N + c] = -(((1.0 / fmax_f(sum, mindensdiv)) / qs(LSP)) * chrgflux);
+    double total = 0.0;
+#pragma unroll
+    for (int i = 0; i < LSP - 1; ++i) {
+      n[i] = in ? fmax_f(n[i], mindens) : mindensdiv;
+      ns[i * g.N + c] = n[i];
+      total = total + n[i];
+    }
+    ns[(LSP - 1) * g.N + c] = in ? total : mindensdiv;
+  }
+  __syncthreads();
+  if (!in) return;
+  const long k = (i1 - 1) + (long)g.lx1 * ((i2 - 1) + (long)g.lx2 * (i3 - 1));
+#pragma unroll
+  for (int i = 0; i < LSP - 1; ++i) {
+    const double vl = 0.5 * (lv[i * nt + t - 1] + v[i]);
+    const double vr = 0.5 * (v[i] + lv[i * nt + t + 1]);
+    const double m = fmin_f(vr - vl, 0.0);
+    Q[i * ni + k] = (((n[i] * ms(i + 1)) * 0.25) * (xicon * xicon)) * (m * m);
+  }
+  Q[(LSP - 1) * ni + k] = 0.0;
+}
+
+// The compression substep of the block fused per cell (src/libgemini.cpp:200-205):
+// RK2_global_boundary, compression, rhoe2T, clean_param(3).  Interior cells read the held
+// boundary velocity at its source, so the ghost cells can store it in the same pass (a
+// source is never a target: the ghost layers chain x3, x2, x1 as the reference's three
+// assignments do).  Ghost cells end at 100 K whatever rhoe2T gives them.  The compressed
+// energy density goes into the temperature only: the block ends with T2rhoe over every
+// cell.  Divides by the grid's spacings and by the cell's h1 h2 h3 use reciprocals.
+// Bound by HBM, 52 values a cell: 2.27 ms at 512x256x192 (4.8 TB/s), 3.18 ms with the
+// boundaries as three launches, the energy density stored and four IEEE divides a species.
+template <bool D2, bool D3>
+__global__ __launch_bounds__(TPB) void k_compression_rhoe2T_clean(DevGrid g, double dt, const double* ns,
+                                                                  double* vs1, double* vs2, double* vs3,
+                                                                  const double* Q, const double* rhoes,
+                                                                  double* Ts, const int* nul) {
   const long ni = (long)g.lx1 * g.lx2 * g.lx3;
   const long s2 = g.L1, s3 = (long)g.L1 * g.L2;
   for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < g.N;
@@ -252,6 +316,18 @@ __global__ void k_compression_rhoe2T_clean(DevGrid g, double dt, const double* n
     cell_of(g, c, i1, i2, i3);
     if (!interior(g, i1, i2, i3)) {
       for (int isp = 0; isp < LSP; ++isp) Ts[isp * g.N + c] = 100.0;
+      const long o3 = g.flagper ? 0 : i3 == 0 ? s3 : i3 == g.lx3 + 1 ? -s3 : 0;
+      const long o2 = i2 == 0 ? s2 : i2 == g.lx2 + 1 ? -s2 : 0;
+      const long o1 = i1 == 0 ? 1 : i1 == g.lx1 + 1 ? -1 : 0;
+      const long c23 = c + o2 + o3, c123 = c23 + o1;
+      for (int isp = 0; isp < LSP; ++isp) {
+        const long o = isp * g.N;
+        if (c123 != c) vs1[o + c] = vs1[o + c123];
+        if (c23 != c) {
+          vs2[o + c] = vs2[o + c23];
+          vs3[o + c] = vs3[o + c23];
+        }
+      }
       continue;
     }
     const bool isnull = is_null(g, nul, i1, i2, i3);
@@ -260,23 +336,26 @@ __global__ void k_compression_rhoe2T_clean(DevGrid g, double dt, const double* n
     const double* h2 = g.h2;
     const double* h3 = g.h3;
     const double m1a = h2[c + 1] * h3[c + 1], m1b = h2[c - 1] * h3[c - 1];
-    const double d1 = g.dx1[i1 + 1] + g.dx1[i1];
-    double m2a = 0.0, m2b = 0.0, d2 = 1.0, m3a = 0.0, m3b = 0.0, d3 = 1.0;
-    if (g.lx2 > 1) { m2a = h1[c + s2] * h3[c + s2]; m2b = h1[c - s2] * h3[c - s2]; d2 = g.dx2[i2 + 1] + g.dx2[i2]; }
-    if (g.lx3 > 1) { m3a = h1[c + s3] * h2[c + s3]; m3b = h1[c - s3] * h2[c - s3]; d3 = g.dx3[i3 + 1] + g.dx3[i3]; }
-    const double hc = (h1[c] * h2[c]) * h3[c];
-    for (int isp = 1; isp <= LSP; ++isp) {
+    const double d1 = g.dx1[i1 + 1] + g.dx1[i1], y1 = g.rdx1s[i1];
+    const long u1 = i1 == g.lx1 ? c : c + 1, l1 = i1 == 1 ? c : c - 1;
+    const long u2 = i2 == g.lx2 ? c : c + s2, l2 = i2 == 1 ? c : c - s2;
+    const long u3 = i3 == g.lx3 && !g.flagper ? c : c + s3, l3 = i3 == 1 && !g.flagper ? c : c - s3;
+    double m2a = 0.0, m2b = 0.0, d2 = 1.0, y2 = 1.0, m3a = 0.0, m3b = 0.0, d3 = 1.0, y3 = 1.0;
+    if (D2) { m2a = h1[c + s2] * h3[c + s2]; m2b = h1[c - s2] * h3[c - s2]; d2 = g.dx2[i2 + 1] + g.dx2[i2]; y2 = g.rdx2s[i2]; }
+    if (D3) { m3a = h1[c + s3] * h2[c + s3]; m3b = h1[c - s3] * h2[c - s3]; d3 = g.dx3[i3 + 1] + g.dx3[i3]; y3 = g.rdx3s[i3]; }
+    const double hc = (h1[c] * h2[c]) * h3[c], yc = 1.0 / hc;
+#pragma unroll 1
+    for (int isp = 1; isp <= LSP; ++isp) {       // (unrolled: 222 registers, 2.66 ms)
       const long o = (isp - 1) * g.N;
-      double dv = (m1a * vs1[o + c + 1] - m1b * vs1[o + c - 1]) / d1;
-      if (g.lx2 > 1) dv = dv + (m2a * vs2[o + c + s2] - m2b * vs2[o + c - s2]) / d2;
-      if (g.lx3 > 1) dv = dv + (m3a * vs3[o + c + s3] - m3b * vs3[o + c - s3]) / d3;
-      dv = dv / hc;
+      double dv = div_rcp(m1a * vs1[o + u1] - m1b * vs1[o + l1], d1, y1);
+      if (D2) dv = dv + div_rcp(m2a * vs2[o + u2] - m2b * vs2[o + l2], d2, y2);
+      if (D3) dv = dv + div_rcp(m3a * vs3[o + u3] - m3b * vs3[o + l3], d3, y3);
+      dv = div_rcp(dv, hc, yc);
       const double gm1 = gammas(isp) - 1.0;
       const double q = Q[(isp - 1) * ni + k];
       const double e0 = rhoes[o + c];
       const double half = e0 - ((dt / 2.0) * (e0 * gm1 + q)) * dv;
       const double e = e0 - (dt * (half * gm1 + q)) * dv;
-      rhoes[o + c] = e;
       const double t = fmax_f(((gm1 / kB) * e) / fmax_f(ns[o + c], mindensdiv), 100.0);
       Ts[o + c] = isnull ? 100.0 : fmax_f(t, 100.0);
     }
@@ -388,8 +467,9 @@ void launch_gridrates(const DevGrid& g, const DevState& s, double* work, hipStre
 void launch_compression_rhoe2T_clean(const DevGrid& g, const DevState& s, const double* Q,
                                      double dt, const int* nul, hipStream_t st) {
   timing_begin("compression", st);
-  hipLaunchKernelGGL(k_compression_rhoe2T_clean,
-                     dim3(grid_capped(g.N)), dim3(TPB), 0, st, g,
+  auto kernel = g.lx2 > 1 ? (g.lx3 > 1 ? k_compression_rhoe2T_clean<true, true> : k_compression_rhoe2T_clean<true, false>)
+                          : (g.lx3 > 1 ? k_compression_rhoe2T_clean<false, true> : k_compression_rhoe2T_clean<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(grid_capped(g.N)), dim3(TPB), 0, st, g,
                      dt, s.ns, s.vs1, s.vs2, s.vs3, Q, s.rhoes, s.Ts, nul);
   timing_end("compression", st);
 }
@@ -401,6 +481,20 @@ void launch_rhov12v1_clean_density(const DevGrid& g, const DevState& s, const in
                      dim3(grid_capped(g.N)), dim3(TPB), 0, st, g,
                      s.ns, s.rhovs1, s.vs1, nul);
   timing_end("rhov12v1", st);
+}
+
+// Without null cells, and where a block of threads holds a column; false: nothing launched,
+// the caller takes the separate passes.  Short columns share blocks of about 256 threads.
+bool launch_rhov12v1_clean_artvisc(const DevGrid& g, const DevState& s, double* Q, const int* nul,
+                                   hipStream_t st) {
+  if (nul || g.L1 > 1024) return false;
+  const int cols = g.L1 < TPB ? TPB / g.L1 : 1, threads = (cols * g.L1 + 63) / 64 * 64;
+  const long blocks = ((long)g.L2 * g.L3 + cols - 1) / cols;
+  timing_begin("rhov12v1", st);
+  hipLaunchKernelGGL(k_rhov12v1_clean_artvisc, dim3((unsigned)blocks), dim3(threads),
+                     (LSP - 1) * threads * sizeof(double), st, g, cols, s.ns, s.rhovs1, s.vs1, Q);
+  timing_end("rhov12v1", st);
+  return true;
 }
 
 void launch_clean_T2rhoe(const DevGrid& g, const DevState& s, const int* nul, hipStream_t st) {

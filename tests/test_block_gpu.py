@@ -150,3 +150,29 @@ def test_grid_rates_when_threads_loop_over_cells():
     _, ref_rates = oracle.dt_calc(g, st, 0.9)
     assert np.array_equal(tr.grid_rates(), ref_rates)
     tr.set_residency(0)
+
+
+@pytest.mark.parametrize("grid,size", [
+    ("cart", (4, 5, 3)), ("cart", (60, 7, 6)), ("cart", (252, 3, 2)), ("cart", (253, 3, 2)),
+    ("cart", (1020, 2, 3)), ("cart", (1021, 2, 3)), ("cart", (40, 1, 9)), ("cart", (40, 9, 1)),
+    ("cart", (40, 1, 1)), ("periodic", (28, 5, 8)), ("dipole", (40, 9, 7))])
+def test_block_without_null_cells(grid, size):
+    """The passes that need no null cells: columns of 8 cells (32 to a block) up to the longest
+    that a block holds and one more, each combination of directions, periodic x3."""
+    g = ga.dipole_grid(*size) if grid == "dipole" else ga.cartesian_grid(*size, flagper=grid == "periodic")
+    st = ga.synthetic_state(g, seed=5, perturb=g.lx2 > 1 and g.lx3 > 1)
+    dt = ga.cfl_dt(g, st)
+    tr = Transport(g, st.nn, st.Tn)
+    Q = np.zeros((g.lx1, g.lx2, g.lx3, 7), order="F")
+    with oracle.pow_mode(1):
+        ref, got = st.copy(), st.copy()
+        tr.set_interface_vels(got)
+        tr.set_residency(1)
+        tr.push(got)
+        for _ in range(2):
+            oracle.fluid_adv_block(g, ref, dt, Q=Q)
+            tr.fluid_adv_block(dt)
+        tr.pull(got)
+    assert np.array_equal(got.fluidvars, ref.fluidvars)
+    assert np.array_equal(got.fluidauxvars[..., :14], ref.fluidauxvars[..., :14])
+    tr.close()
