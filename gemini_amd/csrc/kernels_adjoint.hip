@@ -306,21 +306,24 @@ __device__ __forceinline__ double lambda_e_dT(const CellIn<true>& c, double lam_
   return lam_e * (2.5 / T - dden / den);
 }
 
-// scratch slots per (row, column), column-interleaved: slot k of row i of column col at
-// scr[((i-1)*NSA + k)*ncol + col]
+// scratch slots per (row, column): groups of 64 columns, in a group row by row, in a row slot
+// by slot, 64 columns each, so that a lane reaches its row's slots from one address
 enum : int {
-  A0 = 0, A1, A2, AY, AL, AS,      // TR: pivot row, rhs -> U^T solve -> w1, multiplier, swap
-  B0, B1, B2, BY, BL, BS,          // BDF2: the same, BY: rhs -> mu -> U^T solve -> w2
-  X1, X2,                          // TR and BDF2 solutions
+  A0 = 0, A1, A2, AY, AL, AI,      // TR: s1 s2 s3 and rhs -> pivot row, rhs (then BDF2's) -> U^T
+                                   // solve -> w1; multiplier; 1/pivot
+  B0, B1, B2, BY, BL, BI,          // BDF2: the same, BY: dL/dTe after the step -> mu -> U^T solve
+                                   // -> w2 (BL of row 1 is SINGULAR for a column without an adjoint)
+  X1, X2,                          // TR and BDF2 solutions (X2 before: the rhs term in T)
   NSA
 };
+constexpr double SINGULAR = 2.0;   // (a multiplier is at most 1)
 
+// one column of the scratch
 struct Col {
-  double* scr;
-  long ncol;
-  __device__ double& operator()(int i, int k) const {
-    return scr[((long)(i - 1) * NSA + k) * ncol];
-  }
+  double* p;                       // row 1, slot NSA/2 (immediate offsets reach 4 KB either way)
+  __device__ Col(const double* scratch, int N, long col)
+      : p(const_cast<double*>(scratch) + (((col >> 6) * N * NSA + NSA / 2) * 64 + (col & 63))) {}
+  __device__ double& operator()(int i, int k) const { return p[(long)(i - 1) * (NSA * 64) + (k - NSA / 2) * 64]; }
 };
 
 struct AdjArgs {
@@ -333,31 +336,29 @@ struct AdjArgs {
 };
 
 // pivoted elimination step bringing in row (a, b, cc | d) against the pending row
-// (r0, r1 | rb), as dgbtf2 + dgbtrs do it (kernels_diffusion.hip): stores the pivot row,
-// its rhs, the multiplier and the interchange
+// (r0, r1 | rb), as dgbtf2 + dgbtrs do it (kernels_diffusion.hip): stores the pivot row, its
+// reciprocal and rhs and the multiplier.  An interchange shows in the third entry, which is
+// +0 without one (and -0 where an interchange brings a zero).  The zero tests of the band
+// routines only skip work that changes nothing, and are left out.
+template <bool RHS>
 __device__ __forceinline__ bool adj_elim(const Col& q, int j, int s0, double& r0, double& r1,
-                                         double* rb, double a, double b, double cc, double d) {
+                                         double& rb, double a, double b, double cc, double d) {
   const bool swap = fabs(a) > fabs(r0);
-  double p0, p1, p2, pd, o0, o1, o2, od;
-  if (swap) { p0 = a; p1 = b; p2 = cc; pd = d; o0 = r0; o1 = r1; o2 = 0.0; od = rb ? *rb : 0.0; }
-  else { p0 = r0; p1 = r1; p2 = 0.0; pd = rb ? *rb : 0.0; o0 = a; o1 = b; o2 = cc; od = d; }
-  double l = 0.0;
-  const bool sing = p0 == 0.0;
-  if (!sing) {
-    const double rp = 1.0 / p0;
-    l = rp * o0;
-    if (p1 != 0.0) o1 = o1 + l * (-p1);
-    if (p2 != 0.0) o2 = o2 + l * (-p2);
-    if (rb && pd != 0.0) od = od + l * (-pd);
-  }
+  const double p0 = swap ? a : r0, p1 = swap ? b : r1, p2 = swap ? (cc == 0.0 ? -0.0 : cc) : 0.0;
+  const double o0 = swap ? r0 : a, o1 = swap ? r1 : b, o2 = swap ? 0.0 : cc;
+  const double rp = 1.0 / p0, l = rp * o0;
   q(j, s0) = p0; q(j, s0 + 1) = p1; q(j, s0 + 2) = p2;
-  if (rb) q(j, s0 + 3) = pd;
-  q(j, s0 + 4) = l;
-  q(j, s0 + 5) = swap ? 1.0 : 0.0;
-  r0 = o1; r1 = o2;
-  if (rb) *rb = od;
-  return sing;
+  q(j, s0 + 4) = l; q(j, s0 + 5) = rp;
+  r0 = o1 + l * (-p1);
+  r1 = o2 + l * (-p2);
+  if (RHS) {
+    const double pd = swap ? d : rb, od = swap ? rb : d;
+    q(j, s0 + 3) = pd;
+    rb = od + l * (-pd);
+  }
+  return p0 == 0.0;
 }
+__device__ __forceinline__ bool interchanged(double p2) { return __double_as_longlong(p2) != 0; }
 
 // Every pass below walks the rows of a column in order with a loop-carried recurrence.
 // Row data are fetched P rows ahead into a register ring, so the loads of later rows are
@@ -386,249 +387,357 @@ __device__ __forceinline__ void stream_rows(int first, int count, Fetch fetch, B
   }
 }
 
-constexpr int PF = 8;            // ring depth of the light passes
-constexpr int PFI = 2;           // ring depth of the passes that read the cell inputs
+constexpr int PF = 12;           // ring depth of the passes (8: 8 % slower, 16: spills)
 
 struct R4 { double a, b, c, d; };
-struct R5 { double a, b, c, d, e; };
 
-// dtbsv (upper, no transpose) over stored rows s0..s0+2 with rhs slot sy, into slot sx;
-// with mask_lam, also mu(i) = dL/dx(i) through the output floor into slot sy
-__device__ __forceinline__ void adj_backsub(const Col& q, int N, int s0, int sy, int sx,
-                                            const double* lam = nullptr) {
+// dtbsv (upper, no transpose) over stored rows s0..s0+2 with the rhs in AY, into slot sx;
+// with MU, also mu(i) = dL/dx(i) through the output floor into BY
+template <bool MU>
+__device__ __forceinline__ void adj_backsub(const Col& q, int N, int s0, int sx) {
   double x1 = 0.0, x2 = 0.0;                         // x(i+1), x(i+2)
-  auto fetch = [&](int i, R5& r) {
+  struct R { double a, b, c, y, d, e; };
+  stream_rows<PF, -1, R>(N, N, [&](int i, R& r) {
     const int c = clampi(i, 1, N);
-    r.a = q(c, s0); r.b = q(c, s0 + 1); r.c = q(c, s0 + 2); r.d = q(c, sy);
-    r.e = lam ? lam[c] : 0.0;
-  };
-  stream_rows<PF, -1, R5>(N, N, fetch, [&](int i, const R5& r) {
-    double acc = r.d;
-    if (i + 2 <= N && x2 != 0.0) acc = acc - x2 * r.c;
-    if (i + 1 <= N && x1 != 0.0) acc = acc - x1 * r.b;
-    if (acc != 0.0) acc = acc / r.a;
-    q(i, sx) = acc;
-    if (lam) q(i, sy) = acc >= 100.0 ? r.e : 0.0;
+    r.a = q(c, s0); r.b = q(c, s0 + 1); r.c = q(c, s0 + 2); r.y = q(c, s0 + 5); r.d = q(c, AY);
+    if (MU) r.e = q(c, BY);
+  }, [&](int i, const R& r) {
+    const double x = div_rcp((r.d - x2 * r.c) - x1 * r.b, r.a, r.y);
+    q(i, sx) = x;
+    if (MU) q(i, BY) = x >= 100.0 ? r.e : 0.0;
     x2 = x1;
-    x1 = acc;
+    x1 = x;
   });
 }
 
-// M^T w = rhs for a matrix factored by adj_elim into slots s0..s0+5.  The rhs is slot
-// s0+3, or with cw != 0 the interior rows of cw * (slot BY); slot s0+3 ends holding w.
+// M^T w = rhs for a matrix factored by adj_elim into slots s0...  The rhs is slot s0+3, or
+// with CW the interior rows of cw * (slot BY); slot s0+3 ends holding w.
 // U^T z = rhs top-down, then the eliminations transposed bottom-up: z(j) -= l_j z(j+1),
 // then the interchange.
+template <bool CW>
 __device__ __forceinline__ void adj_solveT(const Col& q, int N, int s0, double cw = 0.0) {
   double zm1 = 0.0, zm2 = 0.0;                       // z(i-1), z(i-2)
   double u1m1 = 0.0, u2m1 = 0.0, u2m2 = 0.0;         // U1(i-1), U2(i-1), U2(i-2)
-  const int sr = cw != 0.0 ? BY : s0 + 3;
-  stream_rows<PF, 1, R4>(1, N, [&](int i, R4& r) {
+  struct R { double a, b, c, y, d; };
+  stream_rows<PF, 1, R>(1, N, [&](int i, R& r) {
     const int c = clampi(i, 1, N);
-    r.a = q(c, s0); r.b = q(c, s0 + 1); r.c = q(c, s0 + 2); r.d = q(c, sr);
-  }, [&](int i, const R4& r) {
-    const double rhs = cw == 0.0 ? r.d : (i >= 2 && i <= N - 1 ? cw * r.d : 0.0);
-    const double z = ((rhs - u1m1 * zm1) - u2m2 * zm2) / r.a;
+    r.a = q(c, s0); r.b = q(c, s0 + 1); r.c = q(c, s0 + 2); r.y = q(c, s0 + 5);
+    r.d = q(c, CW ? BY : s0 + 3);
+  }, [&](int i, const R& r) {
+    const double rhs = !CW ? r.d : (i >= 2 && i <= N - 1 ? cw * r.d : 0.0);
+    const double z = div_rcp((rhs - u2m2 * zm2) - u1m1 * zm1, r.a, r.y);
     q(i, s0 + 3) = z;
     zm2 = zm1; zm1 = z;
     u2m2 = u2m1;
     u1m1 = r.b; u2m1 = r.c;
   });
   double carry = q(N, s0 + 3);
-  stream_rows<PF, -1, R4>(N - 1, N - 1, [&](int j, R4& r) {
+  struct T { double z, l, c; };
+  stream_rows<PF, -1, T>(N - 1, N - 1, [&](int j, T& r) {
     const int c = clampi(j, 1, N);
-    r.a = q(c, s0 + 3); r.b = q(c, s0 + 4); r.c = q(c, s0 + 5);
-  }, [&](int j, const R4& r) {
-    const double a = r.a - r.b * carry;
-    if (r.c != 0.0) {
-      q(j + 1, s0 + 3) = a;
-    } else {
-      q(j + 1, s0 + 3) = carry;
-      carry = a;
-    }
+    r.z = q(c, s0 + 3); r.l = q(c, s0 + 4); r.c = q(c, s0 + 2);
+  }, [&](int j, const T& r) {
+    const double a = r.z - r.l * carry;
+    const bool swap = interchanged(r.c);
+    q(j + 1, s0 + 3) = swap ? a : carry;
+    carry = swap ? carry : a;
   });
   q(1, s0 + 3) = carry;
 }
 
-// one lane per electron column (x2, x3)
-__global__ __launch_bounds__(64) void k_adj_trbdf2(DevGrid g, DevState s, AdjArgs A,
-                                                    double* scratch) {
+// Electron inputs of row r of column (i2, i3)
+__device__ __forceinline__ CellIn<true> adj_cell(const DevGrid& g, const DevState& s, const AdjArgs& A,
+                                                 int r, int i2, int i3, long col) {
+  const long c = gix(g, r, i2, i3), k = (long)g.lx1 * col + r - 1, ni = (long)g.lx1 * g.lx2 * g.lx3;
+  CellIn<true> v;
+  v.T = A.TD[c];
+  v.n = A.NE1[c];
+  v.h1 = g.h1[c]; v.h2 = g.h2[c]; v.h3 = g.h3[c];
+  v.n1 = s.nn[k]; v.n2 = s.nn[ni + k]; v.n3 = s.nn[2 * ni + k];
+  v.J = s.J1[c];
+  v.kap = s.kappa ? s.kappa[col] : 1.0;
+  return v;
+}
+
+// row i's entries from the coefficients C, B of the row and D of it and its neighbours
+struct RowTerms { double s1, s2, s3; };
+__device__ __forceinline__ RowTerms adj_row(const DevGrid& g, int i, double C, double B, double Dm,
+                                            double Dc, double Dp) {
+  const double* dx1i = g.dx1i - 1;
+  const double Dh = 0.5 * (Dm + Dc), Dh1 = 0.5 * (Dc + Dp);
+  RowTerms t;
+  t.s1 = ((C * Dh) / dx1i[i]) / g.dx1[i];
+  t.s3 = ((C * Dh1) / dx1i[i]) / g.dx1[i + 1];
+  t.s2 = B / (g.dx1[i + 1] + g.dx1[i]);
+  return t;
+}
+
+// The adjoint of TRBDF2 in three kernels.  Its recurrences run one lane per column, and a
+// grid of a few thousand columns gives a wave to one CU in five: everything that is no
+// recurrence is done by cell, in tiles that read the fields along x1 and the scratch along
+// the columns (LDS turns one into the other).  192x64x48: 228 us, of which some 160 are the
+// recurrences; one kernel with a lane per column took 728, most of it in two passes that read
+// the fields with the stride of a column.
+constexpr int TR_ROWS = 32, TC = 16, LDT = TR_ROWS + 1;      // a tile's rows and columns in LDS
+
+// s1, s2, s3 of the rows 2..N-1 and the right-hand sides, into the slots A0..AY, B0..B2 and X2;
+// dL/dTe of all rows into BY
+__global__ __launch_bounds__(TPB) void k_adj_terms(DevGrid g, DevState s, AdjArgs A, double* scratch) {
+  __shared__ double lT[TC * LDT], lC[TC * LDT], lB[TC * LDT], lD[TC * LDT],
+      lL[TC * LDT];
   const long ncol = (long)g.lx2 * g.lx3;
-  const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= ncol) return;
+  const int N = g.lx1;
+  const unsigned row_tiles = (N - 2 + TR_ROWS - 3) / (TR_ROWS - 2);
+  const int first = (int)(blockIdx.x % row_tiles) * (TR_ROWS - 2) + 1;  // the tile's rows first..
+  const long col0 = (long)(blockIdx.x / row_tiles) * TC;
+  const double gm1kB = (gammas(LSP) - 1.0) / kB;
+  for (int u = threadIdx.x; u < TR_ROWS * TC; u += TPB) {
+    const int rr = u % TR_ROWS, cc = u / TR_ROWS, r = first + rr;
+    const long col = col0 + cc;
+    if (r <= N && col < ncol) {
+      const int i2 = (int)(col % g.lx2) + 1, i3 = (int)(col / g.lx2) + 1;
+      const CellIn<true> c = adj_cell(g, s, A, r, i2, i3, col);
+      double C, B, D;
+      cell_coeffs<true, true>(c, LSP, gm1kB, C, B, D);
+      const int o = cc * LDT + rr;
+      lT[o] = c.T; lC[o] = C; lB[o] = B; lD[o] = D;
+      lL[o] = A.lam[gix(g, r, i2, i3)];
+    }
+  }
+  __syncthreads();
+  const double dt2 = A.dt / 2.0, dt3 = A.dt / 3.0, c13 = 1.0 / 3.0;
+  for (int u = threadIdx.x; u < TR_ROWS * TC; u += TPB) {
+    const int cc = u % TC, rr = u / TC, i = first + rr;
+    const long col = col0 + cc;
+    if (i > N || col >= ncol) continue;
+    const int o = cc * LDT + rr;
+    const Col q(scratch, N, col);
+    if (i == 1 || i == N) q(i, BY) = lL[o];
+    if (rr < 1 || rr > TR_ROWS - 2 || i > N - 1) continue;
+    const RowTerms t = adj_row(g, i, lC[o], lB[o], lD[o - 1], lD[o], lD[o + 1]);
+    const double t1 = t.s1 / 2.0, t2 = t.s2 / 2.0, t3 = t.s3 / 2.0;
+    const double a = -t1 + t2, c = -t3 - t2;
+    q(i, A0) = t.s1; q(i, A1) = t.s2; q(i, A2) = t.s3;
+    q(i, B0) = t.s1; q(i, B1) = t.s2; q(i, B2) = t.s3;
+    q(i, AY) = ((lT[o] / dt2 - a * lT[o - 1]) - (t3 + t1) * lT[o]) - c * lT[o + 1];
+    q(i, X2) = -((c13 * lT[o]) / dt3);
+    q(i, BY) = lL[o];
+  }
+}
+
+// The two solves and their transposes: a block of two waves to 64 columns, a lane per column
+// in each.  The waves factor the TR and the BDF2 matrix side by side; the first goes on
+// through the passes that depend on each other.  Bound by its chains: rows times eight passes
+// times a row's dependent operations and their issue by a lone wave, some 250 cycles; so
+// pivots keep their reciprocals (div_rcp is exact), an interchange is read off the pivot row,
+// and a row's slots lie within the immediate offsets of one address (246 us without the three).
+__global__ __launch_bounds__(128) void k_adj_trbdf2(DevGrid g, DevState s, AdjArgs A,
+                                                     double* scratch) {
+  __shared__ int bad[64];
+  const long ncol = (long)g.lx2 * g.lx3;
+  const int lane = threadIdx.x & 63;
+  const bool second = threadIdx.x >= 64;
+  const long col = (long)blockIdx.x * 64 + lane;
+  const bool active = col < ncol;
   const int N = g.lx1;
   const int i2 = (int)(col % g.lx2) + 1, i3 = (int)(col / g.lx2) + 1;
-  const long cb = gix(g, 0, i2, i3), kb = (long)N * col;
-  const long ni = (long)g.lx1 * g.lx2 * g.lx3;
-  Col q{scratch + col, ncol};
-  DevState se = s;                                   // the diffusion's inputs from the tape
-  se.Ts = const_cast<double*>(A.TD);
-  se.ns = const_cast<double*>(A.NE1);
+  const long kb = (long)N * col;
+  const Col q(scratch, N, active ? col : ncol - 1);
   const double* dx1 = g.dx1;
-  const double* dx1i = g.dx1i - 1;
-  const double gm1kB = (gammas(LSP) - 1.0) / kB;
   const double dt2 = A.dt / 2.0, K1 = 1.0 / dt2;
   const double dt3 = A.dt / 3.0, K2 = 1.0 / dt3;
-  const double c13 = 1.0 / 3.0, c43 = 4.0 / 3.0;
-  const double kap = s.kappa ? s.kappa[col] : 1.0;
-  const bool flux = s.qtop != nullptr;
-
-  // per-row inputs: T, coefficients C, B, D, conductivity without kappa; in pass I also
-  // both solutions and both adjoint solutions
-  struct Row { double T, C, B, D, lam_e, h1, h23, x1, x2, w1, w2; CellIn<true> in; };
-  auto fetch_in = [&](int r, CellIn<true>& c) {
-    cell_load<true, true>(g, se, 0, cb, kb, ni, clampi(r, 1, N), c,
-                          hcol_index(g, (int)col, clampi(r, 1, N)), (int)col);
-  };
-  auto make_row = [&](const CellIn<true>& c, Row& w) {
-    w.in = c;
-    w.in.kap = kap;
-    w.T = c.T;
-    w.lam_e = cell_lambda<true, false>(w.in, LSP);
-    cell_coeffs<true, true>(w.in, LSP, gm1kB, w.C, w.B, w.D);
-    w.h1 = c.h1;
-    w.h23 = c.h2 * c.h3;
-  };
-  double Tmin, Tmax;
-  {
+  const double c43 = 4.0 / 3.0;
+  double Tmin = 0.0, Tmax = 0.0, aN = 0.0, bN = 1.0;
+  bool sing = false;
+  if (active) {
     const double Tn1 = s.Tn[kb], TnN = s.Tn[kb + N - 1];
     if (g.gridflag == 0) { Tmin = Tn1; Tmax = TnN; }
     else if (g.gridflag == 1) { Tmax = TnN; Tmin = A.Teinf; }
     else { Tmin = Tn1; Tmax = A.Teinf; }
+    if (s.qtop) {
+      const CellIn<true> c = adj_cell(g, s, A, N, i2, i3, col);
+      aN = -1.0 / dx1[N];
+      bN = 1.0 / dx1[N];
+      Tmax = (s.qtop[col] * c.h1) / (cell_lambda<true, false>(c, LSP) * c.kap);
+    }
+    // pass A (top-down): the factorisation, the TR right-hand side eliminated alongside (rows
+    // read ahead of the pivot rows that replace them)
+    double e0 = 1.0, e1 = 0.0, eb = Tmin;            // pending row (row 1: identity)
+    if (!second) {
+      stream_rows<PF, 1, R4>(2, N - 2, [&](int i, R4& r) {
+        const int c = clampi(i, 1, N);
+        r.a = q(c, A0); r.b = q(c, A1); r.c = q(c, A2); r.d = q(c, AY);
+      }, [&](int i, const R4& r) {
+        const double t1 = r.a / 2.0, t2 = r.b / 2.0, t3 = r.c / 2.0;
+        sing |= adj_elim<true>(q, i - 1, A0, e0, e1, eb, -t1 + t2, (K1 + t3) + t1, -t3 - t2, r.d);
+      });
+      sing |= adj_elim<true>(q, N - 1, A0, e0, e1, eb, aN, bN, 0.0, Tmax);   // boundary row N
+      q(N, A0) = e0; q(N, A1) = 0.0; q(N, A2) = 0.0; q(N, AY) = eb; q(N, AI) = 1.0 / e0;
+    } else {
+      stream_rows<PF, 1, R4>(2, N - 2, [&](int i, R4& r) {
+        const int c = clampi(i, 1, N);
+        r.a = q(c, B0); r.b = q(c, B1); r.c = q(c, B2);
+      }, [&](int i, const R4& r) {
+        sing |= adj_elim<false>(q, i - 1, B0, e0, e1, eb, -r.a + r.b, (K2 + r.c) + r.a, -r.c - r.b, 0.0);
+      });
+      sing |= adj_elim<false>(q, N - 1, B0, e0, e1, eb, aN, bN, 0.0, 0.0);
+      q(N, B0) = e0; q(N, B1) = 0.0; q(N, B2) = 0.0; q(N, BI) = 1.0 / e0;
+    }
+    sing |= e0 == 0.0;
   }
-  double aN = 0.0, bN = 1.0, lamN = 0.0, h1N = 0.0;
-  if (flux) {
-    CellIn<true> c;
-    Row top;
-    fetch_in(N, c);
-    make_row(c, top);
-    lamN = top.lam_e * kap;
-    h1N = top.h1;
-    aN = -1.0 / dx1[N];
-    bN = 1.0 / dx1[N];
-    Tmax = (s.qtop[col] * h1N) / lamN;
-  }
-  auto coeffs = [&](int i, const Row& rm, const Row& rc, const Row& rp, double& s1, double& s2,
-                    double& s3) {
-    const double Dh = 0.5 * (rm.D + rc.D), Dh1 = 0.5 * (rc.D + rp.D);
-    s1 = ((rc.C * Dh) / dx1i[i]) / dx1[i];
-    s3 = ((rc.C * Dh1) / dx1i[i]) / dx1[i + 1];
-    s2 = rc.B / (dx1[i + 1] + dx1[i]);
-  };
-
-  // pass A (top-down): both factorisations, the TR right-hand side eliminated alongside;
-  // row r's arrival completes row r-1
-  bool sing = false;
-  double e0 = 1.0, e1 = 0.0, eb = Tmin;              // TR pending row (row 1: identity)
-  double f0 = 1.0, f1 = 0.0;                         // BDF2 pending row
-  Row rm, rc, rp;
-  stream_rows<PFI, 1, CellIn<true>>(1, N, fetch_in, [&](int r, const CellIn<true>& c) {
-    rm = rc; rc = rp;
-    make_row(c, rp);
-    if (r < 3) return;
-    const int i = r - 1;
-    double s1, s2, s3;
-    coeffs(i, rm, rc, rp, s1, s2, s3);
-    const double t1 = s1 / 2.0, t2 = s2 / 2.0, t3 = s3 / 2.0;
-    const double a = -t1 + t2, b = (K1 + t3) + t1, cc = -t3 - t2;
-    const double d = ((rc.T / dt2 - a * rm.T) - (t3 + t1) * rc.T) - cc * rp.T;
-    sing |= adj_elim(q, i - 1, A0, e0, e1, &eb, a, b, cc, d);
-    sing |= adj_elim(q, i - 1, B0, f0, f1, nullptr, -s1 + s2, (K2 + s3) + s1, -s3 - s2, 0.0);
-  });
-  sing |= adj_elim(q, N - 1, A0, e0, e1, &eb, aN, bN, 0.0, Tmax);   // boundary row N
-  sing |= adj_elim(q, N - 1, B0, f0, f1, nullptr, aN, bN, 0.0, 0.0);
-  q(N, A0) = e0; q(N, A1) = 0.0; q(N, A2) = 0.0; q(N, AY) = eb;
-  q(N, B0) = f0; q(N, B1) = 0.0; q(N, B2) = 0.0;
-  sing |= e0 == 0.0 || f0 == 0.0;
-  if (sing) {                                        // no adjoint of a singular solve
-    for (int i = 1; i <= N; ++i) A.lam[cb + i] = __builtin_nan("");
+  if (second) bad[lane] = sing;
+  __syncthreads();
+  if (second || !active) return;
+  if (sing || bad[lane]) {                           // no adjoint of a singular solve
+    q(1, BL) = SINGULAR;
     return;
   }
-
   // pass B: TR solution
-  adj_backsub(q, N, A0, AY, X1);
+  adj_backsub<false>(q, N, A0, X1);
   // pass C: BDF2 right-hand side through the stored eliminations (row 1: Tmin, row N: Tmax)
+  // into AY
   {
     double rb = Tmin;
     stream_rows<PF, 1, R4>(1, N - 1, [&](int j, R4& r) {
       const int c = clampi(j, 1, N - 1);
-      r.a = A.TD[cb + c + 1]; r.b = q(c + 1, X1); r.c = q(c, BS); r.d = q(c, BL);
+      r.a = q(c + 1, X2); r.b = q(c + 1, X1); r.c = q(c, B2); r.d = q(c, BL);
     }, [&](int j, const R4& r) {
-      const double d = j + 1 >= N ? Tmax : -((c13 * r.a) / dt3) + (c43 * r.b) / dt3;
-      const bool swap = r.c != 0.0;
-      const double pd = swap ? d : rb;
-      double od = swap ? rb : d;
-      if (pd != 0.0) od = od + r.d * (-pd);
-      q(j, BY) = pd;
-      rb = od;
+      const double d = j + 1 >= N ? Tmax : r.a + div_rcp(c43 * r.b, dt3, K2);
+      const bool swap = interchanged(r.c);
+      const double pd = swap ? d : rb, od = swap ? rb : d;
+      q(j, AY) = pd;
+      rb = od + r.d * (-pd);
     });
-    q(N, BY) = rb;
+    q(N, AY) = rb;
   }
   // pass D: BDF2 solution, and mu = dL/dx2 through the output floor into BY
-  adj_backsub(q, N, B0, BY, X2, A.lam + cb);
+  adj_backsub<true>(q, N, B0, X2);
   // passes E-F: w2
-  adj_solveT(q, N, B0);
+  adj_solveT<false>(q, N, B0);
   // passes G-H: w1 from dL/dx1 = (4/3)/(dt/3) w2 on the interior rows
-  adj_solveT(q, N, A0, c43 / dt3);
+  adj_solveT<true>(q, N, A0, c43 / dt3);
+}
 
-  // pass I (top-down): chain w1, w2 through the matrix and rhs entries of rows 2..N-1
-  //   dL/dM1(i,k) = -w1(i) (x1(k) + T(k))   (M1 x1 = (2/(dt/2) - M1) T on those rows)
-  //   dL/dM2(i,k) = -w2(i) x2(k)
-  // to s1 = C Dh(i)/dx1i/dx1(i), s3 = C Dh(i+1)/dx1i/dx1(i+1) (TR uses s/2), then Dh, D,
-  // lambda = kappa lambda_e(T), and the direct T terms of both right-hand sides.
-  double gk = 0.0, gqc = 0.0;
-  double gDh_p = 0.0, gDh_c = 0.0, gDh_n = 0.0;     // dL/dDh(i-1), (i), (i+1) so far
-  double gT_m = 0.0, gT_c = 0.0, gT_n = 0.0;         // dL/dT(i-1), (i), (i+1) so far
-  // row j complete: D(j) = lambda(j) h2 h3 / h1 enters Dh(j) and Dh(j+1)
-  auto finish = [&](int j, const Row& w, double gDh_j, double gDh_j1, double gT_j) {
-    const double gD = 0.5 * (gDh_j + gDh_j1);
-    double glam = gD * (w.h23 / w.h1);
-    if (flux && j == N) {                            // row N rhs: q h1(N) / lambda(N)
-      const double gg = w.w1 + w.w2;
-      glam += -gg * (Tmax / lamN);
-      gqc += gg * (h1N / lamN);
+// Chain w1, w2 through the matrix and rhs entries of rows 2..N-1
+//   dL/dM1(i,k) = -w1(i) (x1(k) + T(k))   (M1 x1 = (2/(dt/2) - M1) T on those rows)
+//   dL/dM2(i,k) = -w2(i) x2(k)
+// to s1 = C Dh(i)/dx1i/dx1(i), s3 = C Dh(i+1)/dx1i/dx1(i+1) (TR uses s/2), then Dh, D,
+// lambda = kappa lambda_e(T), and the direct T terms of both right-hand sides.  A block walks
+// the rows of TC columns in tiles with two rows more on each side, and sums a column's
+// dL/dkappa in row order.
+__global__ __launch_bounds__(TPB) void k_adj_chain(DevGrid g, DevState s, AdjArgs A, const double* scratch) {
+  // T C B D x1 x2 w1 w2; then u v tm tc tn in place of x1 .. w2 and B, the kappa terms in x1
+  __shared__ double l[8][TC * LDT];
+  constexpr int CELLS = TR_ROWS * TC / TPB;
+  const long ncol = (long)g.lx2 * g.lx3;
+  const long col0 = (long)blockIdx.x * TC;
+  const int N = g.lx1;
+  const double gm1kB = (gammas(LSP) - 1.0) / kB;
+  const double dt2 = A.dt / 2.0, K1 = 1.0 / dt2, dt3 = A.dt / 3.0, c13 = 1.0 / 3.0;
+  const double* dx1i = g.dx1i - 1;
+  double gk = 0.0;
+  for (int first = -1; first + 2 <= N; first += TR_ROWS - 4) {          // tile rows first..first+31
+    CellIn<true> in[CELLS];
+    double lam_e[CELLS];
+#pragma unroll
+    for (int v = 0; v < CELLS; ++v) {
+      const int u = threadIdx.x + v * TPB, rr = u % TR_ROWS, cc = u / TR_ROWS, r = first + rr;
+      const long col = col0 + cc;
+      lam_e[v] = 0.0;
+      if (r < 1 || r > N || col >= ncol) continue;
+      in[v] = adj_cell(g, s, A, r, (int)(col % g.lx2) + 1, (int)(col / g.lx2) + 1, col);
+      const int o = cc * LDT + rr;
+      lam_e[v] = cell_lambda<true, false>(in[v], LSP);
+      l[0][o] = in[v].T;
+      cell_coeffs<true, true>(in[v], LSP, gm1kB, l[1][o], l[2][o], l[3][o]);
     }
-    gk += glam * w.lam_e;
-    A.lam[cb + j] = gT_j + glam * (kap * lambda_e_dT(w.in, w.lam_e));
-  };
-  struct RawI { CellIn<true> in; double x1, x2, w1, w2; };
-  stream_rows<PFI, 1, RawI>(1, N, [&](int r, RawI& v) {
-    const int c = clampi(r, 1, N);
-    fetch_in(c, v.in);
-    v.x1 = q(c, X1); v.x2 = q(c, X2); v.w1 = q(c, AY); v.w2 = q(c, BY);
-  }, [&](int r, const RawI& v) {
-    rm = rc; rc = rp;
-    make_row(v.in, rp);
-    rp.x1 = v.x1; rp.x2 = v.x2; rp.w1 = v.w1; rp.w2 = v.w2;
-    if (r < 3) return;
-    const int i = r - 1;
-    double s1, s2, s3;
-    coeffs(i, rm, rc, rp, s1, s2, s3);
-    const double t1 = s1 / 2.0, t2 = s2 / 2.0, t3 = s3 / 2.0;
-    const double a = -t1 + t2, cc = -t3 - t2;
-    const double w1 = rc.w1, w2 = rc.w2;
-    const double G1a = -w1 * (rm.x1 + rm.T), G1b = -w1 * (rc.x1 + rc.T), G1c = -w1 * (rp.x1 + rp.T);
-    const double G2a = -w2 * rm.x2, G2b = -w2 * rc.x2, G2c = -w2 * rp.x2;
-    const double gs1 = 0.5 * (G1b - G1a) + (G2b - G2a);
-    const double gs3 = 0.5 * (G1b - G1c) + (G2b - G2c);
-    gDh_c += gs1 * ((rc.C / dx1i[i]) / dx1[i]);
-    gDh_n += gs3 * ((rc.C / dx1i[i]) / dx1[i + 1]);
-    gT_m += -w1 * a;                                  // row i: -a T(i-1)
-    gT_c += w1 * (K1 - (t3 + t1)) - (c13 / dt3) * w2;
-    gT_n += -w1 * cc;                                 // row i: -c T(i+1)
-    finish(i - 1, rm, gDh_p, gDh_c, gT_m);
-    gDh_p = gDh_c; gDh_c = gDh_n; gDh_n = 0.0;
-    gT_m = gT_c; gT_c = gT_n; gT_n = 0.0;
-  });
-  finish(N - 1, rc, gDh_p, gDh_c, gT_m);
-  finish(N, rp, gDh_c, 0.0, gT_c);
-  if (A.gk) A.gk[col] += gk;
-  if (A.gq) A.gq[col] += gqc;
+#pragma unroll
+    for (int v = 0; v < CELLS; ++v) {
+      const int u = threadIdx.x + v * TPB, cc = u % TC, rr = u / TC, r = first + rr;
+      const long col = col0 + cc;
+      if (r < 1 || r > N || col >= ncol) continue;
+      const Col q(scratch, N, col);
+      const int o = cc * LDT + rr;
+      l[4][o] = q(r, X1); l[5][o] = q(r, X2); l[6][o] = q(r, AY); l[7][o] = q(r, BY);
+    }
+    __syncthreads();
+    double uu[CELLS], vv[CELLS], tm[CELLS], tc[CELLS], tn[CELLS];
+#pragma unroll
+    for (int v = 0; v < CELLS; ++v) {
+      const int t = threadIdx.x + v * TPB, rr = t % TR_ROWS, cc = t / TR_ROWS, i = first + rr;
+      uu[v] = vv[v] = tm[v] = tc[v] = tn[v] = 0.0;
+      if (rr < 1 || rr > TR_ROWS - 2 || i < 2 || i > N - 1 || col0 + cc >= ncol) continue;
+      const int o = cc * LDT + rr;
+      const double *T = l[0] + o, *x1 = l[4] + o, *x2 = l[5] + o, *D = l[3] + o;
+      const double C = l[1][o], w1 = l[6][o], w2 = l[7][o];
+      const RowTerms s_ = adj_row(g, i, C, l[2][o], D[-1], D[0], D[1]);
+      const double t1 = s_.s1 / 2.0, t2 = s_.s2 / 2.0, t3 = s_.s3 / 2.0;
+      const double a = -t1 + t2, c = -t3 - t2;
+      const double G1a = -w1 * (x1[-1] + T[-1]), G1b = -w1 * (x1[0] + T[0]), G1c = -w1 * (x1[1] + T[1]);
+      const double G2a = -w2 * x2[-1], G2b = -w2 * x2[0], G2c = -w2 * x2[1];
+      const double gs1 = 0.5 * (G1b - G1a) + (G2b - G2a);
+      const double gs3 = 0.5 * (G1b - G1c) + (G2b - G2c);
+      uu[v] = gs1 * ((C / dx1i[i]) / g.dx1[i]);        // to Dh(i)
+      vv[v] = gs3 * ((C / dx1i[i]) / g.dx1[i + 1]);    // to Dh(i+1)
+      tm[v] = -w1 * a;                                 // row i: -a T(i-1)
+      tc[v] = w1 * (K1 - (t3 + t1)) - (c13 / dt3) * w2;
+      tn[v] = -w1 * c;                                 // row i: -c T(i+1)
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < CELLS; ++v) {
+      const int t = threadIdx.x + v * TPB, o = (t / TR_ROWS) * LDT + t % TR_ROWS;
+      l[4][o] = uu[v]; l[5][o] = vv[v]; l[6][o] = tm[v]; l[7][o] = tn[v];
+    }
+    __syncthreads();
+    double kterm[CELLS];
+#pragma unroll
+    for (int v = 0; v < CELLS; ++v) {
+      const int t = threadIdx.x + v * TPB, rr = t % TR_ROWS, cc = t / TR_ROWS, j = first + rr;
+      const long col = col0 + cc;
+      kterm[v] = 0.0;
+      if (rr < 2 || rr > TR_ROWS - 3 || j < 1 || j > N || col >= ncol) continue;
+      const int o = cc * LDT + rr;
+      double* lam = A.lam + gix(g, j, (int)(col % g.lx2) + 1, (int)(col / g.lx2) + 1);
+      const Col q(scratch, N, col);
+      if (q(1, BL) == SINGULAR) {
+        *lam = __builtin_nan("");
+        continue;
+      }
+      // dL/dDh(j) and (j+1); D(j) = lambda(j) h2 h3 / h1 enters both
+      const double gDh = l[5][o - 1] + uu[v], gDh1 = vv[v] + l[4][o + 1];
+      const double gT = (l[7][o - 1] + tc[v]) + l[6][o + 1];
+      double glam = (0.5 * (gDh + gDh1)) * ((in[v].h2 * in[v].h3) / in[v].h1);
+      if (s.qtop && j == N) {                          // row N rhs: q h1(N) / lambda(N)
+        const double gg = q(N, AY) + q(N, BY);
+        const double lamN = lam_e[v] * in[v].kap;
+        glam += -gg * (((s.qtop[col] * in[v].h1) / lamN) / lamN);
+        if (A.gq) A.gq[col] += gg * (in[v].h1 / lamN);
+      }
+      kterm[v] = glam * lam_e[v];
+      *lam = gT + glam * (in[v].kap * lambda_e_dT(in[v], lam_e[v]));
+    }
+    // (B is not read any more; rows of other tiles and of singular columns hold 0)
+#pragma unroll
+    for (int v = 0; v < CELLS; ++v) {
+      const int t = threadIdx.x + v * TPB;
+      l[2][(t / TR_ROWS) * LDT + t % TR_ROWS] = kterm[v];
+    }
+    __syncthreads();
+    if (threadIdx.x < TC) {
+#pragma unroll
+      for (int rr = 2; rr <= TR_ROWS - 3; ++rr) gk += l[2][threadIdx.x * LDT + rr];
+    }
+    __syncthreads();
+  }
+  const long col = col0 + threadIdx.x;
+  if (threadIdx.x < TC && col < ncol && A.gk && Col(scratch, N, col)(1, BL) != SINGULAR) A.gk[col] += gk;
 }
 
 }  // namespace
 
 size_t adjoint_scratch_bytes(const DevGrid& g) {
-  return (size_t)NSA * g.lx1 * g.lx2 * g.lx3 * sizeof(double);
+  return (size_t)NSA * g.lx1 * (((long)g.lx2 * g.lx3 + 63) / 64 * 64) * sizeof(double);
 }
 
 void launch_tape_vels(const DevGrid& g, const DevState& s, double* v1, double* v2, double* v3,
@@ -647,8 +756,12 @@ void launch_adjoint_step(const DevGrid& g, const DevState& s, const AdjTape& t, 
   const dim3 cells(grid_for(g.N)), blk(TPB);
   AdjArgs A{t.TD, t.NE1, lam, gk, gq, dt, Teinf};
   timing_begin("adj_trbdf2", st);
-  hipLaunchKernelGGL(k_adj_trbdf2, dim3((unsigned)((ncol + 63) / 64)), dim3(64), 0, st, g, s, A,
+  const unsigned tiles = (unsigned)((ncol + TC - 1) / TC);
+  const unsigned row_tiles = (g.lx1 - 2 + TR_ROWS - 3) / (TR_ROWS - 2);     // (lx1 >= 4)
+  hipLaunchKernelGGL(k_adj_terms, dim3(row_tiles * tiles), dim3(TPB), 0, st, g, s, A, scratch);
+  hipLaunchKernelGGL(k_adj_trbdf2, dim3((unsigned)((ncol + 63) / 64)), dim3(128), 0, st, g, s, A,
                      scratch);
+  hipLaunchKernelGGL(k_adj_chain, dim3(tiles), dim3(TPB), 0, st, g, s, A, scratch);
   timing_end("adj_trbdf2", st);
   timing_begin("adj_advection", st);
   hipLaunchKernelGGL(k_adj_rhoe2T, cells, blk, 0, st, g, lam, t.TD, t.NE1);

@@ -126,6 +126,35 @@ def test_adjoint_matches_numpy_adjoint(kind):
         run.close()
 
 
+@pytest.mark.parametrize("kind,size", [
+    ("cart", (4, 3, 2)), ("cart", (30, 5, 3)), ("cart", (31, 4, 4)), ("cart", (32, 17, 1)), ("dipole", (33, 9, 7)),
+    ("cart", (57, 13, 5)), ("dipole", (62, 7, 3)), ("cart", (64, 5, 13))])
+def test_adjoint_at_tile_edges(kind, size):
+    """Columns of one to three row tiles with none or one row over, numbers of columns around
+    the 16 of a tile and the 64 of a wave, a grid whose columns end without a heat flux."""
+    g = ga.dipole_grid(*size) if kind == "dipole" else ga.cartesian_grid(*size)
+    st = ga.synthetic_state(g, seed=3, perturb=g.lx3 > 1)
+    dt = min(ga.cfl_dt(g, st), 0.5)
+    rng = np.random.default_rng(3)
+    kappa = 1.0 + 0.2 * rng.uniform(-1.0, 1.0, (g.lx2, g.lx3))
+    qtop = 1e-5 * rng.uniform(0.0, 1.0, (g.lx2, g.lx3)) if g.gridflag == 2 else None
+    w = rng.standard_normal(g.padded)
+    gk_np, gq_np, lam_np, _ = A.gradient(g, st, dt, 2, kappa, qtop, w)
+    run = TransportRun(g, st, dt, 2, every=1)
+    try:
+        run.forward(col_tensor(kappa), col_tensor(qtop))
+        gk, gq = run.backward(torch.tensor(np.asfortranarray(w).ravel(order="F"), device=DEV))
+        gk = gk.cpu().numpy().reshape(g.lx3, g.lx2).T
+        assert np.max(np.abs(gk - gk_np)) <= 1e-9 * np.max(np.abs(gk_np))
+        if qtop is not None:
+            gq = gq.cpu().numpy().reshape(g.lx3, g.lx2).T
+            assert np.max(np.abs(gq - gq_np)) <= 1e-9 * np.max(np.abs(gq_np))
+        lam = run.grad_Te0.cpu().numpy().reshape(g.padded, order="F")
+        assert np.max(np.abs(lam - lam_np)) <= 1e-9 * np.max(np.abs(lam_np))
+    finally:
+        run.close()
+
+
 def test_checkpoint_spacing_does_not_change_the_gradient():
     g, st, dt, kappa, qtop, rng = case("cart", seed=5)
     w = torch.tensor(rng.standard_normal(int(np.prod(g.padded))), device=DEV)
