@@ -57,8 +57,8 @@ struct Coef {
 // 8-byte slots per row and species, each written and read (a pivot row, its right-hand
 // side and a multiplier for each solve); the terms, the temperature and the block states
 // take 3.4 slots for an ion and 4.4 for the electrons.  With the ions' shared metric factors
-// and the cheaper x**2.5 and divisions: 512x256x192 7.91 -> 5.88 ms, 255x113x67 0.87 -> 0.62,
-// 301x127x75 1.19 -> 0.83 (backward Euler 256x128x96 0.66 -> 0.50), 128x64x1 0.225 -> 0.209.
+// the cheaper x**2.5 and divisions, and no tests for zero entries: 512x256x192 7.91 -> 5.84 ms,
+// 255x113x67 0.87 -> 0.57, 301x127x75 1.19 -> 0.79 (backward Euler 256x128x96 0.66 -> 0.485).
 //
 // Rows are kept lane-interleaved in HBM (one 512-byte segment per row and slot for the
 // wave) and outputs are staged through LDS so global stores are coalesced.  Blocks are
@@ -129,8 +129,12 @@ struct Pivot {
 
 // Pivoted elimination step (dgbtf2 with dgbtrs's forward solve) bringing in the row
 // (a, b, cc | d): returns the pivot row, advances the state.  A zero pivot leaves the other
-// row as it is, a zero entry of the pivot row its column (dger skips it).  Written without
-// branches: a step under a branch could not overlap the next row's independent work.
+// row as it is.  Written without branches: a step under a branch could not overlap the next
+// row's independent work.  (The band routines also skip zero entries; the product of one
+// changes at most the sign of a zero, which no temperature shows, and testing for them took
+// 6 % of the solve at 255x113x67 and 10 % at 128x64x1.)  Rows interchange at most cells where
+// the diffusion number is large, so steps that assume the pending row is the larger, with
+// these as the way out, took twice as long.
 __device__ __forceinline__ Pivot elim_step(Elim& e, double a, double b, double cc, double d,
                                            bool& swap, double* mult = nullptr) {
   swap = fabs(a) > fabs(e.r0);
@@ -143,25 +147,18 @@ __device__ __forceinline__ Pivot elim_step(Elim& e, double a, double b, double c
                od = swap ? e.rb : d;
   const bool live = p.u0 != 0.0;
   const double rp = 1.0 / p.u0;
-  const double l = rp * o0;
-  if (mult) *mult = live ? l : 0.0;
-  const double n1 = o1 + l * (-p.u1), n2 = o2 + l * (-p.u2), nd = od + l * (-p.y);
-  e.r0 = live & (p.u1 != 0.0) ? n1 : o1;
-  e.r1 = live & (p.u2 != 0.0) ? n2 : o2;
-  e.rb = live & (p.y != 0.0) ? nd : od;
+  const double l = live ? rp * o0 : 0.0;
+  if (mult) *mult = l;
+  e.r0 = o1 + l * (-p.u1);
+  e.r1 = o2 + l * (-p.u2);
+  e.rb = od + l * (-p.y);
   e.singular = e.singular | !live;
   return p;
 }
 
-// one row of dtbsv, column-oriented: x(i+2) U2 comes off first, then x(i+1) U1; a zero x(j)
-// contributes nothing, a zero row stays zero
+// one row of dtbsv, column-oriented: x(i+2) U2 comes off first, then x(i+1) U1
 __device__ __forceinline__ double back_step(const Pivot& p, double x1, double x2) {
-  const double a2 = p.y - x2 * p.u2;
-  double acc = x2 != 0.0 ? a2 : p.y;
-  const double a1 = acc - x1 * p.u1;
-  acc = x1 != 0.0 ? a1 : acc;
-  const double q = acc / p.u0;
-  return acc != 0.0 ? q : acc;
+  return ((p.y - x2 * p.u2) - x1 * p.u1) / p.u0;
 }
 
 template <int R, bool BE, bool ELEC, bool EXT>
@@ -614,8 +611,9 @@ __global__ __launch_bounds__(64, 2) void k_diffusion(DevGrid g, DevState s, doub
 // one wave eliminates both systems at once (lanes 0-31 the first solve, 32-63 the BDF2
 // matrix, one instruction stream) and keeps the pivot rows in the place of the terms it has
 // used, so nothing is formed twice and each pass is one chain of a few dozen instructions.
-// Same operations and order as above.  Wave kernel -> this one: 128x64x1 188 -> 66 us,
-// 96x24x20 148 -> 58, 64x24x16 103 -> 41, 24x12x8 48 -> 18, 500x10x10 699 -> 243.
+// Same operations and order as above.  128x64x1 58 us, 96x24x20 52 (the wave kernel 188 and
+// 148 before its zero tests went, this one 65 and 57 then; and 64x24x16 103 and 41, 24x12x8 48
+// and 18, 500x10x10 699 and 243).
 //
 // LDS rows of Q_SLOTS x W doubles and one more (which spreads the rows over the banks for the
 // threads of the first phase, which run along x1): row r at r RS.  Rows 0, N+1 and N+2 exist
