@@ -680,15 +680,13 @@ int run_step(double dt, double* tape) {
   // converted energy entering the x3 sweep, so a recorded step converts as a pass)
   const bool fuse = !tape && preconvert_fusable(g);
   if (fuse) {
-    launch_set_global_boundaries_preconvert(g, s, st);
-    launch_save_v1_boundaries(g, s, st);
+    launch_set_global_boundaries_preconvert(g, s, st);   // (:168 and :170)
     launch_sweep3_preconvert(g, s, dt, st, c.tune);
   } else {
     launch_v12rhov1_T2rhoe(g, s, true, true, st);        // libgemini.cpp:155-156
     if (tape) keep(0, s.ns);
-    launch_set_global_boundaries(g, s, LSP, st);         // :168
+    launch_set_global_boundaries(g, s, LSP, st, true);   // :168 and :170 (x1 planes kept for next step)
     halo_fields({NS, RHOVS1, RHOES, VS2, VS3});          // :169
-    launch_save_v1_boundaries(g, s, st);                 // :170 (x1 planes kept for next step)
     if (tape) {
       keep(1, s.rhoes);
       const AdjTape v = tape_view(tape);
@@ -731,14 +729,12 @@ int run_block(double dt) {
   const DevState& s = c.s;
   hipStream_t st = c.stream;
   if (preconvert_fusable(g)) {                           // as in run_step
-    launch_set_global_boundaries_preconvert(g, s, st);
-    launch_save_v1_boundaries(g, s, st);
+    launch_set_global_boundaries_preconvert(g, s, st);   // (:168 and :170)
     launch_sweep3_preconvert(g, s, dt, st, c.tune);
   } else {
     launch_v12rhov1_T2rhoe(g, s, true, true, st);        // libgemini.cpp:155-156
-    launch_set_global_boundaries(g, s, LSP, st);         // :168
+    launch_set_global_boundaries(g, s, LSP, st, true);   // :168 and :170
     halo_fields({NS, RHOVS1, RHOES, VS2, VS3});          // :169
-    launch_save_v1_boundaries(g, s, st);                 // :170
     launch_sweep(g, s, 3, F_ALL, dt, true, st, c.tune);  // :174-176
   }
   launch_sweep(g, s, 1, F_ALL, dt, true, st, c.tune);   // :178-180

@@ -88,10 +88,13 @@ void launch_v12rhov1_T2rhoe(const DevGrid& g, const DevState& s, bool mom, bool 
 void launch_rhov12v1(const DevGrid& g, const DevState& s, hipStream_t st);
 void launch_rhoe2T(const DevGrid& g, const DevState& s, hipStream_t st);
 void launch_post_convert(const DevGrid& g, const DevState& s, hipStream_t st);  // both above
-void launch_set_global_boundaries(const DevGrid& g, const DevState& s, int lsp, hipStream_t st);
+// save_v1: launch_save_v1_boundaries of all species with it (lsp = 7)
+void launch_set_global_boundaries(const DevGrid& g, const DevState& s, int lsp, hipStream_t st,
+                                  bool save_v1 = false);
 // the fused step's form of v12rhov1 + T2rhoe + ghost fill + x3 sweep: the conversions are
 // folded into the ghost fill and the x3 sweep (all sides global, x3 not periodic)
 bool preconvert_fusable(const DevGrid& g);
+// (with launch_save_v1_boundaries)
 void launch_set_global_boundaries_preconvert(const DevGrid& g, const DevState& s, hipStream_t st);
 void launch_sweep3_preconvert(const DevGrid& g, const DevState& s, double dt, hipStream_t st,
                               const Tuning& tune);

@@ -37,3 +37,24 @@ def test_sweep_dispatch_matches_oracle(shape, periodic):
             tr.pull(got)
             compare(got, ref, exact=VARS)
     tr.close()
+
+
+@pytest.mark.parametrize("size", [(4, 1, 1), (5, 1, 7), (4, 2, 1), (12, 3, 2), (61, 4, 9), (130, 17, 16)])
+def test_ghost_fill_in_one_launch(size):
+    """Inner columns that end as one, two or all of the ghost columns around them, blocks of
+    columns and of cells with remainders."""
+    g = ga.cartesian_grid(*size)
+    st = ga.synthetic_state(g, seed=9, perturb=g.lx2 > 1 and g.lx3 > 1)
+    rng = np.random.default_rng(9)
+    oracle.op(g, st, "v12rhov1")
+    oracle.op(g, st, "T2rhoe")
+    st.fluidvars[...] *= rng.uniform(0.5, 1.5, st.fluidvars.shape)
+    st.fluidauxvars[..., :14] *= rng.uniform(0.5, 1.5, st.fluidauxvars[..., :14].shape)
+    tr = Transport(g, st.nn, st.Tn)
+    tr.set_interface_vels(st)
+    a, b = st.copy(), st.copy()
+    oracle.op(g, a, "set_global_boundaries_allspec")
+    tr.set_global_boundaries_allspec(b)
+    assert np.array_equal(a.fluidvars, b.fluidvars)
+    assert np.array_equal(a.fluidauxvars[..., :14], b.fluidauxvars[..., :14])
+    tr.close()
