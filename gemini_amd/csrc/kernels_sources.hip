@@ -22,14 +22,15 @@
 // pairs run in lexicographic order, which adds each species' terms in the reference's
 // isp2 order; self-collision terms are exact zeros and are skipped.
 //
-// On 512x256x192 the energy pass moves 13.5 GB in 3.33 ms, the momentum pass 13.5 GB in
-// 3.79 ms, the mass pass 9.9 GB in 1.92 ms (a large copy takes 3.1, 3.1 and 2.3 ms for as
+// On 512x256x192 the energy pass needs 13.1 GB and takes 3.33 ms, the momentum pass 14.3 GB
+// and 3.7 ms, the mass pass 9.9 GB and 1.92 ms (a large copy takes 3.0, 3.3 and 2.3 ms for as
 // much).  The first two were bound by their instructions, some 8000 a cell, at 5.5 and
 // 6.5 ms: erf and exp in every pair; register arrays indexed by a rolled loop's pair, or 130
 // KB of unrolled code that misses the instruction cache; the edge logarithms of a gradient
 // inlined once per use.  Blocks of 128 threads are 2 to 4 % faster than 256.  Momentum is
-// held to 168 registers (3 waves per SIMD: 3.79 ms against 4.25); energy at 168 spills and
-// takes 5.1 ms against 3.33 at 223.
+// held to 168 registers (3 waves per SIMD: 3.8 ms against 4.25; 3.7 with its momenta read
+// where they are used, which takes the last spills and 3 GB of scratch traffic away); energy
+// at 168 spills and takes 5.1 ms against 3.33 at 223.
 #include "gemhip_internal.h"
 
 #pragma clang fp contract(fast)
@@ -338,8 +339,6 @@ __global__ __launch_bounds__(TPB, 3) void k_src_momentum(DevGrid g, DevState s, 
   double n[LSP], r[LSP - 1];
 #pragma unroll
   for (int i = 0; i < LSP; ++i) n[i] = s.ns[i * g.N + c];
-#pragma unroll
-  for (int i = 0; i < LSP - 1; ++i) r[i] = s.rhovs1[i * g.N + c];
   if (q.interior) {
     const long ni = (long)g.lx1 * g.lx2 * g.lx3, k = q.k;
     const int i1 = q.i1;
@@ -403,9 +402,12 @@ __global__ __launch_bounds__(TPB, 3) void k_src_momentum(DevGrid g, DevState s, 
       const double geom = (((((w2 * w2) * h3) * dh2dx1 + ((w3 * w3) * h2) * dh3dx1) * nsp) * m) / h1h2h3;
       const double Pp = ((((P[isp - 1] + (nsp * qs(isp)) * (E1f + Epol1)) - ionpress) - gQ) + geom) +
                         (nsp * m) * g1;
-      r[isp - 1] = etd(r[isp - 1], Pp, L[isp - 1], dt);
+      r[isp - 1] = etd(s.rhovs1[(isp - 1) * g.N + c], Pp, L[isp - 1], dt);   // (so late: registers)
       s.rhovs1[(isp - 1) * g.N + c] = r[isp - 1];
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < LSP - 1; ++i) r[i] = s.rhovs1[i * g.N + c];
   }
   // momentum_source_loss_solve (multifluid.f90:510-527), whole padded grid
   double chrgflux = 0.0;
