@@ -606,28 +606,35 @@ __global__ __launch_bounds__(64, 2) void k_diffusion(DevGrid g, DevState s, doub
 // ---------------------------------------------------------------- small grids
 // A grid with few columns leaves most of the GPU idle under the kernel above, whose waves then
 // take 1.5 us a row: four passes of a serial chain, the cells' conductivity and factors formed
-// by the same wave.  Here a workgroup of four waves owns W columns of one species and keeps
-// everything in LDS (nine doubles a row and column): all four form the parabolic terms, then
-// one wave eliminates both systems at once (lanes 0-31 the first solve, 32-63 the BDF2
-// matrix, one instruction stream) and keeps the pivot rows in the place of the terms it has
+// by the same wave.  Here a workgroup of 4 to 16 waves owns W columns of one species and keeps
+// everything in LDS (nine doubles a row and column): all form the matrices' rows, then one
+// wave eliminates both systems at once (lanes 0-31 the first solve, 32-63 the BDF2
+// matrix, one instruction stream) and keeps the pivot rows in the place of the rows it has
 // used, so nothing is formed twice and each pass is one chain of a few dozen instructions.
-// Same operations and order as above.  128x64x1 58 us, 96x24x20 52 (the wave kernel 188 and
-// 148 before its zero tests went, this one 65 and 57 then; and 64x24x16 103 and 41, 24x12x8 48
-// and 18, 500x10x10 699 and 243).
+// Same operations and order as above.  128x64x1 53.8 us, 96x24x20 46.5, 64x24x16 35 (the wave
+// kernel 188, 148 and 103; with the rows formed by the solving wave, and zero tests in it, this
+// one 65, 57 and 41).
 //
 // LDS rows of Q_SLOTS x W doubles and one more (which spreads the rows over the banks for the
 // threads of the first phase, which run along x1): row r at r RS.  Rows 0, N+1 and N+2 exist
 // and hold nothing: the walks read a row or two ahead.
-enum : int { Q_T1 = 0, Q_T3 = 1, Q_T2 = 2, Q_Y = 3,      // terms, then U0 U1 U2 and the rhs
+enum : int { Q_T1 = 0, Q_T3 = 1, Q_T2 = 2, Q_Y = 3,      // terms, then the first matrix's row
+                                                         // and rhs, then U0 U1 U2 and the rhs
              Q_T = 4,                                    // temperature, then the BDF2 rhs, x
-             Q_V = 5, Q_SLOTS = 9 };                     // C B D, then V0 V1 V2 and multiplier
+             Q_V = 5, Q_SLOTS = 9 };                     // C B D, then the BDF2 row, then V0 V1
+                                                         // V2 and multiplier
 __host__ __device__ inline size_t small_lds_bytes(int N, int W) {
   return (size_t)(N + 3) * (Q_SLOTS * W + 1) * sizeof(double) +
          (size_t)((N + 31) / 32) * W * sizeof(int);
 }
 
+// threads of a block: two of the wide blocks seldom share a CU, and their four or two waves a
+// SIMD hide the latency of the cells' inputs (256 threads: 96x24x20 51 us, 64x24x16 38; these
+// 46.5 and 35)
+__host__ __device__ constexpr int small_threads(int W) { return W >= 8 ? W * 64 : 256; }
+
 template <int W, bool BE, bool EXT>
-__global__ __launch_bounds__(256) void k_diffusion_small(DevGrid g, DevState s, Coef k1, Coef bdf,
+__global__ __launch_bounds__(small_threads(W)) void k_diffusion_small(DevGrid g, DevState s, Coef k1, Coef bdf,
                                                          double Teinf) {
   extern __shared__ double lds[];
   const int N = g.lx1, tid = threadIdx.x;
@@ -672,7 +679,7 @@ __global__ __launch_bounds__(256) void k_diffusion_small(DevGrid g, DevState s, 
     t2 = elec ? div_rcp(B, dxr + dxl, g.rdx1s[r]) : 0.0;
   };
   // ---- terms: threads along x1 (columns past the last repeat it)
-  for (int t = tid; t < N * W; t += 256) {
+  for (int t = tid; t < N * W; t += small_threads(W)) {
     const int c = t / N, r = t - c * N + 1;
     double T, C, B, D;
     cell(r, min(c0 + c, ncol - 1), T, C, B, D);
@@ -680,13 +687,34 @@ __global__ __launch_bounds__(256) void k_diffusion_small(DevGrid g, DevState s, 
     at(Q_V, r, c) = C; at(Q_V + 1, r, c) = B; at(Q_V + 2, r, c) = D;
   }
   __syncthreads();
-  for (int t = tid; t < N * W; t += 256) {
+  for (int t = tid; t < N * W; t += small_threads(W)) {
     const int c = t / N, r = t - c * N + 1;
     if (r == 1 || r == N) continue;
     double t1, t2, t3;
     terms(r, at(Q_V, r, c), at(Q_V + 1, r, c), at(Q_V + 2, r - 1, c), at(Q_V + 2, r, c),
           at(Q_V + 2, r + 1, c), t1, t2, t3);
     at(Q_T1, r, c) = t1; at(Q_T3, r, c) = t3; at(Q_T2, r, c) = t2;
+  }
+  __syncthreads();
+  // first solve: TR takes half of each term; backward Euler the whole, as BDF2
+  auto rhs1 = [&](double a, double tsum, double cc, double Tm, double Tc, double Tp) {
+    if (BE) return div_rcp(Tc, k1.dt, k1.K);
+    return ((div_rcp(Tc, k1.dt2, k1.K) - a * Tm) - tsum * Tc) - cc * Tp;
+  };
+  constexpr double half = BE ? 1.0 : 0.5;
+  // ---- the matrices' rows, so that the solving wave has only their elimination to do
+  for (int t = tid; t < N * W; t += small_threads(W)) {
+    const int c = t / N, r = t - c * N + 1;
+    if (r == 1 || r == N) continue;
+    const double f1 = at(Q_T1, r, c), f2 = at(Q_T2, r, c), f3 = at(Q_T3, r, c);
+    const double t1 = f1 * half, t2 = f2 * half, t3 = f3 * half;
+    const double a = -t1 + t2, cc = -t3 - t2;
+    at(Q_T1, r, c) = a; at(Q_T1 + 1, r, c) = (k1.K + t3) + t1; at(Q_T1 + 2, r, c) = cc;
+    at(Q_Y, r, c) = rhs1(a, t3 + t1, cc, at(Q_T, r - 1, c), at(Q_T, r, c), at(Q_T, r + 1, c));
+    if (!BE) {
+      at(Q_V, r, c) = -f1 + f2; at(Q_V + 1, r, c) = (bdf.K + f3) + f1; at(Q_V + 2, r, c) = -f3 - f2;
+      at(Q_V + 3, r, c) = 0.0;                         // (a right-hand side that nothing uses)
+    }
   }
   __syncthreads();
   // ---- the solves: one wave; lanes past W repeat the last column
@@ -713,32 +741,22 @@ __global__ __launch_bounds__(256) void k_diffusion_small(DevGrid g, DevState s, 
     }
     const int nw = (N + 31) / 32;
     int* prec = (EXT && elec && s.pivrec) ? s.pivrec + ((long)col * 2 + (second ? 1 : 0)) * nw : nullptr;
-    // first solve: TR takes half of each term; backward Euler and BDF2 the whole
-    const double half = BE || second ? 1.0 : 0.5, K = second ? bdf.K : k1.K;
     const int out = second ? Q_V : Q_T1;
-    auto rhs1 = [&](double a, double tsum, double cc, double Tm, double Tc, double Tp) {
-      if (BE) return div_rcp(Tc, k1.dt, k1.K);
-      return ((div_rcp(Tc, k1.dt2, k1.K) - a * Tm) - tsum * Tc) - cc * Tp;
-    };
     Elim e{1.0, 0.0, Tmin, false};
-    double Tm = at(Q_T, 1, c), Tc = at(Q_T, 2, c);
-    double n1 = at(Q_T1, 2, c), n2 = at(Q_T2, 2, c), n3 = at(Q_T3, 2, c), nT = at(Q_T, 3, c);
-    double* in = &at(0, 3, c);                         // the next row's terms
+    const double* in = &at(out, 2, c);                 // the next row
+    double na = in[0], nb = in[W], nc = in[2 * W], nd = in[3 * W];
     double* po = &at(out, 1, c);                       // pivot rows
     // step j brings row j+1 in; the bits of its interchanges, 32 steps a word
     auto step = [&](bool last) -> bool {
-      const double t1 = n1 * half, t2 = n2 * half, t3 = n3 * half, Tp = nT;
-      n1 = in[Q_T1 * W]; n2 = in[Q_T2 * W]; n3 = in[Q_T3 * W]; nT = in[Q_T * W + RS];
+      double a = na, b = nb, cc = nc, d = nd, l;
       in += RS;
-      double a = -t1 + t2, b = (K + t3) + t1, cc = -t3 - t2, l;
-      double d = rhs1(a, t3 + t1, cc, Tm, Tc, Tp);
+      na = in[0]; nb = in[W]; nc = in[2 * W]; nd = in[3 * W];
       if (last) { a = aN; b = bN; cc = 0.0; d = Tmax; }
       bool sw;
       const Pivot p = elim_step(e, a, b, cc, d, sw, &l);
       po[0] = p.u0; po[W] = p.u1; po[2 * W] = p.u2;
       po[3 * W] = second ? l : p.y;
       po += RS;
-      Tm = Tc; Tc = Tp;
       return sw;
     };
     auto word = [&](int j, int bits) {
@@ -772,8 +790,7 @@ __global__ __launch_bounds__(256) void k_diffusion_small(DevGrid g, DevState s, 
         cell(r + 1, col, T2, C2, B2, D2);
         double t1, t2, t3;
         terms(r, C1, B1, D0, D1, D2, t1, t2, t3);
-        const double h = BE ? 1.0 : 0.5;
-        t1 *= h; t2 *= h; t3 *= h;
+        t1 *= half; t2 *= half; t3 *= half;
         at(Q_Y, r, c) = rhs1(-t1 + t2, t3 + t1, -t3 - t2, T0, T1, T2);
         T0 = T1; D0 = D1; T1 = T2; C1 = C2; B1 = B2; D1 = D2;
       }
@@ -835,7 +852,7 @@ __global__ __launch_bounds__(256) void k_diffusion_small(DevGrid g, DevState s, 
     }
   }
   __syncthreads();
-  for (int t = tid; t < N * W; t += 256) {
+  for (int t = tid; t < N * W; t += small_threads(W)) {
     const int c = t / N, r = t - c * N + 1, col = c0 + c;
     if (col < ncol) s.Ts[so + gix(g, r, col % g.lx2 + 1, col / g.lx2 + 1)] = at(Q_T, r, c);
   }
@@ -961,12 +978,11 @@ size_t diffusion_noalloc_bytes(const DevGrid& g) {
 namespace {
 // Columns per block of the small-grid kernel, 0 where the wave kernel is faster: the fewest
 // that leave at most one block per CU (the solving waves of two would share a SIMD), else the
-// most that fit the LDS, if that takes at most two rounds of blocks: a round takes 0.5-0.7 us
-// a row, the wave kernel 1.4-1.6 at these sizes (98x40x36, 2.46 rounds: 160 by waves, 167
-// here; 300x20x20, 2.73: 435 and 437; 64x64x64, 3.5: 125 and 170).
-#ifndef SMALL_ROUNDS
-#define SMALL_ROUNDS 2.0
-#endif
+// most that fit the LDS, if that makes at most three blocks per CU.  A block costs its CU 0.45
+// us a row or more, at once or in turn, the wave kernel 1.3-1.8 us a row for all at these sizes
+// (us, wave kernel and this: 2.5 blocks 98x40x36 145 and 135; 2.73 16x40x40 43 and 31, 64x40x40
+// 102 and 92, 128x40x40 182 and 172; 3.9 64x48x48 107 and 121; 6.2 9x60x60 34 and 48, 33x60x61
+// 68 and 120; 22 9x115x113 47 and 147).
 int small_columns(const DevGrid& g) {
   constexpr size_t LDS = 160 * 1024;
   constexpr long CUS = 256;
@@ -977,7 +993,7 @@ int small_columns(const DevGrid& g) {
     if (b > LDS) break;
     const long blocks = (ncol + W - 1) / W * LSP;
     if (blocks <= CUS) return W;
-    best = (double)blocks <= SMALL_ROUNDS * CUS * (double)(LDS / b) ? W : 0;
+    best = blocks <= 3 * CUS ? W : 0;
   }
   return best;
 }
@@ -985,7 +1001,7 @@ int small_columns(const DevGrid& g) {
 template <int W>
 void small_launch(const DevGrid& g, const DevState& s, int diffsolvetype, double Teinf,
                   const Coef& tr, const Coef& bdf, const Coef& be, hipStream_t st) {
-  const dim3 grd((unsigned)(((long)g.lx2 * g.lx3 + W - 1) / W), LSP), blk(256);
+  const dim3 grd((unsigned)(((long)g.lx2 * g.lx3 + W - 1) / W), LSP), blk(small_threads(W));
   const size_t b = small_lds_bytes(g.lx1, W);
   if (diffsolvetype == 1)
     hipLaunchKernelGGL((k_diffusion_small<W, true, false>), grd, blk, b, st, g, s, be, bdf, Teinf);

@@ -43,6 +43,26 @@ def test_diffusion_tiles_match_oracle(shape, solver):
     tr.close()
 
 
+@pytest.mark.parametrize("shape", [
+    # blocks of 8 and 16 columns (512 and 1024 threads), the last one partly filled, up to three
+    # blocks a CU and just beyond
+    (96, 24, 20), (150, 15, 17), (98, 40, 36), (61, 41, 43),
+    # and many more columns, short and long rows
+    (9, 135, 135), (16, 108, 107), (24, 91, 91), (33, 71, 70)])
+def test_wide_blocks_and_the_wave_kernel_beyond_them(shape):
+    g = ga.cartesian_grid(*shape)
+    st = ga.synthetic_state(g, seed=sum(shape))
+    st.Ts[...] *= np.random.default_rng(1).uniform(0.5, 2.0, st.Ts.shape)
+    np.maximum(st.Ts, 100.0, out=st.Ts)
+    ref, got = st.copy(), st.copy()
+    with oracle.pow_mode(1):
+        oracle.op(g, ref, "energy_diffusion", dt=0.3, diffsolvetype=2)
+    tr = Transport(g, st.nn, st.Tn, own_context=True, diffsolvetype=2)
+    tr.energy_diffusion(got, 0.3)
+    compare(got, ref, exact=("Ts", "ns"))
+    tr.close()
+
+
 @pytest.mark.parametrize("solver", [2, 1])
 def test_singular_columns_in_both_kernels(solver):
     """Zero temperature on five rows and an infinite step make exact zero pivots."""
