@@ -159,7 +159,8 @@ constexpr double W2_NEAR = 1.0;
 // branch, so that the 21 unrolled pairs stay one run of instructions.  Pairs beyond enter
 // with zeros there, are marked in a mask, and lanes that hold any add them afterwards in a
 // rolled loop over the partner, whose values it reads again (it is never entered at ordinary
-// drifts, and its erf and exp would otherwise be part of every pair).
+// drifts, and its erf and exp would otherwise be part of every pair).  So are pairs whose W**2
+// is not a number.
 template <bool PSI, int NX, typename ADD>
 __device__ __forceinline__ void coulomb_terms(const DevGrid& g, const DevState& s, long c, const double* n,
                                               const double* T, const double* v1, ADD add) {
@@ -191,6 +192,8 @@ __device__ __forceinline__ void coulomb_terms(const DevGrid& g, const DevState& 
         if (!(far >> pair_bit(a, b) & 1u)) continue;
         const long o = (long)(y - 1) * g.N + c;
         const double Ty = s.Ts[o], vy = s.vs1[o], ny = s.ns[o];
+        // an infinite Teff (whose reciprocal root is no number above): 1/Teff**1.5 is zero
+        if (T[x - 1] == __builtin_inf() || Ty == __builtin_inf()) continue;
         const Pair p = coulomb_pair(ms(x), ms(y), T[x - 1], Ty, v1[x - 1], vy);
         double Phi, Psi;
         drift_far(p.W2, Phi, Psi);

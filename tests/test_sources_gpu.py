@@ -115,6 +115,38 @@ def test_drift_functions_over_their_branches(lx1):
             assert max_rel(a, b, f) <= RTOL, f"{which} {f}"
 
 
+@pytest.mark.parametrize("isp", [0, 3])              # the partner of lower, of higher index
+@pytest.mark.parametrize("which,fields,finite", [("momentum", ("vs1", "rhovs1"), 5),
+                                                 ("energy", ("Ts", "rhoes"), 0)])
+def test_infinite_temperature_of_one_species(isp, which, fields, finite):
+    """Teff**1.5 of a Coulomb pair is infinite then and the pair does not collide: in the
+    momentum pass the other ions of the cell, and every other cell, keep finite values (in the
+    energy pass its zero rate times the temperature is no number)."""
+    g = ga.cartesian_grid(20, 6, 5)
+    st = ga.synthetic_state(g, seed=8, perturb=True)
+    atm = ga.synthetic_atmosphere(g, st, seed=8)
+    for name in ("v12rhov1", "T2rhoe", "set_global_boundaries_allspec"):
+        oracle.op(g, st, name)
+    Q = np.zeros((g.lx1, g.lx2, g.lx3, 7), order="F")
+    oracle.op(g, st.copy(), "VNRicht_artvisc", Q=Q)
+    tr = transport(g, st, atm)
+    tr.VNRicht_artvisc(st.copy())
+    a = st.copy()
+    a.Ts[11, 5, 4, isp] = np.inf
+    b = a.copy()
+    oracle.source_loss(g, a, atm, 0.1, which, Q=Q)
+    tr.source_loss(b, which, 0.1)
+    for f in fields:
+        k, blk = FIELDS[f]
+        x, y = getattr(a, blk)[..., k:k + 7], getattr(b, blk)[..., k:k + 7]
+        fin = np.isfinite(x)
+        assert fin[11, 5, 4].sum() == finite
+        differ = np.argwhere(fin != np.isfinite(y))
+        assert len(differ) == 0, f"{f}: {differ[:7].tolist()}"
+        x, y = np.where(fin, x, 0.0), np.where(fin, y, 0.0)
+        assert np.all(np.abs(x - y) <= RTOL * np.max(np.abs(x), axis=(0, 1, 2))), f
+
+
 def null_cells(g, below):
     alt = np.asarray(g.planes["alt"][0])[2:-2, 2:-2].T          # (lx1, lx2)
     m = np.broadcast_to((alt < below)[:, :, None], (g.lx1, g.lx2, g.lx3))
