@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
                                    (24, 16, 17), (33, 20, 13), (40, 14, 14),
                                    # more columns than the small-grid kernel takes
                                    (9, 115, 113), (16, 92, 91), (24, 77, 78), (33, 60, 61),
-                                   # lines that take it from 16 columns a block to two
+                                   # long lines: two columns a block, the last one the wave kernel
                                    (110, 3, 5), (230, 3, 3), (440, 2, 3), (700, 1, 3), (1100, 1, 2)])
 @pytest.mark.parametrize("solver", [2, 1])
 def test_diffusion_tiles_match_oracle(shape, solver):
@@ -60,6 +60,97 @@ def test_wide_blocks_and_the_wave_kernel_beyond_them(shape):
     tr = Transport(g, st.nn, st.Tn, own_context=True, diffsolvetype=2)
     tr.energy_diffusion(got, 0.3)
     compare(got, ref, exact=("Ts", "ns"))
+    tr.close()
+
+
+# columns a block of the small-grid kernel owns there (0: the wave kernel takes the grid)
+WIDTHS = [((17, 8, 16), 4), ((150, 15, 17), 8), ((96, 24, 20), 16), ((98, 40, 36), 16),
+          # 1024 threads and the shortest rows, four and two columns because more do not fit
+          # the LDS, the longest row that fits and one more
+          ((4, 23, 21), 16), ((300, 20, 20), 4), ((600, 10, 20), 2), ((1073, 2, 2), 2),
+          ((1074, 2, 2), 0),
+          # blocks that outnumber the CUs three times
+          ((61, 41, 43), 0), ((24, 77, 78), 0)]
+
+
+def small_columns(lx1, lx2, lx3):
+    """The kernel's rule: the fewest columns that leave one block per CU, else the most that
+    fit the LDS if that makes at most three."""
+    best = 0
+    for w in (2, 4, 8, 16):
+        if (lx1 + 3) * (9 * w + 1) * 8 + (lx1 + 31) // 32 * w * 4 > 160 * 1024:
+            break
+        blocks = (lx2 * lx3 + w - 1) // w * 7
+        if blocks <= 256:
+            return w
+        best = w if blocks <= 768 else 0
+    return best
+
+
+@pytest.mark.parametrize("shape,width", WIDTHS)
+def test_both_solvers_at_each_block_width(shape, width):
+    print(f"case {shape} width {width}", flush=True)
+    assert small_columns(*shape) == width
+    g = ga.cartesian_grid(*shape)
+    st = ga.synthetic_state(g, seed=sum(shape))
+    st.Ts[...] *= np.random.default_rng(1).uniform(0.5, 2.0, st.Ts.shape)
+    np.maximum(st.Ts, 100.0, out=st.Ts)
+    for solver in (2, 1):
+        ref, got = st.copy(), st.copy()
+        with oracle.pow_mode(1):
+            oracle.op(g, ref, "energy_diffusion", dt=0.3, diffsolvetype=solver)
+        tr = Transport(g, st.nn, st.Tn, own_context=True, diffsolvetype=solver)
+        tr.energy_diffusion(got, 0.3)
+        compare(got, ref, exact=("Ts", "ns"))
+        tr.close()
+
+
+@pytest.mark.parametrize("shape,width", [((17, 8, 16), 4), ((40, 14, 14), 8), ((96, 24, 20), 16),
+                                         ((24, 77, 78), 0), ((33, 70, 71), 0), ((16, 64, 90), 0)])
+def test_fitting_extension_at_each_block_width(shape, width):
+    """Also the wave kernel of chunk height 8, its groups with columns in turn and with even and
+    odd ones apart; conductivity scale and heat flux together and each alone."""
+    print(f"case {shape} width {width}", flush=True)
+    assert small_columns(*shape) == width
+    g = ga.cartesian_grid(*shape)
+    st = ga.synthetic_state(g, seed=6)
+    rng = np.random.default_rng(7)
+    kappa = rng.uniform(0.5, 1.5, (g.lx2, g.lx3))
+    qtop = rng.uniform(0.0, 1e-5, (g.lx2, g.lx3))
+    tr = Transport(g, st.nn, st.Tn, own_context=True)
+    tr.set_residency(1)
+    for k, q in ((kappa, qtop), (kappa, None), (None, qtop)):
+        ref, got = st.copy(), st.copy()
+        with oracle.pow_mode(1):
+            oracle.transport_step(g, ref, 0.2, kappa=k, qtop=q)
+        tr.set_conductivity_scale(k)
+        tr.set_top_heat_flux(q)
+        tr.push(got)
+        tr.transport_step(0.2)
+        tr.pull(got)
+        compare(got, ref, exact=("Ts", "ns"))
+    tr.close()
+
+
+@pytest.mark.parametrize("shape,width", [((21, 24, 20), 16), ((21, 45, 46), 0), ((24, 46, 46), 0)])
+@pytest.mark.parametrize("solver", [2, 1])
+def test_singular_columns_at_chunk_height_eight(shape, width, solver):
+    """Zero pivots (see test_singular_columns_in_both_kernels) in every column group: rows of
+    odd length put the groups' row windows at every phase."""
+    print(f"case {shape} solver {solver}", flush=True)
+    assert small_columns(*shape) == width
+    g = ga.cartesian_grid(*shape)
+    st = ga.synthetic_state(g, seed=5)
+    st.J1[...] = 0.0
+    cold = np.random.default_rng(3).random((g.lx2, g.lx3, 7)) < 0.04
+    T = st.Ts[8:13, 2:-2, 2:-2, :]
+    T[...] = np.where(cold, 0.0, T)
+    ref, got = st.copy(), st.copy()
+    with oracle.pow_mode(1):
+        oracle.op(g, ref, "energy_diffusion", dt=np.inf, diffsolvetype=solver)
+    tr = Transport(g, st.nn, st.Tn, own_context=True, diffsolvetype=solver)
+    tr.energy_diffusion(got, np.inf)
+    compare(got, ref, exact=("Ts",))
     tr.close()
 
 
