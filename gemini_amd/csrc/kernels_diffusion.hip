@@ -717,9 +717,9 @@ __global__ __launch_bounds__(small_threads(W)) void k_diffusion_small(DevGrid g,
     }
   }
   __syncthreads();
-  // ---- the solves: one wave; lanes past W repeat the last column
-  if ((tid >> 6) == (int)((blockIdx.x >> 8) & 3)) {    // (blocks of one CU on different SIMDs)
-    const int lane = tid & 63, c = min(lane & 31, W - 1);
+  // ---- the solves: the first wave; lanes past W repeat the last column
+  if (tid < 64) {
+    const int lane = tid, c = min(lane & 31, W - 1);
     const bool second = !BE && lane >= 32;             // the BDF2 factorisation
     const int col = min(c0 + c, ncol - 1);
     double Tmin, Tmax, aN = 0.0, bN = 1.0;
