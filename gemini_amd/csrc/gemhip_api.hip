@@ -19,9 +19,9 @@
 #include "gemhip_internal.h"
 #include "gemhip_io.h"
 
-// Work space of gemhip_energy_diffusion_noalloc (TRBDF2 pivot rows, right-hand sides,
-// solutions and row interchanges): a static device array of NOALLOC_SCRATCH_BYTES, one copy
-// on every GPU the library runs on, held until the process ends.  Host code never uses
+// Work space of gemhip_energy_diffusion_noalloc (the wave kernel's kept rows and elimination
+// states): a static device array of NOALLOC_SCRATCH_BYTES, one copy on every GPU the library
+// runs on, held until the process ends.  Host code never uses
 // this name as an address: gemhip_init looks the array's device address up once per
 // device (noalloc_scratch below) and the kernels receive that address.
 #define NOALLOC_SCRATCH_BYTES (256ul << 20)
@@ -1326,9 +1326,11 @@ void energy_diffusion_C(void** cfgC, int* xtype, void** xC, double** fluidvars,
 // static `scratch` array instead of library allocations: Ts and ns are the 7 ghosted species
 // fields of fluidvars(:,:,:,29:35) and (:,:,:,1:7), J1 one ghosted field, all in HBM.  The
 // selected context supplies the grid, neutrals and configuration.  Enqueued on the
-// context's stream (gemhip_synchronize waits for it).  Every pivot row, right-hand side,
-// solution and interchange word is written before it is read within a call, so the work
-// space needs no clearing; calls that overlap on one GPU share it and race.
+// context's stream (gemhip_synchronize waits for it).  A call uses no value of the work space
+// that it has not written (it may read term slots of rows 1 and N that nothing has written, and
+// drops them), so the space needs no clearing; calls that overlap on one GPU share it and race.
+// Which grids are taken is part of the interface and does not follow the work space's layout;
+// what the layout needs is checked as well.
 int gemhip_energy_diffusion_noalloc(double* Ts, const double* ns, const double* J1, double dt) {
   if (!ready(true)) return 1;
   Ctx& c = ctx();
@@ -1337,10 +1339,10 @@ int gemhip_energy_diffusion_noalloc(double* Ts, const double* ns, const double* 
     fail("kernel timing creates events on demand: disable it before allocation-free calls");
     return 3;
   }
-  const size_t need = diffusion_noalloc_bytes(c.g);
-  if (need > (size_t)NOALLOC_SCRATCH_BYTES) {
-    fail("grid %dx%dx%d needs %zu bytes of diffusion work space; the allocation-free entry "
-         "point has %zu", c.lx1, c.lx2, c.lx3, need, (size_t)NOALLOC_SCRATCH_BYTES);
+  const size_t counts = diffusion_noalloc_bytes(c.g), limit = NOALLOC_SCRATCH_BYTES;
+  if (counts > limit || diffusion_scratch_bytes(c.g) > limit) {
+    fail("grid %dx%dx%d is beyond the size limit of the allocation-free entry point: it counts "
+         "as %zu bytes of diffusion work space, the limit is %zu", c.lx1, c.lx2, c.lx3, counts, limit);
     return 4;
   }
   if (c.device >= MAX_DEVICES || !noalloc_scratch[c.device]) {

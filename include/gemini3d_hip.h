@@ -349,7 +349,7 @@ int gemhip_adjoint_step(double dt, const double* tape, double* lam, double* gkap
    fields the caller owns -- Ts and ns the 7 ghosted species fields of
    fluidvars(:,:,:,29:35) and (:,:,:,1:7), J1 one ghosted field -- with the grid,
    neutrals and configuration of the selected context.  The TRBDF2 work space is a static
-   device array of 256 MiB (one per GPU, held until the process ends); grids that need
+   device array of 256 MiB (one per GPU, held until the process ends); grids that count as
    more (7 * ceil(lx2*lx3/64) * (4608*lx1 + 256*ceil(lx1/32) + 256) bytes, about 1000
    columns at lx1 = 512) are rejected with an error.  Calls no allocator; kernel timing
    must be off.  Enqueued on the context's stream (gemhip_synchronize waits).  Calls that

@@ -69,3 +69,31 @@ def test_noalloc_refuses_grids_beyond_its_work_space():
         assert b"work space" in tr.lib.gemhip_last_error()
     finally:
         tr.close()
+
+
+@pytest.mark.parametrize("lx2,taken", [(32, True), (33, False)])
+def test_noalloc_takes_the_grids_of_its_interface(lx2, taken):
+    """The last grid below the limit that the header states and the first one above it."""
+    g = ga.cartesian_grid(512, lx2, 32)
+    counts = 7 * ((lx2 * 32 + 63) // 64) * (4608 * 512 + 256 * 16 + 256)
+    assert (counts <= 256 << 20) == taken
+    st = ga.synthetic_state(g, seed=5)
+    tr = Transport(g, st.nn, st.Tn, own_context=True)
+    try:
+        Ts = _device(st.fluidvars[..., 28:35])
+        ns = _device(st.fluidvars[..., 0:7])
+        J1 = _device(st.electrovars[..., 3])
+        rc = _noalloc(tr, Ts, ns, J1, 0.1)
+        if taken:
+            assert rc == 0, tr.lib.gemhip_last_error()
+            ref = st.copy()
+            tr.energy_diffusion(ref, 0.1)
+            got = Ts.cpu().numpy().reshape((7,) + g.padded[::-1]).transpose(3, 2, 1, 0)
+            assert np.array_equal(got, ref.fluidvars[..., 28:35])
+        else:
+            assert rc == 4
+            err = tr.lib.gemhip_last_error()
+            assert b"size limit" in err and b"counts as %d bytes" % counts in err
+            assert np.array_equal(Ts.cpu().numpy(), np.asfortranarray(st.fluidvars[..., 28:35]).ravel(order="F"))
+    finally:
+        tr.close()
