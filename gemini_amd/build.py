@@ -4,8 +4,10 @@ The HDF5 file layer (csrc/h5io.cpp) is compiled against hdf5.h and loads libhdf5
 file is first read or written, so the library has no load-time dependency on it.
 
 Flags that matter for results:
-  -ffp-contract=off   no fused multiply-add: every product and sum is rounded on its
-                      own, as in the reference's x86-64 build (bit-identical parity),
+  -ffp-contract=off   no fused multiply-add unless written: every product and sum is
+                      rounded on its own, as in the reference's x86-64 build (bit-identical
+                      parity).  kernels_sources.hip, whose rates call transcendental
+                      functions and match to 1e-12, contracts by a pragma of its own,
   -Xclang -target-feature -Xclang -packed-fp32-ops
                       no packed FP32 instructions anywhere in the device code.
 """

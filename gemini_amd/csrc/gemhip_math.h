@@ -2,10 +2,11 @@
 //
 // Everything here must round exactly like the reference build (gfortran for the
 // x86-64 baseline: no FMA, IEEE divide and sqrt, glibc pow).  The library is
-// compiled with -ffp-contract=off, so a*b+c stays two rounded operations; divides
-// stay divides (never a reciprocal multiply).  The header also compiles as plain
-// C++ on the host (GEMHIP_HD expands to nothing) so the CPU tests can check the
-// scalar routines against libm.
+// compiled with -ffp-contract=off, so a*b+c stays two rounded operations; a divide
+// stays one, or is div_rcp, which gives its result from the divisor's correctly
+// rounded reciprocal.  (The source passes alone are held to a tolerance and contract.)
+// The header also compiles as plain C++ on the host (GEMHIP_HD expands to nothing) so
+// the CPU tests can check the scalar routines against libm.
 #pragma once
 
 #include <stdint.h>
@@ -55,7 +56,8 @@ GEMHIP_HD double fmax_f(double a, double b) { return (b > a) ? b : a; }
 // x / b from y = RN(1/b), correctly rounded: q0 = RN(x y) is within a few ulps of x/b,
 // the FMA residual x - b q0 is exact, and one correction step q0 + r y, rounded once,
 // gives RN(x/b) (Markstein's theorem for a correctly rounded reciprocal).  v_div_fixup_f64
-// gives the quotients of zeros (with their sign), infinities and NaN.
+// gives the quotients of zeros (with their sign), infinities and NaN.  The residual is exact
+// while x and the quotient are above 2^-960 or so; below, the result may be off by an ulp.
 __device__ __forceinline__ double div_rcp(double x, double b, double y) {
   const double q0 = x * y;
   const double r = __builtin_fma(-b, q0, x);

@@ -339,7 +339,7 @@ struct AdjArgs {
 // (r0, r1 | rb), as dgbtf2 + dgbtrs do it (kernels_diffusion.hip): stores the pivot row, its
 // reciprocal and rhs and the multiplier.  An interchange shows in the third entry, which is
 // +0 without one (and -0 where an interchange brings a zero).  The zero tests of the band
-// routines only skip work that changes nothing, and are left out.
+// routines only skip work that changes nothing (of finite entries), and are left out.
 template <bool RHS>
 __device__ __forceinline__ bool adj_elim(const Col& q, int j, int s0, double& r0, double& r1,
                                          double& rb, double a, double b, double cc, double d) {

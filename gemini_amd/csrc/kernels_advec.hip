@@ -1504,9 +1504,6 @@ void launch_save_v1_boundaries(const DevGrid& g, const DevState& s, hipStream_t 
   timing_end("save_v1b", st);
 }
 
-// The DMA ring loads 16-byte pairs of cells: every pair must be 16-byte aligned, so rows of
-// an even length (lx1 + 4) and fields at 16-byte aligned addresses; otherwise the sweeps
-// prefetch through registers.
 // Species waves of a block of the x2/x3 sweeps (SHM), seven unless the grid leaves CUs idle:
 // a march is a serial chain, and two species waves on a SIMD take each step in turns.  So
 // while the (x1 block, line) pairs times the groups fit the 256 CUs, the species go to
@@ -1522,6 +1519,9 @@ static int sweep_species(const DevGrid& g, int dir) {
   return pairs * 4 <= SWEEP_CUS ? 2 : pairs * 2 <= SWEEP_CUS ? 4 : LSP;
 }
 
+// The DMA ring loads 16-byte pairs of cells: every pair must be 16-byte aligned, so rows of
+// an even length (lx1 + 4) and fields at 16-byte aligned addresses; otherwise the sweeps
+// prefetch through registers.
 static bool sweep_dma_ok(const DevGrid& g, std::initializer_list<const double*> fields) {
   if (SWEEP_DMA <= 0 || g.L1 % 2 != 0) return false;
   for (const double* f : fields)

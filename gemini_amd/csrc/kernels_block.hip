@@ -240,8 +240,9 @@ __global__ void k_rhov12v1_clean_density(DevGrid g, double* ns, const double* rh
 // The same without null cells, and VNRicht_artvisc with it (src/libgemini.cpp:186-191;
 // clean_param(2) between them changes nothing then).  A block owns whole columns, so that the
 // viscosity finds its x1 neighbours' velocities in LDS and no cell reads a density that
-// another block has cleaned: cols columns of L1 cells, a thread per cell.  Bound by HBM:
-// 1.29 ms at 512x256x192, 1.04 and 0.73 ms as two passes.
+// another block has cleaned: cols columns of L1 cells, a thread per cell.  Against the two
+// passes: 1.63 ms and 1.04 + 0.71 at 512x256x192, 0.115 and 0.090 + 0.063 at 255x113x67,
+// 0.0114 and 0.0109 + 0.0080 at 98x40x36.
 __global__ __launch_bounds__(1024) void k_rhov12v1_clean_artvisc(DevGrid g, int cols, double* ns,
                                                                  const double* rhovs1, double* vs1,
                                                                  double* Q) {

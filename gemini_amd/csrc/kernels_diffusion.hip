@@ -9,14 +9,14 @@
 // Each column (fixed x2, x3, species) is solved by one lane, reproducing operation for
 // operation what the reference computes for it: the conductivity and the band matrix
 // entries in the reference's expression order, then LAPACK's banded LU with partial
-// pivoting (dgbtf2: idamax pivot search, dscal by the reciprocal pivot, dger update
-// skipping zero columns; dgbtrs: row swaps and dger on the right-hand side; dtbsv:
-// column-oriented back substitution).  The matrix is tridiagonal stored with kl=ku=2,
-// so of the band only the three diagonals and the pivoting fill-in can be non-zero;
-// every other term LAPACK forms is a multiply by an exact zero and leaves values
-// unchanged, so those terms are not formed.  The divisions stay true IEEE divisions and
-// the file is built with -ffp-contract=off, which makes the result bit-identical to the
-// reference arithmetic apart from x**2.5 (correctly rounded here, libm pow there).
+// pivoting (dgbtf2: idamax pivot search, dscal by the reciprocal pivot, dger update;
+// dgbtrs: row swaps and dger on the right-hand side; dtbsv: column-oriented back
+// substitution).  The matrix is tridiagonal stored with kl=ku=2, so of the band only the
+// three diagonals and the pivoting fill-in can be non-zero; every other term LAPACK forms
+// is a multiply by an exact zero and leaves values unchanged, so those terms are not
+// formed.  Divisions are IEEE divisions or give their results (div_rcp), and the file is
+// built with -ffp-contract=off, which makes the result bit-identical to the reference
+// arithmetic apart from x**2.5 (correctly rounded here, libm pow there).
 #include <type_traits>
 
 #include "diffusion_cell.h"
@@ -130,9 +130,11 @@ struct Pivot {
 // Pivoted elimination step (dgbtf2 with dgbtrs's forward solve) bringing in the row
 // (a, b, cc | d): returns the pivot row, advances the state.  A zero pivot leaves the other
 // row as it is.  Written without branches: a step under a branch could not overlap the next
-// row's independent work.  (The band routines also skip zero entries; the product of one
-// changes at most the sign of a zero, which no temperature shows, and testing for them took
-// 6 % of the solve at 255x113x67 and 10 % at 128x64x1.)  Rows interchange at most cells where
+// row's independent work.  (The band routines also skip zero entries; while the entries and the
+// pivot's reciprocal are finite, the product of one changes at most the sign of a zero, which no
+// temperature shows.  Columns with an infinite or NaN temperature or density, a step of zero or of
+// infinity come out alike with and without the tests.  These took 6 % of the solve at 255x113x67
+// and 10 % at 128x64x1.)  Rows interchange at most cells where
 // the diffusion number is large, so steps that assume the pending row is the larger, with
 // these as the way out, took twice as long.
 __device__ __forceinline__ Pivot elim_step(Elim& e, double a, double b, double cc, double d,

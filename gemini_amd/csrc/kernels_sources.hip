@@ -12,7 +12,8 @@
 // operation at most: products and sums contract into FMAs in this file, a divide by a
 // compile-time constant (a mass sum, 3) is a multiply by its correctly rounded reciprocal, a
 // Coulomb pair's powers of 1/Teff come from one reciprocal root and its drift functions from
-// their series.  The transcendental functions (exp, log, log10, erf, tanh, sin, and x**p for
+// their series (1/Teff and its root to an ulp or so, where the reference divides and takes a
+// correctly rounded power).  The transcendental functions (exp, log, log10, erf, tanh, sin, and x**p for
 // the fitted exponents) are the device library's, which agree with glibc to about an ulp;
 // x**0.5 is the correctly rounded sqrt.  These passes therefore match the reference to
 // rounding (the tests hold them to 1e-12 of each field's magnitude) rather than bit for bit.
@@ -22,9 +23,10 @@
 // pairs run in lexicographic order, which adds each species' terms in the reference's
 // isp2 order; self-collision terms are exact zeros and are skipped.
 //
-// On 512x256x192 the energy pass needs 13.1 GB and takes 3.33 ms, the momentum pass 14.3 GB
-// and 3.7 ms, the mass pass 9.9 GB and 1.92 ms (a large copy takes 3.0, 3.3 and 2.3 ms for as
-// much).  The first two were bound by their instructions, some 8000 a cell, at 5.5 and
+// On 512x256x192 the energy pass moves 13.6 GB in 3.3 ms, the momentum pass 17.5 GB in 3.75, the
+// mass pass 10.9 GB in 1.97: 4.1, 4.7 and 5.5 TB/s, with vector instructions at 70, 57 and 60 %
+// of the FP64 issue rate.  At two waves a SIMD the energy pass is still held by issue and
+// latency, the other two by both.  The first two had some 8000 instructions a cell, at 5.5 and
 // 6.5 ms: erf and exp in every pair; register arrays indexed by a rolled loop's pair, or 130
 // KB of unrolled code that misses the instruction cache; the edge logarithms of a gradient
 // inlined once per use.  Blocks of 128 threads are 2 to 4 % faster than 256.  Momentum is
@@ -111,8 +113,8 @@ __device__ __forceinline__ double csj_1e6(int x, int y) {
 }
 
 // Psi = exp(-x) and Phi = 3 int_0^1 t^2 exp(-x t^2) dt for x = W**2 in [0, 1]: their power
-// series, sum (-x)^k/k! and sum 3 (-x)^k/(k! (2k+3)), interpolated at Chebyshev points (off
-// by 8e-18 and 3e-17 at most).  A table in memory, so that it is read into scalar registers.
+// series, sum (-x)^k/k! and sum 3 (-x)^k/(k! (2k+3)), interpolated at Chebyshev points (with the
+// rounded coefficients off by 3.7e-17 and 6.1e-17 at most, near x = 1).  A table in memory, so that it is read into scalar registers.
 __constant__ double c_drift[25] = {
     1.0, -0.5999999999999948, 0.21428571428546575, -0.05555555555090525, 0.011363636318628153,
     -0.0019230766656642064, 0.0002777768425337601, -3.5011761846027854e-05, 3.912431467016512e-06,

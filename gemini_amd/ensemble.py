@@ -143,7 +143,11 @@ class Batch:
 
     ``step(n)`` issues n steps on the batch's stream; ``run(n)`` launches n steps captured
     in one HIP graph (cached per n); the knobs ``sweep_pf``, ``diff_chunk`` (kernel
-    variants) and ``grid`` (persistent blocks per CU) change speed only."""
+    variants) and ``grid`` (persistent blocks per CU) change speed only.
+
+    The batched kernels are those of large grids: a member's own launches also have small-grid
+    forms and LDS DMA loads, so :meth:`Ensemble.run` is usually the faster choice (20 steps of
+    64 members of 0.1 M to 5.6 M cells 1.01 s against 1.20 s)."""
 
     KNOBS = {"sweep_pf": (1, 2), "diff_chunk": (4, 8), "grid": (1, 2)}
 

@@ -367,7 +367,10 @@ int gemhip_energy_diffusion_noalloc(double* Ts, const double* ns, const double* 
    the batch exists; members of a batch cannot be destroyed.  The time steps live in HBM,
    so gemhip_batch_set_dt also changes what captured graphs do.  Tuning knobs:
    "sweep_pf" (1, 2), "diff_chunk" (4, 8), "grid" (1, 2: persistent blocks per CU times
-   this); they change speed only.  gemhip_batch_capture returns a graph id for
+   this); they change speed only.  The kernels are the ones for large grids: members do not
+   get the small-grid diffusion, the split x2/x3 sweeps, the LDS DMA loads or the ghost fill in
+   one launch that their own steps use, so a graph of the members' own launches
+   (gemhip_ensemble_capture) is usually the faster form.  gemhip_batch_capture returns a graph id for
    gemhip_ensemble_launch (launched on the batch's stream), released with the batch at
    the latest. */
 int gemhip_batch_create(int n, const int* handles);      /* batch id >= 1, or < 0 */
