@@ -11,28 +11,27 @@
 // Arithmetic follows the reference's expressions, with liberties that cost a few ulp per
 // operation at most: products and sums contract into FMAs in this file, a divide by a
 // compile-time constant (a mass sum, 3) is a multiply by its correctly rounded reciprocal, a
-// Coulomb pair's powers of 1/Teff come from one reciprocal root and its drift functions from
-// their series (1/Teff and its root to an ulp or so, where the reference divides and takes a
-// correctly rounded power).  The transcendental functions (exp, log, log10, erf, tanh, sin, and x**p for
-// the fitted exponents) are the device library's, which agree with glibc to about an ulp;
-// x**0.5 is the correctly rounded sqrt.  These passes therefore match the reference to
-// rounding (the tests hold them to 1e-12 of each field's magnitude) rather than bit for bit.
+// Coulomb pair's powers of 1/Teff come from one reciprocal root (to an ulp or so, where the
+// reference divides and takes a power) and its drift functions from polynomials.  The
+// transcendental functions of the other rates (exp, log, log10, tanh, sin, and x**p for the
+// fitted exponents) are the device library's, which agree with glibc to about an ulp; x**0.5 is
+// the correctly rounded sqrt.  These passes therefore match the reference to rounding (the
+// tests hold them to 1e-12 of each field's magnitude) rather than bit for bit.
 //
 // Ion-ion (Coulomb) terms: Teff, Wsj, Phisj and Psisj of coulomb_colln are symmetric in
 // the species pair, so each unordered pair is evaluated once and feeds both species.  The
 // pairs run in lexicographic order, which adds each species' terms in the reference's
 // isp2 order; self-collision terms are exact zeros and are skipped.
 //
-// On 512x256x192 the energy pass moves 13.6 GB in 3.3 ms, the momentum pass 17.5 GB in 3.75, the
-// mass pass 10.9 GB in 1.97: 4.1, 4.7 and 5.5 TB/s, with vector instructions at 70, 57 and 60 %
-// of the FP64 issue rate.  At two waves a SIMD the energy pass is still held by issue and
+// On 512x256x192 the energy pass moves 13.6 GB in 3.3 ms, the momentum pass 17.5 GB in 3.7, the
+// mass pass 10.9 GB in 1.97: 4.1, 4.7 and 5.5 TB/s, with vector instructions at some 70, 57 and
+// 60 % of the FP64 issue rate.  At two waves a SIMD the energy pass is still held by issue and
 // latency, the other two by both.  The first two had some 8000 instructions a cell, at 5.5 and
 // 6.5 ms: erf and exp in every pair; register arrays indexed by a rolled loop's pair, or 130
 // KB of unrolled code that misses the instruction cache; the edge logarithms of a gradient
-// inlined once per use.  Blocks of 128 threads are 2 to 4 % faster than 256.  Momentum is
-// held to 168 registers (3 waves per SIMD: 3.8 ms against 4.25; 3.7 with its momenta read
-// where they are used, which takes the last spills and 3 GB of scratch traffic away); energy
-// at 168 spills and takes 5.1 ms against 3.33 at 223.
+// inlined once per use.  Blocks of 128 threads are 2 to 4 % faster than 256.  Momentum
+// takes 135 registers (3 waves per SIMD), reading its momenta where they are used; energy 225
+// (two; at 168 it spills and took 5.1 ms against 3.33).
 #include "gemhip_internal.h"
 
 #pragma clang fp contract(fast)
@@ -114,14 +113,24 @@ __device__ __forceinline__ double csj_1e6(int x, int y) {
 
 // Psi = exp(-x) and Phi = 3 int_0^1 t^2 exp(-x t^2) dt for x = W**2 in [0, 1]: their power
 // series, sum (-x)^k/k! and sum 3 (-x)^k/(k! (2k+3)), interpolated at Chebyshev points (with the
-// rounded coefficients off by 3.7e-17 and 6.1e-17 at most, near x = 1).  A table in memory, so that it is read into scalar registers.
-__constant__ double c_drift[25] = {
+// rounded coefficients off by 3.7e-17 and 6.1e-17 at most, near x = 1).  Then, for x above 1,
+// h(u) = 3/2 + 3/4 sqrt(pi) u exp(x) erfc(1/u) with u = 1/sqrt(x), in powers of 2 u - 1: fitted
+// where exp(-x) matters (u above 0.156), its share of Phi off by 2.6e-17 of Phi at most; and 1/k!.
+// Tables in memory, so that they are read into scalar registers.
+__constant__ double c_drift[57] = {
     1.0, -0.5999999999999948, 0.21428571428546575, -0.05555555555090525, 0.011363636318628153,
     -0.0019230766656642064, 0.0002777768425337601, -3.5011761846027854e-05, 3.912431467016512e-06,
     -3.898097348795919e-07, 3.327267488170533e-08, -1.9011473537307833e-09,
     1.0, -0.999999999999999, 0.4999999999999427, -0.16666666666540417, 0.041666666652193346,
     -0.008333333234481316, 0.0013888884549085943, -0.00019841141919339013, 2.4798998659720724e-05,
-    -2.7521178006932173e-06, 2.721363367981267e-07, -2.2905624278899246e-08, 1.2719039650810423e-09};
+    -2.7521178006932173e-06, 2.721363367981267e-07, -2.2905624278899246e-08, 1.2719039650810423e-09,
+    1.66975389374294, 0.3117227437994364, 0.11114017474596585, -0.0289303739213432,
+    0.004581320932399893, 0.0008654691675095566, -0.0011654640359131995, 0.0005916453698633884,
+    -0.00017255696227433563, -7.169342455466241e-06, 4.8919590990281544e-05, -3.839188796818616e-05,
+    1.895223840237792e-05, -5.702602069219486e-06, 2.1974621485947115e-07, 7.00313799736029e-07,
+    -3.1185083070019743e-07, 4.806131617009341e-08,
+    1.0, 1.0, 1.0 / 2.0, 1.0 / 6.0, 1.0 / 24.0, 1.0 / 120.0, 1.0 / 720.0, 1.0 / 5040.0, 1.0 / 40320.0,
+    1.0 / 362880.0, 1.0 / 3628800.0, 1.0 / 39916800.0, 1.0 / 479001600.0, 1.0 / 6227020800.0};
 template <int DEG>
 __device__ __forceinline__ double horner(const double* c, double x) {
   double b = c[DEG];
@@ -130,80 +139,108 @@ __device__ __forceinline__ double horner(const double* c, double x) {
   return b;
 }
 
-// The pair-symmetric part of coulomb_colln (collisions.f90:138-157) for species a < b:
-// 1/Teff**1.5 and W**2.  1/Teff and its power come from one v_rsq_f64: two Newton steps give
-// the reciprocal root to about an ulp, one residual correction its square.
-struct Pair { double iT15, W2; };
-__device__ __forceinline__ Pair coulomb_pair(double ma, double mb, double Ta, double Tb, double va, double vb) {
-  const double x = __builtin_fma(mb, Ta, ma * Tb) * (1.0 / (mb + ma));
+// 1/sqrt(x) to about an ulp: v_rsq_f64 and two Newton steps; and 1/x by one residual correction
+__device__ __forceinline__ double rsqrt2(double x, double& rcp) {
   double y = __builtin_amdgcn_rsq(x);
   y = __builtin_fma(0.5 * y, __builtin_fma(-(x * y), y, 1.0), y);
   y = __builtin_fma(0.5 * y, __builtin_fma(-(x * y), y, 1.0), y);
   const double q = y * y;
-  const double iTeff = __builtin_fma(q, __builtin_fma(-x, q, 1.0), q);
+  rcp = __builtin_fma(q, __builtin_fma(-x, q, 1.0), q);
+  return y;
+}
+
+// The pair-symmetric part of coulomb_colln (collisions.f90:138-157) for species a < b:
+// 1/Teff**1.5 and W**2, from one reciprocal root.
+struct Pair { double iT15, W2; };
+__device__ __forceinline__ Pair coulomb_pair(double ma, double mb, double Ta, double Tb, double va, double vb) {
+  double iTeff;
+  const double y = rsqrt2(__builtin_fma(mb, Ta, ma * Tb) * (1.0 / (mb + ma)), iTeff);
   const double dv = va - vb;
   return {iTeff * y, ((dv * dv) * (((ma * mb) / (ma + mb)) / (2.0 * kB))) * iTeff};
 }
 
-// Phisj and Psisj above W**2 = 1 (the reference's closed form; Phisj is 1 below W = 0.1)
-__device__ __forceinline__ void drift_far(double W2, double& Phi, double& Psi) {
-  const double W = sqrt(W2), iW = 1.0 / W, iW2 = iW * iW;
-  Psi = exp(-W2);
-  Phi = (((3.0 / 4.0) * sqrt(PI)) * erf(W)) * (iW2 * iW) - ((3.0 / 2.0) * iW2) * Psi;
+// Phisj and Psisj above x = W**2 = 1: Phi = (3/4 sqrt(pi) erf(W)/W - 3/2 exp(-x))/x with erf as
+// 1 - exp(-x) (exp(x) erfc(W)).  Off by 5e-16 at most where that form with the library's erf is
+// off by 9e-16.
+__device__ __forceinline__ void drift_far(double x, double& Phi, double& Psi) {
+  x = x > 1e300 ? 1e300 : x;                     // (of an infinite drift: both are zero)
+  double rcp;
+  const double u = rsqrt2(x, rcp);
+  // exp(-x) = 2**n exp(r), |r| <= log(2)/2: the Taylor series to r**13 (off by 4e-18).  (Zero
+  // where x is no number, which Phi shows.)
+  const double xe = x < 800.0 ? x : 800.0;
+  const double n = __builtin_rint(xe * -1.4426950408889634);
+  double r = __builtin_fma(n, -0.6931471805599453, -xe);
+  r = __builtin_fma(n, -2.3190468138462996e-17, r);
+  Psi = __builtin_amdgcn_ldexp(horner<13>(c_drift + 43, r), (int)n);
+  const double e = Psi * horner<17>(c_drift + 25, __builtin_fma(2.0, u, -1.0));
+  Phi = rcp * __builtin_fma((3.0 / 4.0) * sqrt(PI), u, -e);
 }
-// the bit of the unordered pair a < b in a mask of the 21 pairs
-__device__ __forceinline__ constexpr int pair_bit(int a, int b) { return (a - 1) * (14 - a) / 2 + (b - a - 1); }
 constexpr double W2_NEAR = 1.0;
+// the species of pair k of (1,2), (1,3), .., (6,7)
+__device__ __forceinline__ constexpr int pair_a(int k) { return k < 6 ? 1 : k < 11 ? 2 : k < 15 ? 3 : k < 18 ? 4 : k < 20 ? 5 : 6; }
+__device__ __forceinline__ constexpr int pair_b(int k) { return k < 6 ? k + 2 : k < 11 ? k - 3 : k < 15 ? k - 7 : k < 18 ? k - 10 : k < 20 ? k - 12 : 7; }
 
-// The Coulomb terms of all species pairs.  add(x, y, iT15 Phi, iT15 Psi, Ty, v1y, ny) takes
-// species x's share of its collisions with y.  Up to W**2 = 1 (a drift of 1.5 km/s between
-// heavy ions, hundreds of km/s between ions and electrons) Phi and Psi are the series: no
-// branch, so that the 21 unrolled pairs stay one run of instructions.  Pairs beyond enter
-// with zeros there, are marked in a mask, and lanes that hold any add them afterwards in a
-// rolled loop over the partner, whose values it reads again (it is never entered at ordinary
-// drifts, and its erf and exp would otherwise be part of every pair).  So are pairs whose W**2
-// is not a number.
+// The Coulomb terms of all species pairs.  add(x, y, iT15 Phi, iT15 Psi) takes species x's share
+// of its collisions with y.  Up to W**2 = 1 (a drift of 1.5 km/s between heavy ions, 6 between
+// H+ and O+, hundreds between ions and electrons) Phi and Psi are the series; a wave with a
+// lane that is beyond in any pair of a group of seven (or has no number) branches for the group.
+// Each branch ends a run of instructions, and a pair's chain is long: by single pairs ordinary
+// cells took 4 % longer than by sevens (255x113x67 energy 284 us and 273).  Left to a loop of
+// their own over the partner, whose values it read again, with erf and exp evaluated for both
+// species of a pair, the pairs beyond cost more than they had before there was a series: H+
+// flowing out at 20 km/s 491 and 617 us (energy and momentum, 255x113x67, erf and exp in every
+// pair), 552 and 348 (that loop), 371 and 312 now; two pairs in three beyond 560 and 689, 883 and
+// 630, 375 and 347.
 template <bool PSI, int NX, typename ADD>
-__device__ __forceinline__ void coulomb_terms(const DevGrid& g, const DevState& s, long c, const double* n,
-                                              const double* T, const double* v1, ADD add) {
-  unsigned far = 0;
+__device__ __forceinline__ void coulomb_terms(const double* T, const double* v1, ADD add) {
+  constexpr int G = 7;                           // pairs of a group
 #pragma unroll
-  for (int a = 1; a < LSP; ++a) {
+  for (int k = 0; k < 21; k += G) {
+    double iT15[G], W2[G], phi[G], psi[G];
+    bool far = false;
 #pragma unroll
-    for (int b = a + 1; b <= LSP; ++b) {
+    for (int j = 0; j < G; ++j) {
+      const int a = pair_a(k + j), b = pair_b(k + j);
       const Pair p = coulomb_pair(ms(a), ms(b), T[a - 1], T[b - 1], v1[a - 1], v1[b - 1]);
-      const bool f = !(p.W2 <= W2_NEAR);
-      const double i = f ? 0.0 : p.iT15;
-      far |= f ? 1u << pair_bit(a, b) : 0u;
-      double phi = horner<11>(c_drift, p.W2);
-      phi = i * (p.W2 < 0.01 ? 1.0 : phi);
-      const double psi = PSI ? i * horner<12>(c_drift + 12, p.W2) : 0.0;
-      const double phi_f = f ? 0.0 : phi, psi_f = f ? 0.0 : psi;   // (0 times an infinity is no zero)
-      add(a, b, phi_f, psi_f, T[b - 1], v1[b - 1], n[b - 1], false);
-      if (b <= NX) add(b, a, phi_f, psi_f, T[a - 1], v1[a - 1], n[a - 1], false);
-      __builtin_amdgcn_sched_barrier(0);         // (keeps one pair's values in registers)
+      iT15[j] = p.iT15;
+      W2[j] = p.W2;
+      far = far || !(W2[j] <= W2_NEAR);
+      const double s = horner<11>(c_drift, W2[j]);
+      phi[j] = W2[j] < 0.01 ? 1.0 : s;
+      psi[j] = PSI ? horner<12>(c_drift + 12, W2[j]) : 0.0;
     }
-  }
-  if (far) {
+    if (__builtin_expect(__any(far), 0)) {
 #pragma unroll
-    for (int x = 1; x <= NX; ++x) {
-#pragma unroll 1
-      for (int y = 1; y <= LSP; ++y) {
-        if (y == x) continue;
-        const int a = x < y ? x : y, b = x < y ? y : x;
-        if (!(far >> pair_bit(a, b) & 1u)) continue;
-        const long o = (long)(y - 1) * g.N + c;
-        const double Ty = s.Ts[o], vy = s.vs1[o], ny = s.ns[o];
-        // an infinite Teff (whose reciprocal root is no number above): 1/Teff**1.5 is zero
-        if (T[x - 1] == __builtin_inf() || Ty == __builtin_inf()) continue;
-        const Pair p = coulomb_pair(ms(x), ms(y), T[x - 1], Ty, v1[x - 1], vy);
-        double Phi, Psi;
-        drift_far(p.W2, Phi, Psi);
-        add(x, y, p.iT15 * Phi, p.iT15 * Psi, Ty, vy, ny, true);
+      for (int j = 0; j < G; ++j) {
+        const int a = pair_a(k + j), b = pair_b(k + j);
+        double phi_f, psi_f;
+        drift_far(W2[j], phi_f, psi_f);
+        if (!(W2[j] <= W2_NEAR)) {
+          phi[j] = phi_f;
+          psi[j] = psi_f;
+        }
+        // an infinite Teff (which has no reciprocal root above): no collisions, no drift
+        if (T[a - 1] == __builtin_inf() || T[b - 1] == __builtin_inf()) {
+          iT15[j] = 0.0;
+          phi[j] = psi[j] = 1.0;
+        }
       }
     }
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      const int a = pair_a(k + j), b = pair_b(k + j);
+      const double f = iT15[j] * phi[j], q = iT15[j] * psi[j];
+      add(a, b, f, q);
+      if (b <= NX) add(b, a, f, q);
+    }
+    __builtin_amdgcn_sched_barrier(0);           // (keeps one group's values in registers)
   }
 }
+
+// the values are formed here: the compiler would move their operations down, past the branches,
+// to the next use, and keep what they are formed from in registers instead
+__device__ __forceinline__ void pin(double& a, double& b) { __asm__ volatile("" : "+v"(a), "+v"(b)); }
 
 struct Cell {
   int i1, i2, i3;
@@ -263,20 +300,19 @@ __global__ __launch_bounds__(TPB) void k_src_energy(DevGrid g, DevState s, DevSo
       }
       P[isp - 1] = Pp;
       L[isp - 1] = m * Ll;
+      pin(P[isp - 1], L[isp - 1]);
       __builtin_amdgcn_sched_barrier(0);
     }
     // ion-ion and ion-electron (Coulomb)
-    coulomb_terms<true, LSP>(g, s, c, n, T, v1,
-        [&](int x, int y, double phi, double psi, double Ty, double v1y, double ny, bool again) {
-          const long o = (long)(y - 1) * g.N + c;
-          const double d1 = v1[x - 1] - v1y, d2 = v2[x - 1] - (again ? s.vs2[o] : v2[y - 1]),
-                       d3 = v3[x - 1] - (again ? s.vs3[o] : v3[y - 1]);
-          const double dv2 = ((d1 * d1) + (d2 * d2)) + (d3 * d3);
-          const double c2 = csj_1e6(x, y) * (2.0 / (ms(x) + ms(y)));
-          const double npsi = ny * psi;
-          P[x - 1] = P[x - 1] + (c2 * kB) * (npsi * Ty) + (c2 * (ms(y) / 3.0)) * (ny * (phi * dv2));
-          L[x - 1] = L[x - 1] + (c2 * ms(x)) * npsi;
-        });
+    coulomb_terms<true, LSP>(T, v1, [&](int x, int y, double phi, double psi) {
+      const double d1 = v1[x - 1] - v1[y - 1], d2 = v2[x - 1] - v2[y - 1], d3 = v3[x - 1] - v3[y - 1];
+      const double dv2 = ((d1 * d1) + (d2 * d2)) + (d3 * d3);
+      const double c2 = csj_1e6(x, y) * (2.0 / (ms(x) + ms(y)));
+      const double ny = n[y - 1], npsi = ny * psi;
+      P[x - 1] = P[x - 1] + (c2 * kB) * (npsi * T[y - 1]) + (c2 * (ms(y) / 3.0)) * (ny * (phi * dv2));
+      L[x - 1] = L[x - 1] + (c2 * ms(x)) * npsi;
+      pin(P[x - 1], L[x - 1]);
+    });
 #pragma unroll
     for (int i = 1; i <= LSP; ++i) P[i - 1] = (n[i - 1] * (ms(i) * (1.0 / (gammas(i) - 1.0)))) * P[i - 1];
     // inelastic electron-neutral collisions (sources.f90:350-373)
@@ -365,14 +401,15 @@ __global__ __launch_bounds__(TPB, 3) void k_src_momentum(DevGrid g, DevState s, 
       for (int isp2 = 1; isp2 <= 4; ++isp2) Ll = Ll + maxwell(isp, isp2, nnk[isp2 - 1], Tn, T[isp - 1]);
       P[isp - 1] = Ll * vn1;                     // (times ns ms, applied at the end)
       L[isp - 1] = Ll;
+      pin(P[isp - 1], L[isp - 1]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    coulomb_terms<false, LSP - 1>(g, s, c, n, T, v1,
-        [&](int x, int y, double phi, double, double, double v1y, double ny, bool) {
-          const double nphi = csj_1e6(x, y) * (ny * phi);
-          L[x - 1] = L[x - 1] + nphi;
-          P[x - 1] = P[x - 1] + nphi * v1y;
-        });
+    coulomb_terms<false, LSP - 1>(T, v1, [&](int x, int y, double phi, double) {
+      const double nphi = csj_1e6(x, y) * (n[y - 1] * phi);
+      L[x - 1] = L[x - 1] + nphi;
+      P[x - 1] = P[x - 1] + nphi * v1[y - 1];
+      pin(P[x - 1], L[x - 1]);
+    });
 #pragma unroll
     for (int i = 1; i < LSP; ++i) P[i - 1] = (n[i - 1] * ms(i)) * P[i - 1];
     // geometric factors, ambipolar field, gravity (sources.f90:248-288)
