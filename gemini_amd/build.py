@@ -6,8 +6,8 @@ file is first read or written, so the library has no load-time dependency on it.
 Flags that matter for results:
   -ffp-contract=off   no fused multiply-add unless written: every product and sum is
                       rounded on its own, as in the reference's x86-64 build (bit-identical
-                      parity).  kernels_sources.hip, whose rates call transcendental
-                      functions and match to 1e-12, contracts by a pragma of its own,
+                      parity).  The energy and momentum sources (kernels_sources.hip), whose
+                      rates match to 1e-12, contract by a pragma of their own,
   -Xclang -target-feature -Xclang -packed-fp32-ops
                       no packed FP32 instructions anywhere in the device code.
 """

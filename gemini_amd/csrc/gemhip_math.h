@@ -4,7 +4,7 @@
 // x86-64 baseline: no FMA, IEEE divide and sqrt, glibc pow).  The library is
 // compiled with -ffp-contract=off, so a*b+c stays two rounded operations; a divide
 // stays one, or is div_rcp, which gives its result from the divisor's correctly
-// rounded reciprocal.  (The source passes alone are held to a tolerance and contract.)
+// rounded reciprocal.  (The energy and momentum sources are held to a tolerance and contract.)
 // The header also compiles as plain C++ on the host (GEMHIP_HD expands to nothing) so
 // the CPU tests can check the scalar routines against libm.
 #pragma once

@@ -9,14 +9,16 @@
 // back to temperature / velocity / electron density.  The rates never touch HBM.
 //
 // Arithmetic follows the reference's expressions, with liberties that cost a few ulp per
-// operation at most: products and sums contract into FMAs in this file, a divide by a
-// compile-time constant (a mass sum, 3) is a multiply by its correctly rounded reciprocal, a
-// Coulomb pair's powers of 1/Teff come from one reciprocal root (to an ulp or so, where the
-// reference divides and takes a power) and its drift functions from polynomials.  The
-// transcendental functions of the other rates (exp, log, log10, tanh, sin, and x**p for the
-// fitted exponents) are the device library's, which agree with glibc to about an ulp; x**0.5 is
-// the correctly rounded sqrt.  These passes therefore match the reference to rounding (the
-// tests hold them to 1e-12 of each field's magnitude) rather than bit for bit.
+// operation at most: products and sums of the energy and momentum passes contract into FMAs
+// (which takes them from 3.59 and 3.71 ms to 3.33 and 3.65 at 512x256x192; the mass pass gains
+// nothing by it and rounds each on its own), a divide by a compile-time constant (a mass sum,
+// 3) is a multiply by its correctly rounded reciprocal, a Coulomb pair's powers of 1/Teff come
+// from one reciprocal root (to an ulp or so, where the reference divides and takes a power)
+// and its drift functions from polynomials.  The transcendental functions of the other rates
+// (exp, log, log10, tanh, sin, and x**p for the fitted exponents) are the device library's,
+// which agree with glibc to about an ulp; x**0.5 is the correctly rounded sqrt.  These passes
+// therefore match the reference to rounding (the tests hold them to 1e-12 of each field's
+// magnitude) rather than bit for bit.
 //
 // Ion-ion (Coulomb) terms: Teff, Wsj, Phisj and Psisj of coulomb_colln are symmetric in
 // the species pair, so each unordered pair is evaluated once and feeds both species.  The
@@ -70,6 +72,7 @@ __device__ __forceinline__ double mn(int isp2) {
 
 // calculus.in.f90:174-196
 __device__ __forceinline__ double etd(double f, double P, double L, double dt) {
+#pragma clang fp contract(off)
   const double Ldt = L * dt;
   const double expL = exp(-1.0 * Ldt);
   if (Ldt > 1e-10) return f * expL + (P / L) * (1.0 - expL);
@@ -467,6 +470,7 @@ __global__ __launch_bounds__(TPB, 3) void k_src_momentum(DevGrid g, DevState s, 
 // kreac fits of srcsContinuity: ((((c0 s1 c1 t) s2 c2 t^2) s3 c3 t^3) s4 c4 t^4)
 __device__ __forceinline__ double poly4(double t, double c0, double c1, double c2, double c3,
                                         double c4, bool p1, bool p2, bool p3, bool p4) {
+#pragma clang fp contract(off)
   const double t2 = t * t, t3 = t2 * t, t4 = t2 * t2;
   double r = c0;
   r = p1 ? r + c1 * t : r - c1 * t;
@@ -485,6 +489,7 @@ __device__ __forceinline__ double poly4(double t, double c0, double c1, double c
 template <bool CLEAN>
 __global__ __launch_bounds__(TPB) void k_src_mass(DevGrid g, DevState s, DevSources a, double dt,
                                                   const int* nul) {
+#pragma clang fp contract(off)
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.N) return;
   const Cell q = decode(g, c);
