@@ -412,8 +412,9 @@ __device__ __forceinline__ void adj_backsub(const Col& q, int N, int s0, int sx)
 
 // M^T w = rhs for a matrix factored by adj_elim into slots s0...  The rhs is slot s0+3, or
 // with CW the interior rows of cw * (slot BY); slot s0+3 ends holding w.
-// U^T z = rhs top-down, then the eliminations transposed bottom-up: z(j) -= l_j z(j+1),
-// then the interchange.
+// U^T z = rhs top-down (z(i-1), the chain's last value, comes off last; the error is the same in
+// either order), then the eliminations transposed bottom-up: z(j) -= l_j z(j+1), then the
+// interchange.
 template <bool CW>
 __device__ __forceinline__ void adj_solveT(const Col& q, int N, int s0, double cw = 0.0) {
   double zm1 = 0.0, zm2 = 0.0;                       // z(i-1), z(i-2)
