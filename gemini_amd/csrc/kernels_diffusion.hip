@@ -720,8 +720,8 @@ __global__ __launch_bounds__(small_threads(W)) void k_diffusion_small(DevGrid g,
   }
   __syncthreads();
   // ---- the solves: the first wave; lanes past W repeat the last column
-  if (tid < 64) {
-    const int lane = tid, c = min(lane & 31, W - 1);
+  if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
+    const int lane = tid & 63, c = min(lane & 31, W - 1);
     const bool second = !BE && lane >= 32;             // the BDF2 factorisation
     const int col = min(c0 + c, ncol - 1);
     double Tmin, Tmax, aN = 0.0, bN = 1.0;
